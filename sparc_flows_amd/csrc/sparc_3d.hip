@@ -14,12 +14,13 @@
 // state a + deltat * RHS; every other step one pass applies
 // FILTER_VARS_3D_HORIZ_PML (physics.f90:836-882).
 //
-// Layout: fields [nz][ny][nx], x fastest.  A z pass gives each lane one (x, y)
-// column and streams it bottom to top and back (the Thomas sweeps of dbyd2 /
-// mtridag), so the 64 lanes of a wave touch 64 consecutive doubles per row.
-// At nx = ny = 256 a pass has 65536 columns, 1024 waves, one per SIMD: the
-// sweeps issue their loads in chunks of rows (and Zv runs four independent
-// chains) so that each lane keeps tens of loads in flight.
+// Layout: fields [nz][ny][nx], x fastest.  The z passes run segmented
+// (sparc_zseg.hip) wherever zseg3_fits; the forms here are for the other
+// grids (nz above 512, a few nz that no cut fits, fields of 2^31 bytes and
+// more).  They give each lane one (x, y) column and stream it bottom to top and
+// back (the Thomas sweeps of dbyd2 / mtridag), so the 64 lanes of a wave touch
+// 64 consecutive doubles per row, with loads issued in chunks of rows (and four
+// independent chains in Zv) to keep tens of them in flight.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -32,6 +33,7 @@
 #include "sparc_device.h"
 #include "sparc_host.h"
 #include "sparc_launch.h"
+#include "sparc_zseg.h"
 
 namespace sparc {
 namespace d3 {
@@ -109,45 +111,6 @@ __global__ __launch_bounds__(64) void k3_ddy_any(const double *__restrict__ in, 
     }
 }
 
-// Arguments of the two z passes.
-struct Z3 {
-    const double *B;            // Zp: xi_z; Zv: v_x (v_y, v_z follow at +N, +2N)
-    double *W;                  // forward-sweep values, one [nz][nxy] block per chain
-    size_t N;                   // points per field
-    int nxy, nz, nb, nt;
-    const double *stretch;      // [nz]
-    DbyCoef cf;
-    Tri tr1, tr0;               // dbyd2 factors for ibc 1 and ibc 0
-    const double *rhoinv;       // [nz] 1/rho0
-    const double *az, *bz;      // [npml][nxy]
-    const double *psi;          // z-PML variables of this stage [2][npml][nxy]: d xi_z/dz, d p/dz
-    // the next stage's input (step.f90:60-62) or, after the fifth stage, the
-    // updated state (:107-108): out = base + beta * RHS, for the fields and
-    // the z-PML variables; the fifth stage also keeps the RHS in rhs
-    const double *a, *pml;      // base: state a [6][nz][nxy], pmlvars [2][npml][nxy]
-    double *tnext, *pnext;      // T of the next stage (or a), its PML variables (or pmlvars)
-    double beta;
-    int last;
-    // Zp
-    const double *dxi, *dyi;    // d xi_x/dx, d xi_y/dy
-    const double *c2rho0, *gp0, *gr0;   // [nz][nxy], PML factor applied
-    const double *rho0, *g;     // [nz]
-    double *P, *RG;             // p; rho' g / rho0
-    // Zv
-    const double *dxv, *dyv;    // d v_i/dx, d v_i/dy, [3][nz][nxy]
-    const double *v0x, *v0y, *v0z;
-    const double *dxp, *dyp;    // d p/dx, d p/dy
-    double *rhs;                // scr [6][nz][nxy]
-    const double *srcdep;       // [nz]
-    Src src;
-    int time, e_rad;
-};
-
-__device__ __forceinline__ int pml_index(int j, int nz, int nb, int nt)
-{
-    return j < nb ? j : (j >= nz - nt ? nb + (j - (nz - nt)) : -1);
-}
-
 // Forward elimination (dbyd2.f + mtridag.f:96-105) of NC columns of one lane
 // at once, rows 2..nz-3 in chunks of U whose loads are issued together: a
 // lane then has NC * U loads in flight instead of one per dependent step.
@@ -197,7 +160,7 @@ __global__ __launch_bounds__(256) void k3_zp(Z3 z)
     sweep_fwd<1, UF>(fw, Bs, Ws, ibc, trs, c, s, nz, z.cf);
     double d = fw[0].ud;
     for (int j0 = nz - 1; j0 >= 0; j0 -= UB) {
-        double w[UB], dxi[UB], dyi[UB], xiz[UB], c2r[UB], gp[UB], gr[UB];
+        double w[UB], dxi[UB], dyi[UB], xiz[UB], c2r[UB];
 #pragma unroll
         for (int u = 0; u < UB; u++) {
             const size_t q = c + (size_t)max(j0 - u, 0) * s;
@@ -206,8 +169,6 @@ __global__ __launch_bounds__(256) void k3_zp(Z3 z)
             dyi[u] = z.dyi[q];
             xiz[u] = z.B[q];
             c2r[u] = z.c2rho0[q];
-            gp[u] = z.gp0[q];
-            gr[u] = z.gr0[q];
         }
 #pragma unroll
         for (int u = 0; u < UB; u++) {
@@ -217,16 +178,19 @@ __global__ __launch_bounds__(256) void k3_zp(Z3 z)
             if (j < nz - 1) d = w[u] - z.tr1.gam[j + 1] * d;
             double dz = d * z.stretch[j];
             const int pj = pml_index(j, nz, z.nb, z.nt);
+            double gp = z.gp0z[j], gr = z.gr0z[j];
             if (pj >= 0) {
                 const size_t qp = c + (size_t)pj * s;
-                const double ps = z.psi[qp];
+                const double ps = z.psi[qp], fz = z.fz[qp];
                 const double rp = z.az[qp] * dz + z.bz[qp] * ps;
                 z.pnext[qp] = z.pml[qp] + z.beta * rp;
                 dz = dz + ps;
+                gp = gp * fz;
+                gr = gr * fz;
             }
             const double div = (dxi[u] + dyi[u]) + dz;
-            z.P[q] = -(c2r[u] * div) - xiz[u] * gp[u];
-            const double rho = -(z.rho0[j] * div) - xiz[u] * gr[u];
+            z.P[q] = -(c2r[u] * div) - xiz[u] * gp;
+            const double rho = -(z.rho0[j] * div) - xiz[u] * gr;
             z.RG[q] = z.rhoinv[j] * rho * z.g[j];
         }
     }
@@ -494,7 +458,9 @@ struct sparc3d_handle {
     const double *cdx = nullptr, *cdy = nullptr;      // circulant columns [2n] (an n that is not a power of two)
     const double *dmx = nullptr, *dmy = nullptr, *d_stretch = nullptr, *d_rhoinv = nullptr, *d_rho0 = nullptr,
                  *d_g = nullptr, *d_srcdep = nullptr;
-    double *c2rho0 = nullptr, *gp0 = nullptr, *gr0 = nullptr, *az = nullptr, *bz = nullptr;
+    double *c2rho0 = nullptr, *az = nullptr, *bz = nullptr, *fz = nullptr;   // fz: PML factor of the gradients below
+    const double *gp0z = nullptr, *gr0z = nullptr;    // [nz] d p0/dz, d rho0/dz before the PML factor
+    ZSeg zseg{};                                      // segmented z passes: sets ibc 1, ibc 0 (img null: no such cut of nz)
     double *v0x = nullptr, *v0y = nullptr, *v0z = nullptr;
     double *a = nullptr, *scr = nullptr, *tmp = nullptr, *pml = nullptr, *psit = nullptr;
     double *DXI = nullptr, *DYI = nullptr, *DX3 = nullptr, *DY3 = nullptr, *P = nullptr, *RG = nullptr,
@@ -615,13 +581,14 @@ static int enqueue_stage(sparc3d_handle *h, int s, int t)
         z.dxi = h->DXI;
         z.dyi = h->DYI;
         z.c2rho0 = h->c2rho0;
-        z.gp0 = h->gp0;
-        z.gr0 = h->gr0;
+        z.gp0z = h->gp0z;
+        z.gr0z = h->gr0z;
+        z.fz = h->fz;
         z.rho0 = h->d_rho0;
         z.g = h->d_g;
         z.P = h->P;
         z.RG = h->RG;
-        RUN3(3, launch_zp(z, h->stream));
+        RUN3(3, zseg3_fits(z, h->zseg) ? launch_zp_seg(z, h->zseg, h->stream) : launch_zp(z, h->stream));
     }
     if ((r = ddx3(h, h->P, h->DXP, nyz))) return r;
     if ((r = ddy3(h, h->P, h->DYP, nz))) return r;
@@ -648,7 +615,7 @@ static int enqueue_stage(sparc3d_handle *h, int s, int t)
         z.src = h->src;
         z.time = t;
         z.e_rad = h->e_rad;
-        RUN3(4, launch_zv(z, h->stream));
+        RUN3(4, zseg3_fits(z, h->zseg) ? launch_zv_seg(z, h->zseg, h->stream) : launch_zv(z, h->stream));
     }
     return SPARC_OK;
 }
@@ -741,6 +708,21 @@ static int setup3(sparc3d_handle *h)
         HCHECK3(h, upload(h->bg_mem, &pc, rbet, h->stream));
         h->tri[ibc] = Tri{pa, pb, pc};
     }
+    // the segmented z passes' tables
+    if (const int m = zseg_length(nz)) {
+        const int sets[2] = {1, 0};
+        std::vector<double> img;
+        ZSeg sg{};
+        sg.m = m;
+        sg.P = (nz + m - 1) / m;
+        dbyd2_coefs(nz, sg.c1, sg.c2, sg.cb);
+        if (build_zseg(nz, m, 2, sets, sg.hw, img)) {
+            double *pi = nullptr;
+            HCHECK3(h, upload(h->bg_mem, &pi, img, h->stream));
+            sg.img = pi;
+            h->zseg = sg;
+        }
+    }
     // z and stretch = 1/dbyd2(z) (initialize.f90:466-470); deltat (:474)
     h->z.resize(nz);
     for (int k = 0; k < nz; k++) h->z[k] = h->model[6 * (size_t)k];
@@ -789,17 +771,15 @@ static int setup3(sparc3d_handle *h)
     std::vector<double> gr0z, gp0z;
     if ((r = host_ddz3(h, h->rho0z, gr0z, h->d_stretch))) return r;
     if ((r = host_ddz3(h, p0z, gp0z, h->d_stretch))) return r;
-    std::vector<double> c2rho0(N), gp0(N), gr0(N);
+    std::vector<double> c2rho0(N);
     for (int k = 0; k < nz; k++)
         for (size_t q = 0; q < nxy; q++) {
             const size_t i = (size_t)k * nxy + q;
             c2rho0[i] = c2[i] * h->rho0z[k];
-            gp0[i] = gp0z[k];
-            gr0[i] = gr0z[k];
         }
     // z-PML (physics.f90:250-296)
     const int nb = h->nb, nt = h->nt, npml = nb + nt;
-    std::vector<double> az((size_t)npml * nxy, 0.0), bz((size_t)npml * nxy, 0.0);
+    std::vector<double> az((size_t)npml * nxy, 0.0), bz((size_t)npml * nxy, 0.0), fz((size_t)npml * nxy, 1.0);
     const double *zz = h->z.data();
     const double a0 = kPi3 * (double)0.005f * diml / dimc;
     for (int k = 0; k < nz; k++) {
@@ -820,17 +800,18 @@ static int setup3(sparc3d_handle *h)
                 dampz = 9.0 * std::sqrt(c2[(size_t)(nz - 1) * nxy + q]) / (zz[nz - 1] - zz[nz - nt]) * (rr * rr);
             }
             const double fd = alphaz / (dampz + alphaz);
-            const size_t i = (size_t)k * nxy + q;
-            gp0[i] *= fd;
-            gr0[i] *= fd;
+            fz[(size_t)pj * nxy + q] = fd;
             if (q == 0) h->g[k] *= fd;
             bz[(size_t)pj * nxy + q] = -alphaz - dampz;
             az[(size_t)pj * nxy + q] = -dampz;
         }
     }
     HCHECK3(h, upload(h->bg_mem, &h->c2rho0, c2rho0, h->stream));
-    HCHECK3(h, upload(h->bg_mem, &h->gp0, gp0, h->stream));
-    HCHECK3(h, upload(h->bg_mem, &h->gr0, gr0, h->stream));
+    HCHECK3(h, upload(h->bg_mem, &h->fz, fz, h->stream));
+    HCHECK3(h, upload(h->bg_mem, &p, gp0z, h->stream));
+    h->gp0z = p;
+    HCHECK3(h, upload(h->bg_mem, &p, gr0z, h->stream));
+    h->gr0z = p;
     HCHECK3(h, upload(h->bg_mem, &h->az, az, h->stream));
     HCHECK3(h, upload(h->bg_mem, &h->bz, bz, h->stream));
     HCHECK3(h, upload(h->bg_mem, &p, h->rhoinvz, h->stream));

@@ -154,4 +154,25 @@ SPARC_HD int seg_kind(int s, int P) { return s == 0 ? 0 : (s == P - 1 ? 2 : 1); 
 // segment's tables differ from the first interior one's.
 bool seg_kind_tables(const SegTables &t, std::vector<double> &out);
 
+
+// ---------------------------------------------------------------------------
+// Tables of the z kernels of sparc_zseg.hip: at most kZSegP segments of m rows.
+constexpr int kZSegP = 32;
+// Segment lengths those kernels are instantiated for.
+#define SPARC_ZSEG_SIZES(X) X(4) X(5) X(6) X(7) X(8) X(10) X(12) X(14) X(16)
+// The shortest of them that cuts nz rows into at most kZSegP segments (half as
+// many up to nz = 160, where blocks of twice the columns then fit) whose last holds at least 3 real rows; 0 if there is none (nz > 512, and a few sizes below).
+int zseg_length(int nz);
+// The device image of nset matrices, one after the other: the banded
+// interface inverse [2P][4hw+4], then the segment tables [5][3][m] by kind,
+// padded to an even count.  sets[k]: an ibc (0..3), plus kZSegT for the
+// transposed matrix.  false if a system is singular.
+constexpr int kZSegT = 4;
+bool build_zseg(int nz, int m, int nset, const int *sets, int &hw, std::vector<double> &img);
+// Doubles of one matrix in that image.
+SPARC_HD int zseg_set_len(int P, int hw, int m) { return (2 * P * (4 * hw + 4) + 15 * m + 1) & ~1; }
+// Rows 0, 1, N-2, N-1 of the map from a column to dbyd2's right-hand side
+// (dbyd2.f:91-172, kept rows 0): eb[5 r + k], columns k (rows 0, 1) or N-5+k.
+void dbyd2_edge_rows(int N2, int ibc, double eb[20]);
+
 }  // namespace sparc

@@ -83,6 +83,94 @@ bool invert(std::vector<double> A, int n, std::vector<double> &inv)
 
 }  // namespace
 
+namespace {
+
+// The five segment tables of one tridiagonal matrix (sub- and super-diagonals
+// lo, up of N rows, diagonal 1), rows [5][nzp] at tabs, and the exact inverse
+// of its 2P x 2P interface system; widens hw to the largest distance in
+// segments to an entry of the inverse above 1e-24 of its row maximum.
+bool seg_one(int N, int m, const std::vector<double> &lo, const std::vector<double> &up, double *tabs,
+             std::vector<double> &Minv, int &hw)
+{
+    const int P = (N + m - 1) / m;
+    const int nzp = P * m, n2 = 2 * P;
+    std::vector<double> lowr(nzp, 0.0), uppr(nzp, 0.0);
+    for (int j = 0; j < N; j++) { lowr[j] = lo[j]; uppr[j] = up[j]; }
+    std::vector<double> rbl(nzp, 1.0), gl(nzp, 0.0), V(nzp, 0.0), W(nzp, 0.0), bet(nzp, 1.0);
+    for (int s = 0; s < P; s++) {
+        const int a0 = s * m;
+        for (int j = a0 + 1; j < a0 + m; j++) {
+            gl[j] = uppr[j - 1] / bet[j - 1];
+            bet[j] = 1.0 - lowr[j] * gl[j];
+            rbl[j] = 1.0 / bet[j];
+        }
+        auto lsolve = [&](std::vector<double> r, double *out) {
+            r[0] = r[0] * rbl[a0];
+            for (int i = 1; i < m; i++) r[i] = (r[i] - lowr[a0 + i] * r[i - 1]) * rbl[a0 + i];
+            for (int i = m - 2; i >= 0; i--) r[i] = r[i] - gl[a0 + i + 1] * r[i + 1];
+            for (int i = 0; i < m; i++) out[a0 + i] = r[i];
+        };
+        std::vector<double> r(m, 0.0);
+        if (s > 0) { r[0] = lowr[a0]; lsolve(r, V.data()); }
+        std::fill(r.begin(), r.end(), 0.0);
+        if (s < P - 1) { r[m - 1] = uppr[a0 + m - 1]; lsolve(r, W.data()); }
+    }
+    std::vector<double> M((size_t)n2 * n2, 0.0);
+    for (int s = 0; s < P; s++) {
+        const int f = s * m, l = s * m + m - 1;
+        M[(size_t)(2 * s) * n2 + 2 * s] = 1.0;
+        M[(size_t)(2 * s + 1) * n2 + 2 * s + 1] = 1.0;
+        if (s > 0) {
+            M[(size_t)(2 * s) * n2 + 2 * s - 1] += V[f];
+            M[(size_t)(2 * s + 1) * n2 + 2 * s - 1] += V[l];
+        }
+        if (s < P - 1) {
+            M[(size_t)(2 * s) * n2 + 2 * s + 2] += W[f];
+            M[(size_t)(2 * s + 1) * n2 + 2 * s + 2] += W[l];
+        }
+    }
+    if (!invert(M, n2, Minv)) return false;
+    for (int k = 0; k < n2; k++) {
+        double rm = 0.0;
+        for (int q = 0; q < n2; q++) rm = std::max(rm, std::fabs(Minv[(size_t)k * n2 + q]));
+        for (int q = 0; q < n2; q++)
+            if (std::fabs(Minv[(size_t)k * n2 + q]) > 1e-24 * rm) hw = std::max(hw, std::abs(q / 2 - k / 2));
+    }
+    const std::vector<double> *all[5] = {&lowr, &rbl, &gl, &V, &W};
+    for (int k = 0; k < 5; k++) std::copy(all[k]->begin(), all[k]->end(), tabs + (size_t)k * nzp);
+    return true;
+}
+
+// Band storage of an interface inverse: row k keeps the entries q =
+// 2 (k/2 - hw) + w, w < 4 hw + 4 (the window around its own segment), zero
+// outside 0..2P-1.
+void band_rows(const std::vector<double> &Minv, int n2, int hw, double *band)
+{
+    const int W = 4 * hw + 4;
+    for (int k = 0; k < n2; k++)
+        for (int w = 0; w < W; w++) {
+            const int q = 2 * (k / 2 - hw) + w;
+            band[(size_t)k * W + w] = q >= 0 && q < n2 ? Minv[(size_t)k * n2 + q] : 0.0;
+        }
+}
+
+// Rows [nrow][3][m] of the first, an interior and the last segment of rows
+// [nrow][nzp]; false if some interior segment's tables differ from the first
+// interior one's.
+bool kind_rows(const double *rows, int nrow, int P, int m, std::vector<double> &out)
+{
+    const int nzp = P * m, sk[3] = {0, P > 1 ? 1 : 0, P - 1};
+    for (int r = 0; r < nrow; r++) {
+        const double *row = rows + (size_t)r * nzp;
+        for (int s = 2; s < P - 1; s++)
+            if (std::memcmp(row + (size_t)s * m, row + m, (size_t)m * sizeof(double))) return false;
+        for (int k = 0; k < 3; k++) out.insert(out.end(), row + (size_t)sk[k] * m, row + (size_t)(sk[k] + 1) * m);
+    }
+    return true;
+}
+
+}  // namespace
+
 bool build_seg_tables(int N, int m, SegTables &t)
 {
     const int P = (N + m - 1) / m;
@@ -91,88 +179,85 @@ bool build_seg_tables(int N, int m, SegTables &t)
     t.m = m;
     t.nzp = nzp;
     t.slots.assign((size_t)3 * 5 * nzp, 0.0);
-    std::vector<double> minv_all;
+    std::vector<double> minv[3];
     int hw = 0;
     const int ibcs[3] = {1, 2, 3};
     for (int slot = 0; slot < 3; slot++) {
-        std::vector<double> lo0, up0;
-        dbyd2_matrix(N, ibcs[slot], lo0, up0);
-        std::vector<double> lowr(nzp, 0.0), uppr(nzp, 0.0);
-        for (int j = 0; j < N; j++) { lowr[j] = lo0[j]; uppr[j] = up0[j]; }
-        std::vector<double> rbl(nzp, 1.0), gl(nzp, 0.0), V(nzp, 0.0), W(nzp, 0.0), bet(nzp, 1.0);
-        for (int s = 0; s < P; s++) {
-            const int a0 = s * m;
-            for (int j = a0 + 1; j < a0 + m; j++) {
-                gl[j] = uppr[j - 1] / bet[j - 1];
-                bet[j] = 1.0 - lowr[j] * gl[j];
-                rbl[j] = 1.0 / bet[j];
-            }
-            auto lsolve = [&](std::vector<double> r, double *out) {
-                r[0] = r[0] * rbl[a0];
-                for (int i = 1; i < m; i++) r[i] = (r[i] - lowr[a0 + i] * r[i - 1]) * rbl[a0 + i];
-                for (int i = m - 2; i >= 0; i--) r[i] = r[i] - gl[a0 + i + 1] * r[i + 1];
-                for (int i = 0; i < m; i++) out[a0 + i] = r[i];
-            };
-            std::vector<double> r(m, 0.0);
-            if (s > 0) { r[0] = lowr[a0]; lsolve(r, V.data()); }
-            std::fill(r.begin(), r.end(), 0.0);
-            if (s < P - 1) { r[m - 1] = uppr[a0 + m - 1]; lsolve(r, W.data()); }
-        }
-        std::vector<double> M((size_t)n2 * n2, 0.0), Minv;
-        for (int s = 0; s < P; s++) {
-            const int f = s * m, l = s * m + m - 1;
-            M[(size_t)(2 * s) * n2 + 2 * s] = 1.0;
-            M[(size_t)(2 * s + 1) * n2 + 2 * s + 1] = 1.0;
-            if (s > 0) {
-                M[(size_t)(2 * s) * n2 + 2 * s - 1] += V[f];
-                M[(size_t)(2 * s + 1) * n2 + 2 * s - 1] += V[l];
-            }
-            if (s < P - 1) {
-                M[(size_t)(2 * s) * n2 + 2 * s + 2] += W[f];
-                M[(size_t)(2 * s + 1) * n2 + 2 * s + 2] += W[l];
-            }
-        }
-        if (!invert(M, n2, Minv)) return false;
-        // window half-width: entries below 1e-24 of their row maximum are dropped
-        for (int k = 0; k < n2; k++) {
-            double rm = 0.0;
-            for (int q = 0; q < n2; q++) rm = std::max(rm, std::fabs(Minv[(size_t)k * n2 + q]));
-            for (int q = 0; q < n2; q++)
-                if (std::fabs(Minv[(size_t)k * n2 + q]) > 1e-24 * rm) hw = std::max(hw, std::abs(q / 2 - k / 2));
-        }
-        minv_all.insert(minv_all.end(), Minv.begin(), Minv.end());   // banded below, once hw is known
-        const std::vector<double> *tabs[5] = {&lowr, &rbl, &gl, &V, &W};
-        for (int k = 0; k < 5; k++)
-            std::copy(tabs[k]->begin(), tabs[k]->end(), t.slots.begin() + (size_t)(5 * slot + k) * nzp);
+        std::vector<double> lo, up;
+        dbyd2_matrix(N, ibcs[slot], lo, up);
+        if (!seg_one(N, m, lo, up, t.slots.data() + (size_t)5 * slot * nzp, minv[slot], hw)) return false;
     }
     t.hw = hw;
-    // band storage: row k keeps the entries q = 2 (k/2 - hw) + w, w < 4 hw + 4
-    // (the window around its own segment), zero outside 0..2P-1
     const int W = 4 * hw + 4;
     t.band.assign((size_t)3 * n2 * W, 0.0);
-    for (int slot = 0; slot < 3; slot++)
-        for (int k = 0; k < n2; k++)
-            for (int w = 0; w < W; w++) {
-                const int q = 2 * (k / 2 - hw) + w;
-                if (q >= 0 && q < n2)
-                    t.band[((size_t)slot * n2 + k) * W + w] = minv_all[((size_t)slot * n2 + k) * n2 + q];
-            }
+    for (int slot = 0; slot < 3; slot++) band_rows(minv[slot], n2, hw, t.band.data() + (size_t)slot * n2 * W);
     return true;
+}
+
+int zseg_length(int N)
+{
+    static const int sizes[] = {
+#define X(v) v,
+        SPARC_ZSEG_SIZES(X)
+#undef X
+    };
+    for (int m : sizes) {
+        const int P = (N + m - 1) / m;
+        if (P <= (N <= 160 ? kZSegP / 2 : kZSegP) && N - (P - 1) * m >= 3) return m;
+    }
+    return 0;
+}
+
+bool build_zseg(int N, int m, int nset, const int *sets, int &hw, std::vector<double> &img)
+{
+    const int P = (N + m - 1) / m;
+    const int nzp = P * m, n2 = 2 * P;
+    std::vector<std::vector<double>> minv(nset), tabs(nset);
+    hw = 0;
+    for (int k = 0; k < nset; k++) {
+        std::vector<double> lo, up;
+        dbyd2_matrix(N, sets[k] & 3, lo, up);
+        if (sets[k] & kZSegT) {                               // the transposed matrix
+            std::vector<double> lt(N, 0.0), ut(N, 0.0);
+            for (int j = 1; j < N; j++) lt[j] = up[j - 1];
+            for (int j = 0; j + 1 < N; j++) ut[j] = lo[j + 1];
+            lo = lt;
+            up = ut;
+        }
+        tabs[k].assign((size_t)5 * nzp, 0.0);
+        if (!seg_one(N, m, lo, up, tabs[k].data(), minv[k], hw)) return false;
+    }
+    const int W = 4 * hw + 4;
+    img.clear();
+    for (int k = 0; k < nset; k++) {
+        std::vector<double> band((size_t)n2 * W);
+        band_rows(minv[k], n2, hw, band.data());
+        img.insert(img.end(), band.begin(), band.end());
+        if (!kind_rows(tabs[k].data(), 5, P, m, img)) return false;
+        if (img.size() & 1) img.push_back(0.0);               // every set starts on 16 bytes
+    }
+    return true;
+}
+
+void dbyd2_edge_rows(int N2, int ibc, double eb[20])
+{
+    double c1, c2, cb[kCB];
+    dbyd2_coefs(N2, c1, c2, cb);
+    for (int k = 0; k < 5; k++) {
+        const double f = k < 4 ? cb[CB_F + k] : 0.0, b = cb[CB_B + k];
+        const double far = (cb[CB_ALPHA2] * f - cb[CB_BETA1] * b) * cb[CB_CNST];
+        eb[k] = ibc & 1 ? far : 0.0;
+        eb[5 + k] = b;
+        eb[10 + 4 - k] = -b;
+        eb[15 + 4 - k] = ibc == 1 || ibc == 2 ? -far : 0.0;
+    }
 }
 
 bool seg_kind_tables(const SegTables &t, std::vector<double> &out)
 {
-    const int P = t.P, m = t.m, nzp = t.nzp;
-    const int sk[3] = {0, P > 1 ? 1 : 0, P - 1};
     out.clear();
-    out.reserve((size_t)15 * 3 * m);
-    for (int r = 0; r < 15; r++) {
-        const double *row = t.slots.data() + (size_t)r * nzp;
-        for (int s = 2; s < P - 1; s++)
-            if (std::memcmp(row + (size_t)s * m, row + m, (size_t)m * sizeof(double))) return false;
-        for (int k = 0; k < 3; k++) out.insert(out.end(), row + (size_t)sk[k] * m, row + (size_t)(sk[k] + 1) * m);
-    }
-    return true;
+    out.reserve((size_t)15 * 3 * t.m);
+    return kind_rows(t.slots.data(), 15, t.P, t.m, out);
 }
 
 }  // namespace sparc

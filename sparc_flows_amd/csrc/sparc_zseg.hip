@@ -1,0 +1,435 @@
+// sparc_zseg.hip -- segmented z kernels: the z passes of a 3D stage
+// (displacement.f90:400-473) with the compact-FD derivatives of dbyd2 /
+// mtridag (dbyd2.f:8-200) solved by segments.
+//
+// A block holds NC neighbouring columns for all nz rows: every column is cut
+// into P <= kZSegP segments of MS rows, one lane per (column, segment), columns
+// fastest, so that a wave instruction touches 64 / NC rows of 8 NC consecutive
+// bytes.  A z-derivative is the segment's right-hand side from a window of MS + 6
+// rows, a Thomas solve of the segment in registers, the exchange of the
+// segment end values through LDS and the exact correction with the interface
+// values (sparc_seg.h, the arithmetic of the 2D column pass).  Each input row
+// is read once from memory (the windows' six halo rows hit the caches) and
+// nothing is written but the results: the one-lane sweeps this replaces write
+// and read back their forward-sweep values and re-read the field.
+#include <algorithm>
+
+#include "sparc_launch.h"
+#include "sparc_zseg.h"
+
+namespace sparc {
+namespace {
+
+// Loads and stores at a 32-bit byte offset from a wave-uniform base address
+// (SGPR base + VGPR offset); arrays indexed this way span less than 2^32 bytes.
+#define SPARC_GLOBAL __attribute__((address_space(1)))
+__device__ __forceinline__ double ldg(const double *base, unsigned ob)
+{
+    return *(const SPARC_GLOBAL double *)((const SPARC_GLOBAL char *)base + ob);
+}
+__device__ __forceinline__ void stg(double *base, unsigned ob, double v)
+{
+    *(SPARC_GLOBAL double *)((SPARC_GLOBAL char *)base + ob) = v;
+}
+
+// A block's logical number: the hardware deals consecutive blocks to the eight
+// XCDs in turn; this gives each XCD one contiguous stretch, so that blocks that
+// share 128-byte lines meet in one L2.
+__device__ __forceinline__ unsigned xcd_block(unsigned id, unsigned n)
+{
+    const unsigned q = n >> 3, r = n & 7, x = id & 7;
+    return x * q + min(x, r) + (id >> 3);
+}
+
+// One lane's part of a column: segment s, rows a .. a + MS - 1 of column c.
+struct Lane {
+    int c, s, a;
+    bool act, first, last;      // a segment of the column; its first; it holds rows nz-2, nz-1
+    unsigned col, rowb;         // byte offset of row 0; bytes per row
+    int nz;
+    // byte offset of row r, clamped to the column
+    __device__ __forceinline__ unsigned row(int r) const { return col + (unsigned)min(max(r, 0), nz - 1) * rowb; }
+    __device__ __forceinline__ bool valid(int i) const { return act && a + i < nz; }
+};
+
+// The window and end rows of one field's segment.
+template <int MS>
+__device__ __forceinline__ void load_window(const double *F, const Lane &ln, double (&win)[MS + 6], double (&e)[5])
+{
+#pragma unroll
+    for (int k = 0; k < MS + 6; k++) win[k] = ldg(F, ln.row(ln.a - 3 + k));
+#pragma unroll
+    for (int k = 0; k < 5; k++) e[k] = 0.0;
+    if (ln.last) {
+#pragma unroll
+        for (int k = 0; k < 5; k++) e[k] = ldg(F, ln.row(ln.nz - 5 + k));
+    }
+}
+
+// n doubles (even) from global memory to LDS by the whole block, 16 bytes per
+// load, four loads in flight.
+__device__ __forceinline__ void stage_lds(double *dst, const double *src, int n, int tid, int nthr)
+{
+    const double2 *s2 = (const double2 *)src;
+    double2 *d2 = (double2 *)dst;
+    const int n2 = n >> 1;
+    for (int q = tid; q < n2; q += 4 * nthr) {
+        double2 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = s2[min(q + u * nthr, n2 - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (q + u * nthr < n2) d2[q + u * nthr] = v[u];
+    }
+}
+
+__device__ __forceinline__ void zero_lds(double *dst, int n, int tid, int nthr)
+{
+    for (int q = tid; q < n; q += nthr) dst[q] = 0.0;
+}
+
+}  // namespace
+
+namespace d3 {
+
+// Zp: d xi_z/dz (ibc 1) with the z-PML (displacement.f90:400-409), div, p and
+// rho' (:411-415), and rho' g / rho0 for RHS v_z (:458).  Bound: HBM, 48 B per
+// point (xi_z, two x/y-derivatives and c^2 rho0 read, two fields written).
+// 16 columns are one 128-byte line of every row.  us per launch, one-lane
+// sweep -> here: 256x256x300 395 -> 290 (3.3 TB/s of a 4.9 TB/s copy),
+// 128x128x150 182 -> 40, 96x90x100 104 -> 20.
+constexpr int kZpCols = 16;
+template <int MS>
+__global__ __launch_bounds__(512) void k3_zp_seg(Z3 z, ZSeg sg)
+{
+    constexpr int NC = kZpCols, U = MS <= 8 ? MS : 4;
+    extern __shared__ __align__(16) double lds[];
+    const int P = sg.P, hw = sg.hw, nzp = P * MS, LY = 2 * P + 4 * hw + 2, nset = zseg_set_len(P, hw, MS);
+    double *const band = lds, *const tabs = band + 2 * P * (4 * hw + 4);
+    double *const yb = lds + nset;                      // [NC][LY]
+    double *const pf = yb + NC * LY;                    // [6][nzp] stretch, d p0/dz, d rho0/dz, rho0, 1/rho0, g
+    const int tid = threadIdx.x, nthr = blockDim.x, nz = z.nz;
+    const unsigned bl = xcd_block(blockIdx.x, gridDim.x);
+    const int c0 = (int)bl * NC + tid % NC;
+    const bool real = c0 < z.nxy;
+    Lane ln;
+    ln.c = tid % NC;
+    ln.s = min(tid / NC, P - 1);
+    ln.act = tid / NC < P && real;
+    ln.a = ln.s * MS;
+    ln.first = ln.s == 0;
+    ln.last = ln.a + MS > nz - 2;
+    ln.rowb = (unsigned)z.nxy * 8u;
+    ln.col = (unsigned)min(c0, z.nxy - 1) * 8u;
+    ln.nz = nz;
+    double win[MS + 6], e[5];
+    load_window<MS>(z.B, ln, win, e);
+    zero_lds(yb, NC * LY, tid, nthr);
+    stage_lds(lds, sg.img, nset, tid, nthr);
+    for (int q = tid; q < nzp; q += nthr) {
+        const int j = min(q, nz - 1);
+        const double v0 = z.stretch[j], v1 = z.gp0z[j], v2 = z.gr0z[j], v3 = z.rho0[j], v4 = z.rhoinv[j], v5 = z.g[j];
+        pf[q] = v0;
+        pf[nzp + q] = v1;
+        pf[2 * nzp + q] = v2;
+        pf[3 * nzp + q] = v3;
+        pf[4 * nzp + q] = v4;
+        pf[5 * nzp + q] = v5;
+    }
+    __syncthreads();
+    const double *const zt = tabs + seg_kind(ln.s, P) * MS;
+    auto tab = [&](int t, int i) { return zt[t * 3 * MS + i]; };
+    double Y[MS], own[MS];
+    seg_rhs<MS>([&](int k) { return win[k]; }, e, Y, ln.a, nz, ln.first, ln.last, 1, 0.0, 0.0, sg.c1, sg.c2, sg.cb);
+#pragma unroll
+    for (int i = 0; i < MS; i++) own[i] = win[3 + i];
+    seg_solve<MS>(Y, tab);
+    double *const yc = yb + ln.c * LY;
+    if (tid / NC < P) {
+        yc[2 * hw + 2 * ln.s] = Y[0];
+        yc[2 * hw + 2 * ln.s + 1] = Y[MS - 1];
+    }
+    __syncthreads();
+    seg_correct<MS>(Y, ln.s, P, hw, yc, band, tab);
+#pragma unroll
+    for (int i0 = 0; i0 < MS; i0 += U) {
+        double dxi[U], dyi[U], c2r[U], fz[U], az[U], bz[U], ps[U], pb[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const unsigned q = ln.row(ln.a + min(i0 + u, MS - 1));
+            dxi[u] = ldg(z.dxi, q);
+            dyi[u] = ldg(z.dyi, q);
+            c2r[u] = ldg(z.c2rho0, q);
+            fz[u] = 1.0;
+            az[u] = bz[u] = ps[u] = pb[u] = 0.0;
+        }
+        if (ln.a + i0 < z.nb || ln.a + min(i0 + U, MS) > nz - z.nt) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int pj = pml_index(min(ln.a + i0 + u, nz - 1), nz, z.nb, z.nt);
+                if (pj >= 0) {
+                    const unsigned qp = ln.col + (unsigned)pj * ln.rowb;
+                    fz[u] = ldg(z.fz, qp);
+                    az[u] = ldg(z.az, qp);
+                    bz[u] = ldg(z.bz, qp);
+                    ps[u] = ldg(z.psi, qp);
+                    pb[u] = ldg(z.pml, qp);
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = i0 + u;
+            if (i >= MS) break;
+            const int j = ln.a + i;
+            const double *const f = pf + j;
+            double dz = Y[i] * f[0];
+            const double gp = f[nzp] * fz[u], gr = f[2 * nzp] * fz[u];
+            const int pj = pml_index(j, nz, z.nb, z.nt);
+            const bool v = ln.valid(i);
+            if (pj >= 0 && v) stg(z.pnext, ln.col + (unsigned)pj * ln.rowb, pb[u] + z.beta * (az[u] * dz + bz[u] * ps[u]));
+            dz = dz + ps[u];
+            const double div = (dxi[u] + dyi[u]) + dz;
+            const double p = -(c2r[u] * div) - own[i] * gp;
+            const double rho = -(f[3 * nzp] * div) - own[i] * gr;
+            if (v) {
+                const unsigned q = ln.col + (unsigned)j * ln.rowb;
+                stg(z.P, q, p);
+                stg(z.RG, q, f[4 * nzp] * rho * f[5 * nzp]);
+            }
+        }
+    }
+}
+
+// Zv: the z-derivatives of v_x, v_y, v_z (ibc 1) and of p (ibc 0, with the
+// z-PML, :422-431) of the lane's segment, all four kept in registers, then RHS
+// v_i = -2 v0 . grad v_i - d_i p / rho0 (:436-452), RHS v_z - rho' g / rho0
+// (:458) + forcing * source_dep (:460-462), RHS xi_i = v_i (:466-468), rows 1
+// and nz zeroed (:470-473).  The xi updates need only v: they are written as
+// each v window passes.  Bound: HBM, 224 B per point (22 fields read, 6
+// written).  us per launch, one-lane sweep -> here: 256x256x300 1350 -> 1105
+// (4.0 TB/s), 128x128x300 968 -> 360, 128x128x150 497 -> 143, 96x90x100 264 ->
+// 68, 32x32x40 91 -> 19.  Segments of at most 10 rows keep the four derivatives
+// and a row's loads in 256 registers; 19-row segments spilled (1440 us at
+// 256x256x300), and 12 to 16 rows (nz above 320) spill a little and still win
+// (256x256x448 2011 -> 1762).  One lane group per field, which reads v0 once
+// per group, took 1500 us there, and blocks of 8 columns 1750: below 128 bytes
+// a row's piece is half a line.
+template <int MS, int NC>
+__global__ __launch_bounds__(512, 2) void k3_zv_seg(Z3 z, ZSeg sg)
+{
+    constexpr int U = 1;
+    extern __shared__ __align__(16) double lds[];
+    const int P = sg.P, hw = sg.hw, nzp = P * MS, LY = 2 * P + 4 * hw + 2, nset = zseg_set_len(P, hw, MS);
+    double *const yb = lds + 2 * nset;                  // [4][NC][LY]
+    double *const pf = yb + 4 * NC * LY;                // [3][nzp] stretch, 1/rho0, source_dep
+    const int tid = threadIdx.x, nthr = blockDim.x, nz = z.nz;
+    const unsigned bl = xcd_block(blockIdx.x, gridDim.x);
+    const int c0 = (int)bl * NC + tid % NC;
+    Lane ln;
+    ln.c = tid % NC;
+    ln.s = min(tid / NC, P - 1);
+    ln.act = tid / NC < P && c0 < z.nxy;
+    ln.a = ln.s * MS;
+    ln.first = ln.s == 0;
+    ln.last = ln.a + MS > nz - 2;
+    ln.rowb = (unsigned)z.nxy * 8u;
+    ln.col = (unsigned)min(c0, z.nxy - 1) * 8u;
+    ln.nz = nz;
+    zero_lds(yb, 4 * NC * LY, tid, nthr);
+    stage_lds(lds, sg.img, 2 * nset, tid, nthr);
+    for (int q = tid; q < nzp; q += nthr) {
+        const int j = min(q, nz - 1);
+        const double v0 = z.stretch[j], v1 = z.rhoinv[j], v2 = z.srcdep[j];
+        pf[q] = v0;
+        pf[nzp + q] = v1;
+        pf[2 * nzp + q] = v2;
+    }
+    // forcing of this column (physics.f90:678-737 for the adjoint)
+    double forcing = 0.0;
+    if (ln.a <= z.e_rad + 4 && ln.a + MS > z.e_rad - 4 && z.time <= z.src.limit) {
+        const int c = (int)(ln.col >> 3);
+        if (z.src.mode == 1)
+            forcing = (z.time >= 0 && z.time < z.src.nfwd) ? z.src.vr[c] * z.src.fwd[z.time] : 0.0;
+        else if (z.src.mode == 2)
+            forcing = lagrange_forcing(z.src, 0, c, z.nxy, z.time);
+    }
+    __syncthreads();
+    const int kofs = 2 * P * (4 * hw + 4) + seg_kind(ln.s, P) * MS;
+    double Y[4][MS];
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+        const double *const band = lds + (f < 3 ? 0 : nset), *const zt = band + kofs;
+        double win[MS + 6], e[5];
+        load_window<MS>(f < 3 ? z.B + (size_t)f * z.N : z.P, ln, win, e);
+        if (f < 3) {
+            const double *const ax = z.a + (size_t)f * z.N;
+            double *const tx = z.tnext + (size_t)f * z.N, *const rx = z.rhs + (size_t)f * z.N;
+            double bx[MS];
+#pragma unroll
+            for (int i = 0; i < MS; i++) bx[i] = ldg(ax, ln.row(ln.a + i));
+#pragma unroll
+            for (int i = 0; i < MS; i++) {
+                const int j = ln.a + i;
+                const double r = j == 0 || j == nz - 1 ? 0.0 : win[3 + i];
+                if (ln.valid(i)) {
+                    const unsigned q = ln.col + (unsigned)j * ln.rowb;
+                    stg(tx, q, bx[i] + z.beta * r);
+                    if (z.last) stg(rx, q, r);
+                }
+            }
+        }
+        seg_rhs<MS>([&](int k) { return win[k]; }, e, Y[f], ln.a, nz, ln.first, ln.last, f < 3 ? 1 : 0, 0.0, 0.0, sg.c1,
+                    sg.c2, sg.cb);
+        seg_solve<MS>(Y[f], [&](int t, int i) { return zt[t * 3 * MS + i]; });
+        if (tid / NC < P) {
+            double *const yc = yb + (f * NC + ln.c) * LY + 2 * hw + 2 * ln.s;
+            yc[0] = Y[f][0];
+            yc[1] = Y[f][MS - 1];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+        const double *const band = lds + (f < 3 ? 0 : nset), *const zt = band + kofs;
+        seg_correct<MS>(Y[f], ln.s, P, hw, yb + (f * NC + ln.c) * LY, band,
+                        [&](int t, int i) { return zt[t * 3 * MS + i]; });
+    }
+    const size_t N = z.N, np = (size_t)(z.nb + z.nt) * z.nxy;
+#pragma unroll
+    for (int i0 = 0; i0 < MS; i0 += U) {
+        double dx[3][U], dy[3][U], u0[3][U], gp[2][U], rg[U], bv[3][U], az[U], bz[U], ps[U], pb[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const unsigned q = ln.row(ln.a + min(i0 + u, MS - 1));
+#pragma unroll
+            for (int f = 0; f < 3; f++) {
+                dx[f][u] = ldg(z.dxv + f * N, q);
+                dy[f][u] = ldg(z.dyv + f * N, q);
+                bv[f][u] = ldg(z.a + (3 + f) * N, q);
+            }
+            u0[0][u] = ldg(z.v0x, q);
+            u0[1][u] = ldg(z.v0y, q);
+            u0[2][u] = ldg(z.v0z, q);
+            gp[0][u] = ldg(z.dxp, q);
+            gp[1][u] = ldg(z.dyp, q);
+            rg[u] = ldg(z.RG, q);
+            az[u] = bz[u] = ps[u] = pb[u] = 0.0;
+        }
+        if (ln.a + i0 < z.nb || ln.a + min(i0 + U, MS) > nz - z.nt) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int pj = pml_index(min(ln.a + i0 + u, nz - 1), nz, z.nb, z.nt);
+                if (pj >= 0) {
+                    const unsigned qp = ln.col + (unsigned)pj * ln.rowb;
+                    az[u] = ldg(z.az, qp);
+                    bz[u] = ldg(z.bz, qp);
+                    ps[u] = ldg(z.psi + np, qp);
+                    pb[u] = ldg(z.pml + np, qp);
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = i0 + u;
+            if (i >= MS) break;
+            const int j = ln.a + i;
+            const bool edge = j == 0 || j == nz - 1, v = ln.valid(i);
+            const unsigned q = ln.col + (unsigned)j * ln.rowb;
+            const double st = pf[j], ri = pf[nzp + j];
+            double adv[3], gpz = Y[3][i] * st;
+#pragma unroll
+            for (int f = 0; f < 3; f++)
+                adv[f] = -2.0 * ((u0[0][u] * dx[f][u] + u0[1][u] * dy[f][u]) + u0[2][u] * (Y[f][i] * st));
+            const int pj = pml_index(j, nz, z.nb, z.nt);
+            if (pj >= 0 && v)
+                stg(z.pnext + np, ln.col + (unsigned)pj * ln.rowb, pb[u] + z.beta * (az[u] * gpz + bz[u] * ps[u]));
+            gpz = gpz + ps[u];
+            double rhs[3];
+            rhs[0] = edge ? 0.0 : adv[0] - ri * gp[0][u];
+            rhs[1] = edge ? 0.0 : adv[1] - ri * gp[1][u];
+            double rz = adv[2] - ri * gpz;
+            rz = rz - rg[u];
+            const int dk = j - z.e_rad;
+            if (dk >= -4 && dk <= 4) rz = rz + forcing * pf[2 * nzp + j];
+            rhs[2] = edge ? 0.0 : rz;
+            if (v) {
+#pragma unroll
+                for (int f = 0; f < 3; f++) {
+                    stg(z.tnext + (3 + f) * N, q, bv[f][u] + z.beta * rhs[f]);
+                    if (z.last) stg(z.rhs + (3 + f) * N, q, rhs[f]);
+                }
+            }
+        }
+    }
+}
+
+namespace {
+
+size_t zp_lds(const ZSeg &sg)
+{
+    return sizeof(double) * ((size_t)zseg_set_len(sg.P, sg.hw, sg.m) + (size_t)kZpCols * yb_len(sg.P, sg.hw) +
+                             (size_t)6 * sg.P * sg.m);
+}
+size_t zv_lds(const ZSeg &sg, int nc)
+{
+    return sizeof(double) * ((size_t)2 * zseg_set_len(sg.P, sg.hw, sg.m) + (size_t)4 * nc * yb_len(sg.P, sg.hw) +
+                             (size_t)3 * sg.P * sg.m);
+}
+
+// Raises a kernel's dynamic-LDS limit when a launch needs more than the default.
+hipError_t allow_lds(const void *k, size_t n)
+{
+    return n > 64 * 1024 ? hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)n) : hipSuccess;
+}
+
+int lanes(int cols, int P) { return (cols * P + 63) / 64 * 64; }
+
+}  // namespace
+
+bool zseg3_fits(const Z3 &z, const ZSeg &sg)
+{
+    return sg.img && sg.P >= 1 && sg.P <= kZSegP && z.N < ((size_t)1 << 28) && zp_lds(sg) <= 160 * 1024 &&
+           zv_lds(sg, sg.P <= kZSegP / 2 ? 32 : 16) <= 160 * 1024;
+}
+
+hipError_t launch_zp_seg(const Z3 &z, const ZSeg &sg, hipStream_t st)
+{
+    const size_t shm = zp_lds(sg);
+    const dim3 grid((unsigned)((z.nxy + kZpCols - 1) / kZpCols)), block(lanes(kZpCols, sg.P));
+#define L(M)                                                                            \
+    if (sg.m == M) {                                                                    \
+        const hipError_t e = allow_lds((const void *)k3_zp_seg<M>, shm);                \
+        if (e != hipSuccess) return e;                                                  \
+        hipLaunchKernelGGL(k3_zp_seg<M>, grid, block, shm, st, z, sg);                  \
+        return hipGetLastError();                                                       \
+    }
+    SPARC_ZSEG_SIZES(L)
+#undef L
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_zv_seg(const Z3 &z, const ZSeg &sg, hipStream_t st)
+{
+    // 32 columns (256 bytes of each row) while they fill the 256 compute units
+    // and 512 threads: 143 us against 183 with 16 at 128x128x150, 68 against 63
+    // at 96x90x100
+    const int nc = sg.P <= kZSegP / 2 && z.nxy >= 32 * 256 ? 32 : 16;
+    const size_t shm = zv_lds(sg, nc);
+    const dim3 grid((unsigned)((z.nxy + nc - 1) / nc)), block(lanes(nc, sg.P));
+#define L(M)                                                                                 \
+    if (sg.m == M) {                                                                         \
+        const void *k = nc == 32 ? (const void *)k3_zv_seg<M, 32> : (const void *)k3_zv_seg<M, 16>; \
+        const hipError_t e = allow_lds(k, shm);                                              \
+        if (e != hipSuccess) return e;                                                       \
+        if (nc == 32) hipLaunchKernelGGL((k3_zv_seg<M, 32>), grid, block, shm, st, z, sg);   \
+        else hipLaunchKernelGGL((k3_zv_seg<M, 16>), grid, block, shm, st, z, sg);            \
+        return hipGetLastError();                                                            \
+    }
+    SPARC_ZSEG_SIZES(L)
+#undef L
+    return hipErrorInvalidValue;
+}
+
+}  // namespace d3
+}  // namespace sparc
