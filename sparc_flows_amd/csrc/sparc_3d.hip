@@ -460,7 +460,7 @@ struct sparc3d_handle {
                  *d_g = nullptr, *d_srcdep = nullptr;
     double *c2rho0 = nullptr, *az = nullptr, *bz = nullptr, *fz = nullptr;   // fz: PML factor of the gradients below
     const double *gp0z = nullptr, *gr0z = nullptr;    // [nz] d p0/dz, d rho0/dz before the PML factor
-    ZSeg zseg{};                                      // segmented z passes: sets ibc 1, ibc 0 (img null: no such cut of nz)
+    ZSeg zseg{};                                      // tables of the segmented z kernels (img null: no such cut of nz)
     double *v0x = nullptr, *v0y = nullptr, *v0z = nullptr;
     double *a = nullptr, *scr = nullptr, *tmp = nullptr, *pml = nullptr, *psit = nullptr;
     double *DXI = nullptr, *DYI = nullptr, *DX3 = nullptr, *DY3 = nullptr, *P = nullptr, *RG = nullptr,
@@ -531,6 +531,29 @@ static int ddx3(sparc3d_handle *h, const double *in, double *out, int nrows)
 static int ddy3(sparc3d_handle *h, const double *in, double *out, int nplanes)
 {
     RUN3(2, launch_ddy(in, out, nplanes, h->nx, h->ny, h->twy, h->dmy, h->cdy, h->stretchy, h->stream));
+    return SPARC_OK;
+}
+
+// d/dz (dbyd2 of ibc times stretch; filt: ddzkern) of nfields fields: the
+// segmented form, or the one-lane sweeps, whose work buffer holds one field.
+static int ddz3(sparc3d_handle *h, const double *in, double *out, int nfields, int ibc, int filt)
+{
+    ZDer a{};
+    a.in = in;
+    a.out = out;
+    a.ncols = (int)h->nxy;
+    a.nz = h->nz;
+    a.nbatch = nfields;
+    a.ibc = ibc;
+    a.stretch = h->d_stretch;
+    a.filt = filt;
+    if (zder_fits(a, h->zseg)) {
+        HCHECK3(h, launch_zder(a, h->zseg, h->stream));
+        return SPARC_OK;
+    }
+    for (int f = 0; f < nfields; f++)
+        HCHECK3(h, launch_ddz_cols(in + f * h->n, out + f * h->n, (int)h->nxy, h->nz, 1, ibc, h->d_stretch, h->cf,
+                                   h->tri[ibc], h->W, filt, h->stream));
     return SPARC_OK;
 }
 
@@ -708,21 +731,7 @@ static int setup3(sparc3d_handle *h)
         HCHECK3(h, upload(h->bg_mem, &pc, rbet, h->stream));
         h->tri[ibc] = Tri{pa, pb, pc};
     }
-    // the segmented z passes' tables
-    if (const int m = zseg_length(nz)) {
-        const int sets[2] = {1, 0};
-        std::vector<double> img;
-        ZSeg sg{};
-        sg.m = m;
-        sg.P = (nz + m - 1) / m;
-        dbyd2_coefs(nz, sg.c1, sg.c2, sg.cb);
-        if (build_zseg(nz, m, 2, sets, sg.hw, img)) {
-            double *pi = nullptr;
-            HCHECK3(h, upload(h->bg_mem, &pi, img, h->stream));
-            sg.img = pi;
-            h->zseg = sg;
-        }
-    }
+    HCHECK3(h, upload_zseg(h->bg_mem, &h->zseg, nz, kZSegSets, h->stream));
     // z and stretch = 1/dbyd2(z) (initialize.f90:466-470); deltat (:474)
     h->z.resize(nz);
     for (int k = 0; k < nz; k++) h->z[k] = h->model[6 * (size_t)k];
@@ -1206,10 +1215,8 @@ int sparc3d_kernels_add(sparc3d_handle *h, const double *fwd, const double *adj)
     if ((r = ddy3(h, fwd + 3 * N, DY + N, 3 * nz))) return r;
     if ((r = ddy3(h, adj + N, DY + 4 * N, nz))) return r;
     // ddzkern (:648-661): dbyd2 ibc 1, stretch, FILTER_VAR_Z
-    const double *zin[5] = {fwd + 2 * N, fwd + 3 * N, fwd + 4 * N, fwd + 5 * N, adj + 2 * N};
-    for (int i = 0; i < 5; i++)
-        HCHECK3(h, launch_ddz_cols(zin[i], DZ + i * N, (int)h->nxy, nz, 1, 1, h->d_stretch, h->cf, h->tri[1], h->W,
-                                   1, h->stream));
+    if ((r = ddz3(h, fwd + 2 * N, DZ, 4, 1, 1))) return r;     // xi_z, v_x, v_y, v_z
+    if ((r = ddz3(h, adj + 2 * N, DZ + 4 * N, 1, 1, 1))) return r;
     const unsigned blocks = (unsigned)std::min<size_t>((N + 255) / 256, 16384);
     hipLaunchKernelGGL(k3_kern_accum, dim3(blocks), dim3(256), 0, h->stream, fwd, adj, DX, DY, DZ, h->K, N);
     HCHECK3(h, hipGetLastError());
@@ -1229,9 +1236,8 @@ int sparc3d_kernels_end(sparc3d_handle *h, double *kc, double *kpsi, double *kvx
     const size_t N = h->n;
     // the psi kernel's curl (CURL_KERN :832-834, bcz = 0) into the derivative scratch
     double *T1 = h->KD, *T2 = h->KD + N;
-    HCHECK3(h, launch_ddz_cols(h->K + N, T1, (int)h->nxy, h->nz, 1, 0, h->d_stretch, h->cf, h->tri[0], h->W, 1,
-                               h->stream));
-    int r;
+    int r = ddz3(h, h->K + N, T1, 1, 0, 1);
+    if (r) return r;
     if ((r = ddx3(h, h->K + 3 * N, T2, h->ny * h->nz))) return r;
     const unsigned blocks = (unsigned)std::min<size_t>((N + 255) / 256, 16384);
     hipLaunchKernelGGL(k3_kern_final, dim3(blocks), dim3(256), 0, h->stream, h->K, T1, T2, h->krho0, h->kc2, N,
@@ -1294,9 +1300,8 @@ int sparc3d_ddy(sparc3d_handle *h, const double *in, double *out, int nplanes)
 int sparc3d_ddz(sparc3d_handle *h, const double *in, double *out, int nfields, int ibc)
 {
     if (!h || !in || !out || nfields < 1 || ibc < 0 || ibc > 3) return SPARC_E_ARG;
-    for (int f = 0; f < nfields; f++)   // the work buffer holds one field
-        HCHECK3(h, launch_ddz_cols(in + f * h->n, out + f * h->n, (int)h->nxy, h->nz, 1, ibc, h->d_stretch, h->cf,
-                                   h->tri[ibc], h->W, 0, h->stream));
+    const int r = ddz3(h, in, out, nfields, ibc, 0);
+    if (r) return r;
     HCHECK3(h, hipStreamSynchronize(h->stream));
     return SPARC_OK;
 }

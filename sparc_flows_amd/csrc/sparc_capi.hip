@@ -90,6 +90,7 @@ struct sparc_handle {
     int kpair_cap = 0;              // Kc the buffer holds
     Bg bg{};
     Tri tri[4]{};
+    ZSeg zseg{};                    // segmented z-derivative (img null: no such cut of nz)
     State st{};
     double *d_scratch = nullptr;    // [S][nz][nx] general scratch
     double *kbuf = nullptr;         // kernel accumulation: D[8], KC, KX, KZ, H, t1, t2, work
@@ -198,6 +199,24 @@ hipError_t upload(DevArena &ar, double **dst, const std::vector<double> &v, hipS
 }
 
 // GPU z-derivative of [nb][nz][ncols] host data (used by the set-up).
+hipError_t upload_zseg(DevArena &ar, ZSeg *out, int nz, int nset, hipStream_t st)
+{
+    *out = ZSeg{};
+    ZSeg sg{};
+    if (!(sg.m = zseg_length(nz))) return hipSuccess;
+    sg.P = (nz + sg.m - 1) / sg.m;
+    dbyd2_coefs(nz, sg.c1, sg.c2, sg.cb);
+    const int sets[kZSegSetsT] = {0, 1, 2, 3, kZSegT | 1, kZSegT | 2, kZSegT | 3};
+    std::vector<double> img;
+    if (!build_zseg(nz, sg.m, nset, sets, sg.hw, img)) return hipSuccess;
+    double *p = nullptr;
+    const hipError_t e = upload(ar, &p, img, st);
+    if (e != hipSuccess) return e;
+    sg.img = p;
+    *out = sg;
+    return hipSuccess;
+}
+
 static int host_ddz(sparc_handle *h, const std::vector<double> &in, std::vector<double> &out,
                     int ncols, int nbatch, int ibc, bool use_stretch, int tri_ibc)
 {
@@ -519,6 +538,7 @@ static int upload_background(sparc_handle *h)
         HCHECK(h, upload(h->bg_mem, &c, rbet, h->stream));
         h->tri[ibc] = Tri{a, b, c};
     }
+    HCHECK(h, upload_zseg(h->bg_mem, &h->zseg, nz, kZSegSetsT, h->stream));
     HCHECK(h, upload(h->bg_mem, &p, h->rhoinv, h->stream)); h->bg.rhoinv = p;
     {
         std::vector<double> rz(nz);
@@ -1554,15 +1574,40 @@ int sparc_ddx(sparc_handle *h, const double *in, double *out, int nrows)
     return SPARC_OK;
 }
 
+// ddz (or, with filt, ddzkern) of nbatch [nz][nx] fields on the handle's stream:
+// the segmented form wherever it fits, else the one-lane sweeps, which need a
+// work buffer as large as the batch.
+static ZDer zder_args(const sparc_handle *h, const double *in, double *out, int nbatch, int ibc, int filt)
+{
+    ZDer a{};
+    a.in = in;
+    a.out = out;
+    a.ncols = h->nx;
+    a.nz = h->nz;
+    a.nbatch = nbatch;
+    a.ibc = ibc;
+    a.stretch = h->bg.stretch;
+    a.filt = filt;
+    return a;
+}
+static hipError_t ddz_batch(const sparc_handle *h, const double *in, double *out, int nbatch, int ibc, int filt,
+                            double *work)
+{
+    const ZDer a = zder_args(h, in, out, nbatch, ibc, filt);
+    if (zder_fits(a, h->zseg)) return launch_zder(a, h->zseg, h->stream);
+    return launch_ddz_cols(in, out, h->nx, h->nz, nbatch, ibc, h->bg.stretch, h->cf, h->tri[ibc], work, filt,
+                           h->stream);
+}
+
 static int ddz_impl(sparc_handle *h, const double *in, double *out, int nbatch, int ibc, int filt)
 {
     if (!h || !in || !out || nbatch < 1 || ibc < 0 || ibc > 3) return SPARC_E_ARG;
     double *work = nullptr;
-    HCHECK(h, hipMalloc((void **)&work, (size_t)nbatch * h->nz * h->nx * sizeof(double)));
-    HCHECK(h, launch_ddz_cols(in, out, h->nx, h->nz, nbatch, ibc, h->bg.stretch, h->cf, h->tri[ibc], work,
-                              filt, h->stream));
+    if (!zder_fits(zder_args(h, in, out, nbatch, ibc, filt), h->zseg))
+        HCHECK(h, hipMalloc((void **)&work, (size_t)nbatch * h->nz * h->nx * sizeof(double)));
+    HCHECK(h, ddz_batch(h, in, out, nbatch, ibc, filt, work));
     HCHECK(h, hipStreamSynchronize(h->stream));
-    HCHECK(h, hipFree(work));
+    if (work) HCHECK(h, hipFree(work));
     return SPARC_OK;
 }
 
@@ -1586,8 +1631,7 @@ int sparc_ddz_noalloc(sparc_handle *h, const double *in, double *out, int nbatch
                     "sparc_ddz_noalloc: nbatch*nz*nx = " + std::to_string(need) +
                         " doubles exceeds the library scratch of " + std::to_string(kScratchDoubles));
     if (!h->scratch_dev) return fail(h, SPARC_E_STATE, "sparc_ddz_noalloc: scratch address unresolved");
-    HCHECK(h, launch_ddz_cols(in, out, h->nx, h->nz, nbatch, ibc, h->bg.stretch, h->cf, h->tri[ibc],
-                              h->scratch_dev, filt, h->stream));
+    HCHECK(h, ddz_batch(h, in, out, nbatch, ibc, filt, h->scratch_dev));
     return SPARC_OK;
 }
 
@@ -1611,7 +1655,6 @@ int sparc_kernels_add(sparc_handle *h, int n_pairs, const double *fwd, const dou
     const int S = h->S, nt = n_pairs;
     const size_t n2 = (size_t)h->nx * h->nz, n = (size_t)S * n2;
     double *KC = h->kbuf + 8 * n, *KX = KC + n, *KZ = KC + 2 * n, *H = KC + 3 * n;
-    const Tri &tr1 = h->tri[1];
     // pairs per chunk: all of them, within 2 GiB of work buffers (20 fields
     // per pair); one gather, one ddx, one ddz and one accumulation launch
     // per chunk instead of 17 launches per pair
@@ -1634,8 +1677,7 @@ int sparc_kernels_add(sparc_handle *h, int n_pairs, const double *fwd, const dou
         HCHECK(h, launch_gather_pairs(fwd, adj, S, nt, k0, Kc, n2, G, h->stream));
         HCHECK(h, launch_ddx_rows(G, Dx, 4 * Kc * S * h->nz, h->nx, h->bg.tw, h->bg.dmul, h->bg.cdx, h->stretchx,
                                   h->stream));
-        HCHECK(h, launch_ddz_cols(G + 4 * per, Dz, h->nx, h->nz, 4 * Kc * S, 1, h->bg.stretch, h->cf, tr1,
-                                  work, 1, h->stream));
+        HCHECK(h, ddz_batch(h, G + 4 * per, Dz, 4 * Kc * S, 1, 1, work));
         HCHECK(h, launch_kern_accum_pairs(fwd, adj, S, nt, k0, Kc, n2, Dx, Dz, KC, KX, KZ, H, h->stream));
     }
     h->kern_pairs += nt;
@@ -1651,8 +1693,7 @@ int sparc_kernels_end(sparc_handle *h, double *kc, double *kpsi, double *kvx, do
     double *KC = h->kbuf + 8 * n, *KX = KC + n, *KZ = KC + 2 * n, *H = KC + 3 * n;
     double *t1 = h->kbuf + 12 * n, *t2 = h->kbuf + 13 * n, *work = h->kbuf + 14 * n;
     // curl (bcz = 0, kernels.f90:832) and unit scalings (:498-579)
-    HCHECK(h, launch_ddz_cols(KX, t1, h->nx, h->nz, S, 0, h->bg.stretch, h->cf, h->tri[0], work, 1,
-                              h->stream));
+    HCHECK(h, ddz_batch(h, KX, t1, S, 0, 1, work));
     HCHECK(h, launch_ddx_rows(KZ, t2, S * h->nz, h->nx, h->bg.tw, h->bg.dmul, h->bg.cdx, h->stretchx, h->stream));
     const double diml = kRsun, dimc = (double)1e6f, e8 = (double)1e-8f, e5 = (double)1e-5f;
     const double dimen = std::pow(diml * e8 * h->xlength * e8 * dimc * e5, -1.0) * 1.0;
@@ -1678,11 +1719,14 @@ int sparc_kernels(sparc_handle *h, int nt, const double *fwd, const double *adj,
 // ---------------------------------------------------------------------------
 // Exact discrete adjoint (sparc_discrete.hip).
 
-// The dense z-derivative matrices of ibc 1, 2, 3 (stretch included; kept rows
+// Where the z-derivative of nbatch fields does not run segmented: the dense
+// z-derivative matrices of ibc 1, 2, 3 (stretch included; kept rows
 // at 0), their transposes and ibc 3's response to its kept last row, built by
 // the library's compact-FD solve of an identity block.
-static int discrete_matrices(sparc_handle *h, DevArena &ar, DiscreteCtx &c)
+static int discrete_matrices(sparc_handle *h, DevArena &ar, DiscreteCtx &c, int nbatch)
 {
+    c.zseg = h->zseg;
+    if (discrete_segmented(c, nbatch)) return SPARC_OK;
     const int nz = h->nz;
     const size_t nn = (size_t)nz * nz;
     std::vector<double> eye(nn, 0.0), m;
@@ -1735,7 +1779,7 @@ int sparc_discrete_gradient(sparc_handle *h, int maxtime, const double *gvz_dev,
     c.steps = h->steps;
     c.orow = h->o_rad;
     auto done = [&](int r) { (void)hipStreamSynchronize(h->stream); ar.release(); return r; };
-    int r = discrete_matrices(h, ar, c);
+    int r = discrete_matrices(h, ar, c, 2 * h->S);
     if (r) return done(r);
     DiscreteWork w{};
     const size_t S = h->S;
@@ -1797,8 +1841,9 @@ int sparc_ddz_T(sparc_handle *h, const double *in_dev, double *out_dev, int nbat
     DevArena ar;
     DiscreteCtx c{};
     c.d = h->d;
+    c.bg = h->bg;
     c.stream = h->stream;
-    int r = discrete_matrices(h, ar, c);
+    int r = discrete_matrices(h, ar, c, nbatch);
     hipError_t e = r ? hipSuccess : discrete_apply(c, in_dev, out_dev, nbatch, ibc + 2, presetN_bar_dev);
     (void)hipStreamSynchronize(h->stream);
     ar.release();

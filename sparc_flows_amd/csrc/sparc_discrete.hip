@@ -14,9 +14,10 @@
 // Building blocks (all batched over the S sources, fields [S][nz][nx]):
 //   * x-derivatives: the library's FFT row kernel; its transpose is -Dx (the
 //     multiplier i k is odd and the Nyquist bin is dropped);
-//   * z-derivatives and their transposes: the dbyd2 map of each ibc as a
-//     dense nz x nz matrix (built by the library's own compact-FD solve of an
-//     identity block), applied by an LDS-tiled kernel (k_dz_dense);
+//   * z-derivatives and their transposes: the segmented compact-FD solve
+//     (sparc_zseg.hip); for an nz that it does not take, the dbyd2 map of each
+//     ibc as a dense nz x nz matrix (built by the library's own compact-FD
+//     solve of an identity block), applied by an LDS-tiled kernel (k_dz_dense);
 //   * pointwise kernels for the PML, pressure, density and flow terms of the
 //     forward stage (k_fwd_b, k_fwd_c) and of its transpose (k_adj_a,
 //     k_adj_b, k_adj_c), the z filter and its transpose.
@@ -413,12 +414,62 @@ inline dim3 grid1(size_t n, int bs = 256) { return dim3((unsigned)((n + bs - 1) 
         if (e_ != hipSuccess) return e_;             \
     } while (0)
 
-static hipError_t dz_dense(const DiscreteCtx &c, const double *in, double *out, int nbatch, const double *M,
-                           const double *vN, const double *pre, size_t preStride, double preScale)
+static ZDer zder_args(const DiscreteCtx &c, const double *in, double *out, int nbatch, int ibc, bool transposed)
 {
+    ZDer a{};
+    a.in = in;
+    a.out = out;
+    a.ncols = c.d.nx;
+    a.nz = c.d.nz;
+    a.nbatch = nbatch;
+    a.ibc = ibc;
+    a.stretch = c.bg.stretch;
+    a.transposed = transposed;
+    if (transposed) dbyd2_edge_rows(c.d.nz, ibc, a.eb);
+    return a;
+}
+
+bool discrete_segmented(const DiscreteCtx &c, int nbatch)
+{
+    return zder_fits(zder_args(c, nullptr, nullptr, nbatch, 1, true), c.zseg);
+}
+
+// out = Dz_ibc in (ibc 1..3), the kept last row of ibc 3 preScale * pre[b *
+// preStride + x] (0 when pre is null), kept first row of ibc 2 0.
+static hipError_t dz(const DiscreteCtx &c, const double *in, double *out, int nbatch, int ibc, const double *pre,
+                     size_t preStride, double preScale)
+{
+    ZDer a = zder_args(c, in, out, nbatch, ibc, false);
+    if (discrete_segmented(c, nbatch)) {
+        a.pre = pre;
+        a.pre_stride = preStride;
+        a.pre_scale = preScale;
+        a.zero_kept = 1;
+        return launch_zder(a, c.zseg, c.stream);
+    }
     dim3 grid((c.d.nx + kTX - 1) / kTX, (c.d.nz + kTJ - 1) / kTJ, nbatch);
-    hipLaunchKernelGGL(k_dz_dense, grid, dim3(256), 0, c.stream, in, out, c.d.nz, c.d.nx, M, vN, pre, preStride,
-                       preScale);
+    hipLaunchKernelGGL(k_dz_dense, grid, dim3(256), 0, c.stream, in, out, c.d.nz, c.d.nx, c.M[ibc - 1],
+                       pre ? c.vN3 : nullptr, pre, preStride, preScale);
+    return hipGetLastError();
+}
+
+// out = Dz_ibc^T in (ibc 1..3, kept rows 0); prebar (may be null) gets the
+// adjoint of ibc 3's kept last row [nbatch][nx].
+static hipError_t dz_T(const DiscreteCtx &c, const double *in, double *out, int nbatch, int ibc, double *prebar)
+{
+    ZDer a = zder_args(c, in, out, nbatch, ibc, true);
+    if (discrete_segmented(c, nbatch)) {
+        a.prebar = prebar;
+        return launch_zder(a, c.zseg, c.stream);
+    }
+    if (prebar) {
+        hipLaunchKernelGGL(k_colsum_w, grid1((size_t)nbatch * c.d.nx), dim3(256), 0, c.stream, in, c.vN3, prebar,
+                           c.d.nz, c.d.nx, nbatch);
+        DCHK(hipGetLastError());
+    }
+    dim3 grid((c.d.nx + kTX - 1) / kTX, (c.d.nz + kTJ - 1) / kTJ, nbatch);
+    hipLaunchKernelGGL(k_dz_dense, grid, dim3(256), 0, c.stream, in, out, c.d.nz, c.d.nx, c.MT[ibc - 1], nullptr,
+                       nullptr, 0, 0.0);
     return hipGetLastError();
 }
 
@@ -439,14 +490,13 @@ static hipError_t fwd_rhs(const DiscreteCtx &c, const DiscreteWork &w, const dou
     DCHK(ddx(c, Y, w.T0, S * d.nz));
     DCHK(ddx(c, Y + 2 * w.SN, D + w.SN, 2 * S * d.nz));
     // dxi_z/dz (ibc 3, kept last row -dxi_x/dx unstretch), dv_x/dz, dv_z/dz (ibc 1)
-    DCHK(dz_dense(c, Y + w.SN, w.T1, S, c.M[2], c.vN3, w.T0 + (size_t)(d.nz - 1) * d.nx, (size_t)d.nz * d.nx,
-                  -c.unstretch_last));
-    DCHK(dz_dense(c, Y + 2 * w.SN, D + 3 * w.SN, 2 * S, c.M[0], nullptr, nullptr, 0, 0.0));
+    DCHK(dz(c, Y + w.SN, w.T1, S, 3, w.T0 + (size_t)(d.nz - 1) * d.nx, (size_t)d.nz * d.nx, -c.unstretch_last));
+    DCHK(dz(c, Y + 2 * w.SN, D + 3 * w.SN, 2 * S, 1, nullptr, 0, 0.0));
     hipLaunchKernelGGL(k_fwd_b, grid1(w.SN), dim3(256), 0, c.stream, d, c.bg, v, Y, w.T0, w.T1, D, w.T2, w.T3, R);
     DCHK(hipGetLastError());
     // dp/dx, dp/dz (ibc 2, its first row 0)
     DCHK(ddx(c, w.T2, w.T0, S * d.nz));
-    DCHK(dz_dense(c, w.T2, w.T1, S, c.M[1], nullptr, nullptr, 0, 0.0));
+    DCHK(dz(c, w.T2, w.T1, S, 2, nullptr, 0, 0.0));
     hipLaunchKernelGGL(k_fwd_c, grid1(w.SN), dim3(256), 0, c.stream, d, c.bg, v, c.src, t, Y, w.T0, w.T1, w.T3,
                        D + w.SN, R);
     return hipGetLastError();
@@ -492,15 +542,12 @@ static hipError_t bwd_step(const DiscreteCtx &c, const DiscreteWork &w, const do
                            w.Yb);
         DCHK(hipGetLastError());
         DCHK(ddx(c, w.FX, w.DFX, 3 * S * d.nz));
-        DCHK(dz_dense(c, w.FZ, w.DFZ, 2 * S, c.MT[0], nullptr, nullptr, 0, 0.0));
-        DCHK(dz_dense(c, w.GZ, w.DGZ, S, c.MT[1], nullptr, nullptr, 0, 0.0));
+        DCHK(dz_T(c, w.FZ, w.DFZ, 2 * S, 1, nullptr));
+        DCHK(dz_T(c, w.GZ, w.DGZ, S, 2, nullptr));
         hipLaunchKernelGGL(k_adj_b, grid1(w.SN), dim3(256), 0, c.stream, d, c.bg, v, w.Rb, w.DFX, w.DFZ, w.DGZ,
                            w.RHOB, Dst + (size_t)s * 5 * w.SN, w.Yb, w.XZP, w.DXB, w.DZB, G);
         DCHK(hipGetLastError());
-        hipLaunchKernelGGL(k_colsum_w, grid1((size_t)S * d.nx), dim3(256), 0, c.stream, w.DZB, c.vN3, w.PB, d.nz,
-                           d.nx, S);
-        DCHK(hipGetLastError());
-        DCHK(dz_dense(c, w.DZB, w.DZ3B, S, c.MT[2], nullptr, nullptr, 0, 0.0));
+        DCHK(dz_T(c, w.DZB, w.DZ3B, S, 3, w.PB));
         hipLaunchKernelGGL(k_adj_preset, grid1((size_t)S * d.nx), dim3(256), 0, c.stream, w.PB, w.DXB, d.nz, d.nx,
                            S, c.unstretch_last);
         DCHK(hipGetLastError());
@@ -566,7 +613,7 @@ hipError_t discrete_flow_chain(const DiscreteCtx &c, const DiscreteWork &w, cons
     const int n2 = d.nz * d.nx;
     hipLaunchKernelGGL(k_flow_in, grid1(w.SN), dim3(256), 0, c.stream, v, n2, rho0, G, w.FX, w.FZ);
     DCHK(hipGetLastError());
-    DCHK(dz_dense(c, w.FX, w.DFX, d.S, c.MT[0], nullptr, nullptr, 0, 0.0));   // Dz1^T (Gx / rho0)
+    DCHK(dz_T(c, w.FX, w.DFX, d.S, 1, nullptr));   // Dz1^T (Gx / rho0)
     DCHK(ddx(c, w.FZ, w.DFZ, d.S * d.nz));                                   // dx (Gz / rho0)
     hipLaunchKernelGGL(k_flow_out, grid1(w.SN), dim3(256), 0, c.stream, v, n2, rho0, c2, psi, scale, dimc, G,
                        w.DFX, w.DFZ, gpsi, gc);
@@ -578,14 +625,8 @@ hipError_t discrete_apply(const DiscreteCtx &c, const double *in, double *out, i
 {
     // which: 0..2 Dz of ibc 1..3, 3..5 their transposes
     if (which < 0 || which > 5) return hipErrorInvalidValue;
-    const double *M = which < 3 ? c.M[which] : c.MT[which - 3];
-    DCHK(dz_dense(c, in, out, nbatch, M, nullptr, nullptr, 0, 0.0));
-    if (which == 5 && presetN_bar) {
-        hipLaunchKernelGGL(k_colsum_w, grid1((size_t)nbatch * c.d.nx), dim3(256), 0, c.stream, in, c.vN3,
-                           presetN_bar, c.d.nz, c.d.nx, nbatch);
-        DCHK(hipGetLastError());
-    }
-    return hipSuccess;
+    return which < 3 ? dz(c, in, out, nbatch, which + 1, nullptr, 0, 0.0)
+                     : dz_T(c, in, out, nbatch, which - 2, which == 5 ? presetN_bar : nullptr);
 }
 
 }  // namespace sparc

@@ -5,6 +5,7 @@
 #include <vector>
 
 #include "sparc_device.h"
+#include "sparc_zseg.h"
 
 // Device buffers owned by a handle, freed together.
 struct DevArena {
@@ -33,3 +34,6 @@ void make_tri(int N2, int ibc, std::vector<double> &lowr, std::vector<double> &g
               std::vector<double> &rbet);
 // Upload a host vector into a new device buffer of the arena.
 hipError_t upload(DevArena &ar, double **dst, const std::vector<double> &v, hipStream_t st);
+// The z kernels' tables of nz rows (sparc_zseg.h): nset sets, kZSegSets or
+// kZSegSetsT; img stays null where no cut of nz fits.
+hipError_t upload_zseg(DevArena &ar, sparc::ZSeg *sg, int nz, int nset, hipStream_t st);

@@ -1,6 +1,7 @@
 // sparc_launch.h -- host-side launchers of the solver kernels.
 #pragma once
 #include "sparc_device.h"
+#include "sparc_zseg.h"
 
 namespace sparc {
 
@@ -52,6 +53,7 @@ struct DiscreteCtx {
     Bg bg;
     Src src;
     hipStream_t stream;
+    ZSeg zseg;                     // segmented z-derivative and its transpose, where they fit; else:
     const double *M[3], *MT[3];    // the z-derivative of ibc 1, 2, 3 as nz x nz matrices, and their transposes
     const double *vN3;             // ibc 3's response to its kept last row [nz]
     double betas[5], deltat, unstretch_last;
@@ -76,6 +78,9 @@ hipError_t discrete_gradient(const DiscreteCtx &c, const DiscreteWork &w, int ma
 hipError_t discrete_flow_chain(const DiscreteCtx &c, const DiscreteWork &w, const double *G, const double *rho0,
                                const double *c2, const double *psi, double scale, double dimc, double *gpsi,
                                double *gc);
+// Whether the discrete adjoint of this grid takes the segmented z-derivative
+// (otherwise its context needs M, MT and vN3).
+bool discrete_segmented(const DiscreteCtx &c, int nbatch);
 // out = Dz_ibc in (which 0..2) or Dz_ibc^T in (which 3..5) for nbatch fields;
 // for which 5 also the adjoint of the kept last row presetN_bar [nbatch][nx].
 hipError_t discrete_apply(const DiscreteCtx &c, const double *in, double *out, int nbatch, int which,

@@ -158,10 +158,14 @@ bool seg_kind_tables(const SegTables &t, std::vector<double> &out);
 // ---------------------------------------------------------------------------
 // Tables of the z kernels of sparc_zseg.hip: at most kZSegP segments of m rows.
 constexpr int kZSegP = 32;
-// Segment lengths those kernels are instantiated for.
+// Segment lengths of the 3D stage passes, and of the z-derivative, whose one
+// chain of registers takes longer segments as well.
 #define SPARC_ZSEG_SIZES(X) X(4) X(5) X(6) X(7) X(8) X(10) X(12) X(14) X(16)
+#define SPARC_ZDER_SIZES(X) SPARC_ZSEG_SIZES(X) X(19) X(20) X(24) X(28) X(32)
+constexpr int kZSegMax3 = 16;
 // The shortest of them that cuts nz rows into at most kZSegP segments (half as
-// many up to nz = 160, where blocks of twice the columns then fit) whose last holds at least 3 real rows; 0 if there is none (nz > 512, and a few sizes below).
+// many up to nz = 160, where blocks of twice the columns then fit) whose last
+// holds at least 3 real rows; 0 if there is none (nz > 1024).
 int zseg_length(int nz);
 // The device image of nset matrices, one after the other: the banded
 // interface inverse [2P][4hw+4], then the segment tables [5][3][m] by kind,

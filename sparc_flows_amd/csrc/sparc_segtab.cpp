@@ -198,7 +198,7 @@ int zseg_length(int N)
 {
     static const int sizes[] = {
 #define X(v) v,
-        SPARC_ZSEG_SIZES(X)
+        SPARC_ZDER_SIZES(X)
 #undef X
     };
     for (int m : sizes) {

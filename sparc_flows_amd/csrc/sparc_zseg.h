@@ -6,13 +6,40 @@
 
 namespace sparc {
 
-// Tables of one nz on the device (build_zseg): sets of one ibc each, one
-// after the other in img; the right-hand side's coefficients by value.
+// Tables of one nz on the device (build_zseg): the sets of ibc 0, 1, 2, 3, then
+// (2D handles) of the transposed matrices of ibc 1, 2, 3; the right-hand side's
+// coefficients by value.
 struct ZSeg {
     int P, m, hw;
     const double *img;
     double c1, c2, cb[kCB];
 };
+constexpr int kZSegSets = 4, kZSegSetsT = 7;
+
+// The z-derivative (ddz, derivatives.f90:10-24; with filt, ddzkern,
+// kernels.f90:648-661) of nbatch fields [nz][ncols], or its transpose.
+struct ZDer {
+    const double *in;
+    double *out;                // may be in
+    int ncols, nz, nbatch, ibc;
+    const double *stretch;      // [nz], or null: plain dbyd2
+    int filt;                   // pass the result through FILTER_VAR_Z
+    // the kept first / last row of ibc 2 / 3: the row of out, or 0 with
+    // zero_kept, or for ibc 3 pre_scale * pre[b * pre_stride + column] when
+    // pre is given
+    int zero_kept;
+    const double *pre;
+    size_t pre_stride;
+    double pre_scale;
+    // transposed (ibc 1..3, kept rows 0): eb from dbyd2_edge_rows; prebar
+    // [nbatch][ncols] gets the adjoint of ibc 3's kept last row (may be null)
+    int transposed;
+    double eb[20];
+    double *prebar;
+};
+// Whether the segmented form takes it: tables, and 32-bit offsets in a field.
+bool zder_fits(const ZDer &a, const ZSeg &sg);
+hipError_t launch_zder(const ZDer &a, const ZSeg &sg, hipStream_t st);
 
 namespace d3 {
 
@@ -58,10 +85,9 @@ __device__ __forceinline__ int pml_index(int j, int nz, int nb, int nt)
     return j < nb ? j : (j >= nz - nt ? nb + (j - (nz - nt)) : -1);
 }
 
-// Whether the segmented passes take this grid: the tables exist (nz <= 512)
-// and a field spans less than 2^31 bytes (32-bit byte offsets).
+// Whether the segmented passes take this grid: segments of at most kZSegMax3
+// rows (nz <= 512) and a field of less than 2^31 bytes (32-bit byte offsets).
 bool zseg3_fits(const Z3 &z, const ZSeg &sg);
-// sg: sets ibc 1, ibc 0.
 hipError_t launch_zp_seg(const Z3 &z, const ZSeg &sg, hipStream_t st);
 hipError_t launch_zv_seg(const Z3 &z, const ZSeg &sg, hipStream_t st);
 

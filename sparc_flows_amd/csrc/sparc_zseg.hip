@@ -90,6 +90,165 @@ __device__ __forceinline__ void zero_lds(double *dst, int n, int tid, int nthr)
 
 }  // namespace
 
+// The z-derivative of a batch of fields, or its transpose: D = S A^-1 B with B
+// dbyd2's right-hand side, A its tridiagonal matrix and S the stretch, so D^T =
+// B^T A^-T S: the solve by the transposed tables first, then B^T, a stencil on
+// the solved column (its four edge rows apart), through an LDS tile.  Bound:
+// HBM for a large batch (16 B per point), latency for a small one.  us per
+// launch, one-lane Thomas sweep (or, in the discrete adjoint, the product with
+// the dense nz x nz matrix) -> here: one 128x150 field 52 -> 6, 16 fields of
+// 256x300 58 -> 7.5 (transposed 9.3).
+constexpr int kZdCols = 16;
+template <int MS, bool TR>
+__global__ __launch_bounds__(512) void k_zder(ZDer z, ZSeg sg)
+{
+    constexpr int NC = kZdCols;
+    extern __shared__ __align__(16) double lds[];
+    const int P = sg.P, hw = sg.hw, nzp = P * MS, LY = 2 * P + 4 * hw + 2, nset = zseg_set_len(P, hw, MS);
+    double *const band = lds, *const yb = lds + nset;       // [NC][LY]
+    double *const tile = yb + NC * LY + 2 * NC;             // filter, transpose: [nzp] rows of NC, two more before and after
+    const int tid = threadIdx.x, nthr = blockDim.x, nz = z.nz;
+    const int c0 = (int)blockIdx.x * NC + tid % NC;
+    const size_t fo = (size_t)blockIdx.y * nz * z.ncols;
+    Lane ln;
+    ln.c = tid % NC;
+    ln.s = min(tid / NC, P - 1);
+    ln.act = tid / NC < P && c0 < z.ncols;
+    ln.a = ln.s * MS;
+    ln.first = ln.s == 0;
+    ln.last = ln.a + MS > nz - 2;
+    ln.rowb = (unsigned)z.ncols * 8u;
+    ln.col = (unsigned)min(c0, z.ncols - 1) * 8u;
+    ln.nz = nz;
+    const bool seg = tid / NC < P;
+    double Y[MS], st[MS];
+#pragma unroll
+    for (int i = 0; i < MS; i++) st[i] = z.stretch ? z.stretch[min(ln.a + i, nz - 1)] : 1.0;
+    double win[MS + 6], e[5], p0 = 0.0, pN = 0.0;
+    if (TR) {
+#pragma unroll
+        for (int i = 0; i < MS; i++) Y[i] = ldg(z.in + fo, ln.row(ln.a + i));
+    } else {
+        load_window<MS>(z.in + fo, ln, win, e);
+        if (z.ibc == 2 && !z.zero_kept) p0 = ldg(z.out + fo, ln.row(0));
+        if (z.ibc == 3 && (z.pre || !z.zero_kept))
+            pN = z.pre ? z.pre_scale * z.pre[(size_t)blockIdx.y * z.pre_stride + (ln.col >> 3)]
+                       : ldg(z.out + fo, ln.row(nz - 1));
+    }
+    zero_lds(yb, NC * LY, tid, nthr);
+    stage_lds(lds, sg.img + (size_t)(TR ? 3 + z.ibc : z.ibc) * nset, nset, tid, nthr);
+    if (TR && tid < 2 * NC) {                               // zero rows around the tile
+        tile[tid - 2 * NC] = 0.0;
+        tile[nzp * NC + tid] = 0.0;
+    }
+    __syncthreads();
+    const double *const zt = band + 2 * P * (4 * hw + 4) + seg_kind(ln.s, P) * MS;
+    auto tab = [&](int t, int i) { return zt[t * 3 * MS + i]; };
+    if (TR) {
+#pragma unroll
+        for (int i = 0; i < MS; i++) Y[i] = ln.a + i < nz ? Y[i] * st[i] : 0.0;
+    } else {
+        seg_rhs<MS>([&](int k) { return win[k]; }, e, Y, ln.a, nz, ln.first, ln.last, z.ibc, p0, pN, sg.c1, sg.c2,
+                    sg.cb);
+    }
+    seg_solve<MS>(Y, tab);
+    double *const yc = yb + ln.c * LY;
+    if (seg) {
+        yc[2 * hw + 2 * ln.s] = Y[0];
+        yc[2 * hw + 2 * ln.s + 1] = Y[MS - 1];
+    }
+    __syncthreads();
+    seg_correct<MS>(Y, ln.s, P, hw, yc, band, tab);
+    double *const oc = z.out + fo;
+    if (!TR) {
+#pragma unroll
+        for (int i = 0; i < MS; i++) Y[i] = Y[i] * st[i];
+        if (!z.filt) {
+#pragma unroll
+            for (int i = 0; i < MS; i++)
+                if (ln.valid(i)) stg(oc, ln.col + (unsigned)(ln.a + i) * ln.rowb, Y[i]);
+            return;
+        }
+    }
+    // rows 0, 1, nz-2, nz-1 of the solved column enter B^T by their own
+    // coefficients: kept apart, and zero in the tile
+    double *const ed = yb;                                  // [4][NC], once every lane has left yb
+    __syncthreads();
+    if (seg) {
+#pragma unroll
+        for (int i = 0; i < MS; i++) {
+            const int j = ln.a + i, er = j < 2 ? j : j - nz + 4;
+            const bool edge = TR && (j < 2 || (j >= nz - 2 && j < nz));
+            tile[j * NC + ln.c] = edge || j >= nz ? 0.0 : Y[i];
+            if (edge) ed[er * NC + ln.c] = Y[i];
+            if (TR && z.prebar && z.ibc == 3 && j == nz - 1 && ln.act)
+                z.prebar[(size_t)blockIdx.y * z.ncols + c0] = Y[i];
+        }
+    }
+    __syncthreads();
+    if (!ln.act) return;
+    const double *const t = tile + ln.c;
+#pragma unroll
+    for (int i = 0; i < MS; i++) {
+        const int j = ln.a + i;
+        if (j >= nz) break;
+        double v;
+        if (TR) {
+            v = sg.c1 * (t[(j - 1) * NC] - t[(j + 1) * NC]) + sg.c2 * (t[(j - 2) * NC] - t[(j + 2) * NC]);
+            const int k = j < 5 ? j : j - nz + 5;
+            if (j < 5) v += z.eb[k] * ed[ln.c] + z.eb[5 + k] * ed[NC + ln.c];
+            if (j >= nz - 5) v += z.eb[10 + j - nz + 5] * ed[2 * NC + ln.c] + z.eb[15 + j - nz + 5] * ed[3 * NC + ln.c];
+        } else if (j == 0 || j == nz - 1) {
+            v = Y[i];
+        } else if (j <= 4 || j >= nz - 5) {                // FILTER_VAR_Z (kernels.f90:891-928)
+            v = 0.5 * (t[(j + 1) * NC] + t[(j - 1) * NC]);
+        } else {
+            v = filt11(t, (size_t)j * NC, NC);
+        }
+        stg(oc, ln.col + (unsigned)j * ln.rowb, v);
+    }
+}
+
+namespace {
+
+size_t zder_lds(const ZDer &a, const ZSeg &sg)
+{
+    return sizeof(double) * ((size_t)zseg_set_len(sg.P, sg.hw, sg.m) + (size_t)kZdCols * yb_len(sg.P, sg.hw) +
+                             (a.filt || a.transposed ? (size_t)kZdCols * (sg.P * sg.m + 4) : 0));
+}
+// Raises a kernel's dynamic-LDS limit when a launch needs more than the default.
+hipError_t allow_lds(const void *k, size_t n)
+{
+    return n > 64 * 1024 ? hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)n) : hipSuccess;
+}
+int lanes(int cols, int P) { return (cols * P + 63) / 64 * 64; }
+
+}  // namespace
+
+bool zder_fits(const ZDer &a, const ZSeg &sg)
+{
+    return sg.img && sg.P <= kZSegP && (size_t)a.nz * a.ncols < ((size_t)1 << 28) && a.nbatch <= 65535 &&
+           zder_lds(a, sg) <= 160 * 1024;
+}
+
+hipError_t launch_zder(const ZDer &a, const ZSeg &sg, hipStream_t st)
+{
+    const size_t shm = zder_lds(a, sg);
+    const dim3 grid((unsigned)((a.ncols + kZdCols - 1) / kZdCols), (unsigned)a.nbatch), block(lanes(kZdCols, sg.P));
+#define L(M)                                                                                     \
+    if (sg.m == M) {                                                                             \
+        const void *k = a.transposed ? (const void *)k_zder<M, true> : (const void *)k_zder<M, false>; \
+        const hipError_t e = allow_lds(k, shm);                                                  \
+        if (e != hipSuccess) return e;                                                           \
+        if (a.transposed) hipLaunchKernelGGL((k_zder<M, true>), grid, block, shm, st, a, sg);    \
+        else hipLaunchKernelGGL((k_zder<M, false>), grid, block, shm, st, a, sg);                \
+        return hipGetLastError();                                                                \
+    }
+    SPARC_ZDER_SIZES(L)
+#undef L
+    return hipErrorInvalidValue;
+}
+
 namespace d3 {
 
 // Zp: d xi_z/dz (ibc 1) with the z-PML (displacement.f90:400-409), div, p and
@@ -125,7 +284,7 @@ __global__ __launch_bounds__(512) void k3_zp_seg(Z3 z, ZSeg sg)
     double win[MS + 6], e[5];
     load_window<MS>(z.B, ln, win, e);
     zero_lds(yb, NC * LY, tid, nthr);
-    stage_lds(lds, sg.img, nset, tid, nthr);
+    stage_lds(lds, sg.img + nset, nset, tid, nthr);         // ibc 1
     for (int q = tid; q < nzp; q += nthr) {
         const int j = min(q, nz - 1);
         const double v0 = z.stretch[j], v1 = z.gp0z[j], v2 = z.gr0z[j], v3 = z.rho0[j], v4 = z.rhoinv[j], v5 = z.g[j];
@@ -237,7 +396,7 @@ __global__ __launch_bounds__(512, 2) void k3_zv_seg(Z3 z, ZSeg sg)
     ln.col = (unsigned)min(c0, z.nxy - 1) * 8u;
     ln.nz = nz;
     zero_lds(yb, 4 * NC * LY, tid, nthr);
-    stage_lds(lds, sg.img, 2 * nset, tid, nthr);
+    stage_lds(lds, sg.img, 2 * nset, tid, nthr);            // ibc 0, ibc 1
     for (int q = tid; q < nzp; q += nthr) {
         const int j = min(q, nz - 1);
         const double v0 = z.stretch[j], v1 = z.rhoinv[j], v2 = z.srcdep[j];
@@ -259,7 +418,7 @@ __global__ __launch_bounds__(512, 2) void k3_zv_seg(Z3 z, ZSeg sg)
     double Y[4][MS];
 #pragma unroll
     for (int f = 0; f < 4; f++) {
-        const double *const band = lds + (f < 3 ? 0 : nset), *const zt = band + kofs;
+        const double *const band = lds + (f < 3 ? nset : 0), *const zt = band + kofs;
         double win[MS + 6], e[5];
         load_window<MS>(f < 3 ? z.B + (size_t)f * z.N : z.P, ln, win, e);
         if (f < 3) {
@@ -291,7 +450,7 @@ __global__ __launch_bounds__(512, 2) void k3_zv_seg(Z3 z, ZSeg sg)
     __syncthreads();
 #pragma unroll
     for (int f = 0; f < 4; f++) {
-        const double *const band = lds + (f < 3 ? 0 : nset), *const zt = band + kofs;
+        const double *const band = lds + (f < 3 ? nset : 0), *const zt = band + kofs;
         seg_correct<MS>(Y[f], ln.s, P, hw, yb + (f * NC + ln.c) * LY, band,
                         [&](int t, int i) { return zt[t * 3 * MS + i]; });
     }
@@ -377,19 +536,11 @@ size_t zv_lds(const ZSeg &sg, int nc)
                              (size_t)3 * sg.P * sg.m);
 }
 
-// Raises a kernel's dynamic-LDS limit when a launch needs more than the default.
-hipError_t allow_lds(const void *k, size_t n)
-{
-    return n > 64 * 1024 ? hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)n) : hipSuccess;
-}
-
-int lanes(int cols, int P) { return (cols * P + 63) / 64 * 64; }
-
 }  // namespace
 
 bool zseg3_fits(const Z3 &z, const ZSeg &sg)
 {
-    return sg.img && sg.P >= 1 && sg.P <= kZSegP && z.N < ((size_t)1 << 28) && zp_lds(sg) <= 160 * 1024 &&
+    return sg.img && sg.m <= kZSegMax3 && sg.P <= kZSegP && z.N < ((size_t)1 << 28) && zp_lds(sg) <= 160 * 1024 &&
            zv_lds(sg, sg.P <= kZSegP / 2 ? 32 : 16) <= 160 * 1024;
 }
 

@@ -58,3 +58,56 @@ def test_two_steps_match_oracle(nx, ny, nz, npml):
     assert rel_l2(s.pml().cpu().numpy(), o.pmlvars) < 1e-11
     for f in range(6):
         assert rel_l2(scr[f], o.scr[f]) < 1e-11, f
+
+
+# (nz, ibc): every table set; short and long segments, the sizes around a new
+# segment length, a last segment of three rows, the longest segment (1024)
+@pytest.mark.parametrize("nx,nz", [(18, 16), (75, 60), (64, 35), (130, 150), (256, 300), (33, 337), (16, 512),
+                                   (16, 700), (20, 1024)])
+def test_z_derivative_and_filter_match_oracle(nx, nz):
+    """ddz for every ibc with kept rows, ddzkern, and the transpose by <D f, w>
+    = <f, D^T w>, on batches of three fields."""
+    import dataclasses
+
+    import oracle
+    from sparc_flows_amd.solver import Sparc
+    from tests.cases import small_case
+
+    p, bg, _, _ = small_case(nx=64, nz=nz, npml=4, flow=False, dc=False)
+    p = dataclasses.replace(p, nx=nx, npmlhor=2)
+    s, o = Sparc(p, bg), oracle.Oracle(p, bg)
+    rng = np.random.default_rng(nz)
+    z = np.linspace(0.0, 1.0, nz)[None, :, None]
+    x = np.arange(nx)[None, None, :]
+    f = sum(np.sin((2 + 3 * k) * z + rng.uniform(0, 6, (3, 1, nx))) * np.cos(0.3 * k * x) for k in range(5))
+    w = rng.standard_normal(f.shape)
+    ft, wt = (torch.as_tensor(v, device="cuda") for v in (f, w))
+    # what the kernels share with the one-lane sweeps: the set-up's stretch
+    ramp = np.broadcast_to(np.arange(nz, dtype=np.float64)[:, None], (nz, nx))
+    lib = s.ddz(torch.as_tensor(np.ascontiguousarray(ramp), device="cuda"), 1).cpu().numpy()
+    ratio = lib / o.ddz(np.ascontiguousarray(ramp), 1)
+    for ibc in range(4):
+        pre = np.zeros_like(f)
+        pre[:, 0], pre[:, -1] = rng.standard_normal((2, 3, nx))
+        got = s.ddz(ft, ibc, torch.as_tensor(pre, device="cuda")).cpu().numpy()
+        ref = np.stack([o.ddz(f[k], ibc, pre[k]) for k in range(3)]) * ratio
+        assert rel_l2(got, ref) < 1e-11, ibc
+    got, plain = s.ddz_kern(ft, 1).cpu().numpy(), s.ddz(ft, 1).cpu().numpy()
+    c = [0.75390625, 0.41015625 / 2, -0.234375 / 2, 0.087890625 / 2, -0.01953125 / 2, 0.001953125 / 2]
+    ref = plain.copy()
+    ref[:, 1:-1] = 0.5 * (plain[:, 2:] + plain[:, :-2])
+    ref[:, 5:nz - 5] = c[0] * plain[:, 5:nz - 5] + sum(
+        c[k] * (plain[:, 5 - k:nz - 5 - k] + plain[:, 5 + k:nz - 5 + k]) for k in range(1, 6))
+    assert rel_l2(got, ref) < 1e-14
+    for ibc in (1, 2, 3):
+        lhs = (s.ddz(ft, ibc) * wt).sum()
+        t = s.ddz_T(wt, ibc)
+        t, pb = t if ibc == 3 else (t, None)
+        size = float((s.ddz(ft, ibc) * wt).abs().sum())
+        assert abs(float(lhs - (ft * t).sum())) < 1e-12 * size, ibc
+        if ibc == 3:                 # the kept last row's adjoint: <D(f; r), w> - <D(f; 0), w> = <r, pb>
+            pre = torch.zeros_like(ft)
+            pre[:, -1] = 1.0 + torch.arange(nx, device="cuda")
+            d = ((s.ddz(ft, 3, pre) - s.ddz(ft, 3)) * wt).sum()
+            r = (pre[:, -1] * pb).sum()
+            assert abs(float(d - r)) < 1e-9 * float((pre[:, -1] * pb).abs().sum())
