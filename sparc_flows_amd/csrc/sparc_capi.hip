@@ -92,10 +92,8 @@ struct sparc_handle {
     Tri tri[4]{};
     ZSeg zseg{};                    // segmented z-derivative (img null: no such cut of nz)
     State st{};
-    double *d_scratch = nullptr;    // [S][nz][nx] general scratch
     double *kbuf = nullptr;         // kernel accumulation: D[8], KC, KX, KZ, H, t1, t2, work
     long kern_pairs = 0;
-    double *d_scratch2 = nullptr;
     int *tctr = nullptr;
 
     // sources
@@ -538,7 +536,7 @@ static int upload_background(sparc_handle *h)
         HCHECK(h, upload(h->bg_mem, &c, rbet, h->stream));
         h->tri[ibc] = Tri{a, b, c};
     }
-    HCHECK(h, upload_zseg(h->bg_mem, &h->zseg, nz, kZSegSetsT, h->stream));
+    if (!h->zseg.img) HCHECK(h, upload_zseg(h->st_mem, &h->zseg, nz, kZSegSetsT, h->stream));   // depends on nz only
     HCHECK(h, upload(h->bg_mem, &p, h->rhoinv, h->stream)); h->bg.rhoinv = p;
     {
         std::vector<double> rz(nz);
@@ -551,6 +549,17 @@ static int upload_background(sparc_handle *h)
     HCHECK(h, upload(h->bg_mem, &p, h->gr0, h->stream)); h->bg.gr0 = p;
     HCHECK(h, upload(h->bg_mem, &p, h->v0x, h->stream)); h->bg.v0x = p;
     HCHECK(h, upload(h->bg_mem, &p, h->v0z, h->stream)); h->bg.v0z = p;
+    {
+        // row-pair copies of the column pass's coefficient arrays
+        const double *const src[3] = {h->bg.c2rho0, h->bg.v0x, h->bg.v0z};
+        const double **const dst[3] = {&h->bg.c2rho0_p, &h->bg.v0x_p, &h->bg.v0z_p};
+        for (int k = 0; k < 3; k++) {
+            double *q = nullptr;
+            HCHECK(h, h->bg_mem.alloc(&q, (size_t)h->d.nzq * h->nx));
+            HCHECK(h, launch_pair_copy(src[k], q, h->nx, nz, h->stream));
+            *dst[k] = q;
+        }
+    }
     HCHECK(h, upload(h->bg_mem, &p, h->g, h->stream)); h->bg.g = p;
     HCHECK(h, upload(h->bg_mem, &p, h->az, h->stream)); h->bg.az = p;
     HCHECK(h, upload(h->bg_mem, &p, h->bz, h->stream)); h->bg.bz = p;
@@ -627,49 +636,31 @@ static int build_seg(sparc_handle *h, int m, SegTab &sg)
     sg.P = P;
     sg.m = m;
     sg.nzp = nzp;
-    std::vector<double> ztab((size_t)kZT * nzp + kCB, 0.0);
-    {
-        double c1, c2;
-        dbyd2_coefs(N, c1, c2, ztab.data() + (size_t)kZT * nzp);
-    }
     // z profiles; rho0, d rho0/dz, d p0/dz and 1/rho0 come from the 1D model
     // and are the same in every column
+    std::vector<double> prof((size_t)kZF * nzp, 0.0);
     for (int j = 0; j < N; j++) {
         const size_t q = (size_t)j * h->nx;
-        ztab[(size_t)0 * nzp + j] = h->stretch[j];
-        ztab[(size_t)1 * nzp + j] = h->g[j];
-        ztab[(size_t)17 * nzp + j] = h->rho0[q];
-        ztab[(size_t)18 * nzp + j] = h->gr0z[j];
-        ztab[(size_t)19 * nzp + j] = h->gp0z[j];
-        ztab[(size_t)20 * nzp + j] = h->rhoinv[q];
+        const double v[kZF] = {h->stretch[j], h->g[j], h->rho0[q], h->gr0z[j], h->gp0z[j], h->rhoinv[q]};
+        for (int r = 0; r < kZF; r++) prof[(size_t)r * nzp + j] = v[r];
         for (int i = 1; i < h->nx; i++)
             if (h->rho0[q + i] != h->rho0[q] || h->rhoinv[q + i] != h->rhoinv[q] ||
                 h->gr0[q + i] != h->gr0z[j] * h->fdec[q + i] || h->gp0[q + i] != h->gp0z[j] * h->fdec[q + i])
                 return fail(h, SPARC_E_ARG, "background density / pressure vary along x");
     }
-    SegTables t;
-    if (!build_seg_tables(N, m, t)) return fail(h, SPARC_E_ARG, "singular interface system");
-    std::copy(t.slots.begin(), t.slots.end(), ztab.begin() + (size_t)2 * nzp);   // rows 2-16
+    SegRows t;
+    if (!build_seg_rows(N, m, t)) return fail(h, SPARC_E_ARG, "singular interface system");
     sg.hw = t.hw;
-    const std::vector<double> &band = t.band;
+    sg.E = t.E;
+    sg.nk = seg_band_kinds(P, t.E);
+    std::vector<double> stage(t.rows), kt;
+    if (!seg_kind_tables(t, kt)) return fail(h, SPARC_E_ARG, "interior segment tables differ");
+    stage.insert(stage.end(), kt.begin(), kt.end());
+    stage.insert(stage.end(), prof.begin(), prof.end());
+    double c1, c2, cb[kCB];
+    dbyd2_coefs(N, c1, c2, cb);
+    stage.insert(stage.end(), cb, cb + kCB);
     double *p = nullptr;
-    HCHECK(h, upload(h->bg_mem, &p, ztab, h->stream));
-    sg.ztab = p;
-    HCHECK(h, upload(h->bg_mem, &p, band, h->stream));
-    sg.Minv = p;
-    std::vector<double> stage(band);
-    {
-        // the segment tables of the first, an interior and the last segment,
-        // then the profiles
-        std::vector<double> kt;
-        if (!seg_kind_tables(t, kt)) return fail(h, SPARC_E_ARG, "interior segment tables differ");
-        static_assert(kZS == 15, "segment-table rows");
-        stage.insert(stage.end(), kt.begin(), kt.end());
-        for (int r = 0; r < kZF; r++)
-            stage.insert(stage.end(), ztab.begin() + (size_t)stage_prow(r) * nzp,
-                         ztab.begin() + (size_t)(stage_prow(r) + 1) * nzp);
-        stage.insert(stage.end(), ztab.begin() + (size_t)kZT * nzp, ztab.begin() + (size_t)kZT * nzp + kCB);
-    }
     HCHECK(h, upload(h->bg_mem, &p, stage, h->stream));
     sg.stage = p;
     return SPARC_OK;
@@ -712,7 +703,7 @@ static int setup_seg(sparc_handle *h)
 
 static int alloc_state(sparc_handle *h)
 {
-    const size_t f = (size_t)h->S * h->nz * h->nx;
+    const size_t f = (size_t)h->S * h->d.nzq * h->nx;
     const size_t pz = (size_t)2 * h->S * h->d.nzpml * h->nx;
     const size_t px = (size_t)2 * h->S * h->nz * h->d.nph;
     DevArena &m = h->st_mem;
@@ -732,10 +723,7 @@ static int alloc_state(sparc_handle *h)
     HCHECK(h, m.alloc(&s.p, f));
     HCHECK(h, m.alloc(&s.rvx, f));
     HCHECK(h, m.alloc(&s.topbc, (size_t)h->S * h->nx));
-    HCHECK(h, m.alloc(&s.w_rho, f));
     HCHECK(h, m.alloc(&s.discard, 256));
-    HCHECK(h, m.alloc(&h->d_scratch, f));
-    HCHECK(h, m.alloc(&h->d_scratch2, f));
     double *t = nullptr;
     HCHECK(h, m.alloc(&t, 1));
     h->tctr = (int *)t;
@@ -744,7 +732,7 @@ static int alloc_state(sparc_handle *h)
 
 static int zero_state(sparc_handle *h)
 {
-    const size_t f = (size_t)h->S * h->nz * h->nx;
+    const size_t f = (size_t)h->S * h->d.nzq * h->nx;
     const size_t pz = (size_t)2 * h->S * h->d.nzpml * h->nx;
     const size_t px = (size_t)2 * h->S * h->nz * h->d.nph;
     State &s = h->st;
@@ -840,7 +828,7 @@ static int enqueue_step(sparc_handle *h, int toff, bool filt_vx, const Sink &sk)
         if (r) return r;
     }
     if (sk.norm2 && !h->profiling)
-        HCHECK(h, launch_vz_norm2(s.a[3], d.S, (size_t)d.nz * d.nx, clk, sk, h->stream));
+        HCHECK(h, launch_vz_norm2(s.a[3], d.S, (size_t)d.nzq * d.nx, clk, sk, h->stream));
     return SPARC_OK;
 }
 
@@ -882,7 +870,7 @@ int sparc_create(const sparc_config *cfg, sparc_handle **out)
         return SPARC_E_ARG;
     }
     if ((double)cfg->nsrc * nz * nx >= (double)(1 << 27)) {
-        // the column pass addresses [2][S][nz][nx] arrays with 32-bit byte offsets
+        // the column pass addresses [S][nzq][nx] arrays with 32-bit byte offsets
         g_create_err = "sparc_create: nsrc * nz * nx must stay below 2^27 points";
         return SPARC_E_ARG;
     }
@@ -901,7 +889,7 @@ int sparc_create(const sparc_config *cfg, sparc_handle **out)
     h->model.assign(cfg->model, cfg->model + 6 * (size_t)nz);
     if (cfg->c2d) h->c2d.assign(cfg->c2d, cfg->c2d + (size_t)nx * nz);
     if (cfg->psi) h->psi.assign(cfg->psi, cfg->psi + (size_t)nx * nz);
-    h->d = Dims{nx, nz, h->S, h->nb, h->nt, h->nb + h->nt, h->nh, 2 * h->nh};
+    h->d = Dims{nx, nz, h->S, (nz + 1) / 2 * 2, h->nb, h->nt, h->nb + h->nt, h->nh, 2 * h->nh};
     h->steps = (int)std::floor(h->outputcad / h->timestep);      // driver.f90:214
     h->cfs = (int)std::floor(h->cadforcing / h->timestep);       // initialize.f90:991
     int ndev = 0;
@@ -1513,8 +1501,7 @@ int sparc_save_checkpoint(sparc_handle *h, void *dev)
     const size_t f = (size_t)h->S * h->nz * h->nx;
     const size_t pz = (size_t)2 * h->S * h->d.nzpml * h->nx, px = (size_t)2 * h->S * h->nz * h->d.nph;
     double *o = (double *)dev;
-    for (int i = 0; i < 4; i++)
-        HCHECK(h, hipMemcpyAsync(o + i * f, h->st.a[i], f * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
+    HCHECK(h, launch_state_copy(h->d, h->st, o, 0, h->stream));
     HCHECK(h, hipMemcpyAsync(o + 4 * f, h->st.pz_base, pz * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
     HCHECK(h, hipMemcpyAsync(o + 4 * f + pz, h->st.px_base, px * sizeof(double), hipMemcpyDeviceToDevice,
                              h->stream));
@@ -1527,8 +1514,7 @@ int sparc_load_checkpoint(sparc_handle *h, const void *dev)
     const size_t f = (size_t)h->S * h->nz * h->nx;
     const size_t pz = (size_t)2 * h->S * h->d.nzpml * h->nx, px = (size_t)2 * h->S * h->nz * h->d.nph;
     const double *o = (const double *)dev;
-    for (int i = 0; i < 4; i++)
-        HCHECK(h, hipMemcpyAsync(h->st.a[i], o + i * f, f * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
+    HCHECK(h, launch_state_copy(h->d, h->st, const_cast<double *>(o), 1, h->stream));
     // the stage copies of the PML variables equal their bases between steps
     for (double *dst : {h->st.pz_base, h->st.pz_tmp})
         HCHECK(h, hipMemcpyAsync(dst, o + 4 * f, pz * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
@@ -1540,20 +1526,14 @@ int sparc_load_checkpoint(sparc_handle *h, const void *dev)
 int sparc_get_state(sparc_handle *h, double *a_dev)
 {
     if (!h || !a_dev) return SPARC_E_ARG;
-    const size_t f = (size_t)h->S * h->nz * h->nx;
-    for (int i = 0; i < 4; i++)
-        HCHECK(h, hipMemcpyAsync(a_dev + i * f, h->st.a[i], f * sizeof(double), hipMemcpyDeviceToDevice,
-                                 h->stream));
+    HCHECK(h, launch_state_copy(h->d, h->st, a_dev, 0, h->stream));
     return SPARC_OK;
 }
 
 int sparc_set_state(sparc_handle *h, const double *a_dev)
 {
     if (!h || !a_dev) return SPARC_E_ARG;
-    const size_t f = (size_t)h->S * h->nz * h->nx;
-    for (int i = 0; i < 4; i++)
-        HCHECK(h, hipMemcpyAsync(h->st.a[i], a_dev + i * f, f * sizeof(double), hipMemcpyDeviceToDevice,
-                                 h->stream));
+    HCHECK(h, launch_state_copy(h->d, h->st, const_cast<double *>(a_dev), 1, h->stream));
     return SPARC_OK;
 }
 

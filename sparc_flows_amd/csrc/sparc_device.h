@@ -2,8 +2,13 @@
 // the solver kernels: the register/LDS FFT used by the x-derivative and the
 // compact-FD (dbyd2) coefficient set used by the z-derivative.
 //
-// Layout in HBM: every field of every source is an [S][nz][nx] array of
-// doubles, x fastest (the reference's column-major a(nx,1,nz) per source).
+// Layout in HBM: every field of every source that crosses the library's boundary
+// is an [S][nz][nx] array of doubles, x fastest (the reference's column-major
+// a(nx,1,nz) per source).  The fields that only the row and column passes see
+// (the state, its stage copy and the arrays they hand each other) hold two
+// consecutive rows side by side, [S][nzq/2][nx][2] with nzq = nz rounded up to
+// even: a lane of the column pass moves two rows of its column in one 16-byte
+// access, and the two rows of a pair make full lines for the row pass.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -13,6 +18,7 @@ namespace sparc {
 // Problem geometry.
 struct Dims {
     int nx, nz, S;            // grid and number of sources in the batch
+    int nzq;                  // rows of a row-pair array: nz rounded up to even
     int npmlbot, npmltop, nzpml;
     int nh, nph;              // horizontal PML width and 2*nh
 };
@@ -25,6 +31,7 @@ struct Bg {
     const double *az, *bz;                                 // [nzpml][nx]
     const double *fz;                                      // [nzpml][nx] PML factor of d p0/dz, d rho0/dz
     const double *ax, *bx;                                 // [nz][nph]
+    const double *c2rho0_p, *v0x_p, *v0z_p;                // row-pair copies for the column pass
     const double *rho0_src;                                // [nx] rho0 at the injection row
     const double *eyekx;                                   // [nx/2+1]
     const double *dmul;                                    // [nx] bin multiplier (see fft_deriv_team)
@@ -53,38 +60,37 @@ struct Tri {
 // segment are identity padding).  Each segment is solved locally (rbl, gl:
 // Thomas factors restarted at the segment start) and corrected with the spikes
 // V (response to the row above the segment) and W (to the row below), weighted
-// by the interface values from the exact inverse Minv of the 2P x 2P
-// interface system.  ztab rows (each nzp = P*m long): 0 stretch, 1 g, then
-// for slot 0 (ibc 1), 1 (ibc 2), 2 (ibc 3): lowr, rbl, gl, V, W (rows 2-16),
-// then the x-independent profiles rho0, d rho0/dz, d p0/dz, 1/rho0 (17-20).
+// by the interface values from the exact inverse of the 2P x 2P interface
+// system.
 constexpr int kSegMax = 64;
-constexpr int kZT = 21;     // then the kCB boundary-row coefficients (sparc_seg.h)
-// The column pass keeps in LDS the kZS segment-table rows of the three dbyd2
-// sets (ztab rows 2-16) for three segments only, [kZS][3][m]: the first, an
-// interior one and the last.  Every interior segment's tables are the same
-// (the coefficients are constant away from the boundary rows and each
-// segment's factorization restarts at its start; the host checks it).  Then
-// the kZF epilogue profiles stretch, g, rho0, d rho0/dz, d p0/dz, 1/rho0,
-// [kZF][nzp] (ztab rows stage_prow(r)).
+// The column pass keeps in LDS, for the three dbyd2 sets (ibc 1, 2, 3), the
+// interface rows by kind [3][nk][2][4hw+4] (sparc_seg.h, seg_band_kind) and the
+// kZS segment-table rows (5 slot + k, k: lowr, rbl, gl, V, W) for three segments
+// only, [kZS][3][m]: the first, an interior one and the last.  Every interior
+// segment's tables are the same (the coefficients are constant away from the
+// boundary rows and each segment's factorization restarts at its start; the
+// host checks it).  Then the kZF epilogue profiles stretch, g, rho0, d rho0/dz,
+// d p0/dz, 1/rho0, [kZF][nzp], and the kCB boundary-row coefficients.
 constexpr int kZS = 15, kZF = 6;
-__host__ __device__ inline int stage_prow(int r) { return r == 0 ? 0 : (r == 1 ? 1 : 15 + r); }
 struct SegTab {
-    int P, m, hw, nzp;              // segments, rows per segment, Minv window, P*m
-    const double *ztab;             // [kZT][nzp], then [kCB]
-    const double *Minv;             // [3][2P][4hw+4]: row k of each inverse, entries 2(k/2-hw)+w
-    const double *stage;            // the column pass's LDS image: Minv, [kZS][3][m] segment tables, [kZF][nzp] profiles, [kCB]
+    int P, m, hw, nzp;              // segments, rows per segment, half-width of the interface rows, P*m
+    int E, nk;                      // end segments with interface rows of their own, kinds of them
+    const double *stage;            // the column pass's LDS image, in the order above
 };
 
-// Prognostic state and work arrays of a batch (device pointers).
+// Element (row k, column x) of one source's row-pair field.
+__host__ __device__ inline size_t pair_index(int nx, int k, int x) { return ((size_t)(k >> 1) * nx + x) * 2 + (k & 1); }
+
+// Prognostic state and work arrays of a batch (device pointers); "pairs":
+// [S][nzq/2][nx][2].
 struct State {
-    double *a[4];           // xi_x, xi_z, v_x, v_z   [S][nz][nx]
+    double *a[4];           // xi_x, xi_z, v_x, v_z   pairs
     double *t[4];           // RK stage state
     double *vx_unf;         // v_x after the final update, before the z filter
     double *pz_base, *pz_tmp;  // [2][S][nzpml][nx]  (psivz, psip)
     double *px_base, *px_tmp;  // [2][S][nz][nph]    (psivx, psi_gradp_x)
-    double *dxixdx, *dxvx, *dxvz, *p, *rvx;  // [S][nz][nx]
+    double *dxixdx, *dxvx, *dxvz, *p, *rvx;  // pairs
     double *topbc;          // [S][nx]
-    double *w_rho;          // partial RHS v_z between column-pass phases [S][nz][nx]
     double *discard;        // >= 256 doubles: target of stores from padding rows
 };
 
@@ -653,6 +659,16 @@ struct FwdSweep {
 // ---------------------------------------------------------------------------
 // Helpers shared by the pass kernels.
 
+// A block's logical number: the hardware deals consecutive blocks to the eight
+// XCDs in turn; this gives each XCD one contiguous stretch, so that blocks that
+// share 128-byte lines meet in one L2.
+__device__ __forceinline__ unsigned xcd_block(unsigned id, unsigned n)
+{
+    const unsigned q = n >> 3, r = n & 7, x = id & 7;
+    return x * q + min(x, r) + (id >> 3);
+}
+
+
 // 11-point z filter (physics2d.f90:517-533, kernels.f90:911-918) at row k of
 // a column whose row stride is s.
 __device__ __forceinline__ double filt11(const double *__restrict__ a, size_t q, size_t s)
@@ -665,25 +681,25 @@ __device__ __forceinline__ double filt11(const double *__restrict__ a, size_t q,
 }
 
 // FILTER_VARS_2D value of row k, column x (HORIZONTAL_PMLS: columns
-// npmlhor..nx-npmlhor+1 and rows 6..nz-1, 1-based, are rewritten).
-__device__ __forceinline__ double filter_vars_2d_at(const double *__restrict__ a, size_t q, int k,
-                                                    int x, int nx, int nz, int nh)
-{
-    if (k < 5 || k > nz - 2 || x < nh - 1 || x > nx - nh) return a[q];
-    if (k <= nz - 6) return filt11(a, q, (size_t)nx);
-    return 0.5 * (a[q + nx] + a[q - nx]);
-}
-
-// The same value with all eleven rows loaded (row indices clamped to the
-// column) and the form selected afterwards, so that a wave whose lanes take
+// npmlhor..nx-npmlhor+1 and rows 6..nz-1, 1-based, are rewritten) of one
+// source's row-pair field a, with all eleven rows loaded (pairs clamped to
+// the column) and the form selected afterwards, so that a wave whose lanes take
 // different forms issues one set of loads instead of one per form.
-__device__ __forceinline__ double filter_vars_2d_sel(const double *__restrict__ a, size_t q, int k,
-                                                     int x, int nx, int nz, int nh)
+__device__ __forceinline__ double filter_vars_2d_sel(const double *__restrict__ a, int k, int x, int nx, int nz, int nh)
 {
-    const size_t q0 = q - (size_t)k * nx;       // row 0 of this column
-    double w[11];
+    // the six row pairs that hold rows k-5 .. k+5, then those rows by the parity of k
+    const int h0 = (k - 5) >> 1, hl = (nz - 1) >> 1;   // floor: k - 5 may be negative
+    double2 p[6];
 #pragma unroll
-    for (int u = 0; u < 11; u++) w[u] = a[q0 + (size_t)min(max(k - 5 + u, 0), nz - 1) * nx];
+    for (int u = 0; u < 6; u++) p[u] = *(const double2 *)(a + ((size_t)min(max(h0 + u, 0), hl) * nx + x) * 2);
+    double w[11];
+    const bool odd = k & 1;                            // k - 5 even: the window starts a pair
+#pragma unroll
+    for (int u = 0; u < 11; u++) {
+        const double e = u & 1 ? p[u >> 1].y : p[u >> 1].x;              // row 2 h0 + u
+        const double o = u & 1 ? p[(u + 1) >> 1].x : p[u >> 1].y;        // row 2 h0 + u + 1
+        w[u] = odd ? e : o;
+    }
     const double f11 = 0.75390625 * w[5] + 0.5 * 0.41015625 * (w[4] + w[6]) +
                        0.5 * -0.234375 * (w[3] + w[7]) +
                        0.5 * 0.087890625 * (w[2] + w[8]) +

@@ -21,14 +21,6 @@
 namespace sparc {
 
 // ---------------------------------------------------------------------------
-// small helpers
-
-__device__ __forceinline__ size_t fidx(const Dims &d, int b, int k, int x)
-{
-    return ((size_t)b * d.nz + k) * d.nx + x;
-}
-
-// ---------------------------------------------------------------------------
 // Generic z-derivative (ddz, derivatives.f90:10-24) of ncols columns of an
 // [nz][ncols] array (x fastest); one lane per column.  stretch may be null
 // (plain dbyd2).  For ibc 2 / 3 the preset boundary row is read from out.
@@ -146,7 +138,7 @@ __global__ __launch_bounds__(64) void k_ddx_rows(const double *__restrict__ in,
 // 64 N2 (circ_deriv_row); lane slots past nx load column nx-1 and store
 // nothing.
 template <int NX, int MODE, int N1 = (NX < 0 ? 64 : FftShape<(NX < 0 ? 16 : NX)>::N1)>
-__global__ __launch_bounds__(64) void k_row(Dims d, Bg bg, State st, RowArgs ra, Clock clk, Sink sink)
+__global__ __launch_bounds__(64, NX == 256 && N1 == 16 ? 2 : 1) void k_row(Dims d, Bg bg, State st, RowArgs ra, Clock clk, Sink sink)
 {
     constexpr bool kAny = NX < 0;
     static_assert(!kAny || N1 == 64, "the any-nx form runs one row on 64 lanes");
@@ -179,13 +171,16 @@ __global__ __launch_bounds__(64) void k_row(Dims d, Bg bg, State st, RowArgs ra,
         }
     }
     const int team = threadIdx.x / N1, t = threadIdx.x % N1;
-    const int r = blockIdx.x * TEAMS + team;
+    // each XCD takes one contiguous stretch of rows: the two rows of a pair share
+    // their lines
+    const int r = (int)xcd_block(blockIdx.x, gridDim.x) * TEAMS + team;
     const bool valid = r < d.S * d.nz;
     const int rc = valid ? r : d.S * d.nz - 1;     // clamped row: loads stay in bounds
     const int b = rc / d.nz, k = rc % d.nz;
     const int nz = d.nz, nh = d.nh, nph = d.nph;
     const int time = clock_t_(clk);
-    const size_t rowq = ((size_t)b * nz + k) * nxr;
+    // row k of source b: element x at rowq + 2 x of a row-pair array
+    const size_t rowq = (size_t)b * d.nzq * nxr + pair_index(nxr, k, 0);
     const size_t pxq0 = ((size_t)b * nz + k) * nph;             // psivx row
     const size_t pxq1 = ((size_t)(d.S + b) * nz + k) * nph;     // psi_gradp_x row
     double *const dump = st.discard + threadIdx.x;              // target of invalid-row stores
@@ -255,25 +250,25 @@ __global__ __launch_bounds__(64) void k_row(Dims d, Bg bg, State st, RowArgs ra,
 #pragma unroll
                 for (int j2 = 0; j2 < N2; j2++) {
                     const int x = colx(j2);
-                    vx[j2] = filter_vars_2d_sel(st.vx_unf, rowq + x, k, x, nxr, nz, nh);
+                    vx[j2] = filter_vars_2d_sel(st.vx_unf + (size_t)b * d.nzq * nxr, k, x, nxr, nz, nh);
                 }
             } else {
 #pragma unroll
-                for (int j2 = 0; j2 < N2; j2++) vx[j2] = st.a[2][rowq + colx(j2)];
+                for (int j2 = 0; j2 < N2; j2++) vx[j2] = st.a[2][rowq + 2 * colx(j2)];
             }
 #pragma unroll
             for (int j2 = 0; j2 < N2; j2++) {
-                re[j2] = ra.xi_x[rowq + colx(j2)];
+                re[j2] = ra.xi_x[rowq + 2 * colx(j2)];
                 im[j2] = vx[j2];
             }
         } else {
 #pragma unroll
             for (int j2 = 0; j2 < N2; j2++) {
                 const int x = colx(j2);
-                const double v = ra.filt_vx ? filter_vars_2d_sel(st.vx_unf, rowq + x, k, x, nxr, nz, nh)
-                                            : st.a[2][rowq + x];
+                const double v = ra.filt_vx ? filter_vars_2d_sel(st.vx_unf + (size_t)b * d.nzq * nxr, k, x, nxr, nz, nh)
+                                            : st.a[2][rowq + 2 * x];
                 vx[j2] = v;
-                re[j2] = ra.xi_x[rowq + x];
+                re[j2] = ra.xi_x[rowq + 2 * x];
                 im[j2] = v;
             }
         }
@@ -285,7 +280,7 @@ __global__ __launch_bounds__(64) void k_row(Dims d, Bg bg, State st, RowArgs ra,
 #pragma unroll
             for (int j2 = 0; j2 < N2; j2++) {
                 const int x = colx(j2);
-                *(ok(j2) ? &st.a[2][rowq + x] : dump) = vx[j2];
+                *(ok(j2) ? &st.a[2][rowq + 2 * x] : dump) = vx[j2];
                 if (snap && ok(j2))
                     sink.snap[((((size_t)b * sink.nsnap + sslot) * sink.nfield + fslot) * nz + k) * nxr + x] = vx[j2];
             }
@@ -297,30 +292,30 @@ __global__ __launch_bounds__(64) void k_row(Dims d, Bg bg, State st, RowArgs ra,
         double zr[N2], zi[N2];
 #pragma unroll
         for (int j2 = 0; j2 < N2; j2++) {
-            zr[j2] = ra.v_z[rowq + colx(j2)];
+            zr[j2] = ra.v_z[rowq + 2 * colx(j2)];
             zi[j2] = 0.0;
         }
         SPARC_FFT_DERIV(zr, zi, t, lds[team], stw, sdm, bg.stretchx);
 #pragma unroll
         for (int j2 = 0; j2 < N2; j2++) {
             const int x = colx(j2);
-            *(ok(j2) ? &st.dxvx[rowq + x] : dump) = im[j2];
-            *(ok(j2) ? &st.dxvz[rowq + x] : dump) = zr[j2];
+            *(ok(j2) ? &st.dxvx[rowq + 2 * x] : dump) = im[j2];
+            *(ok(j2) ? &st.dxvz[rowq + 2 * x] : dump) = zr[j2];
         }
     } else {
         // dx p (stage s) paired with dx xi_x (stage s+1, or nothing in MODE 2)
 #pragma unroll
         for (int j2 = 0; j2 < N2; j2++) {
             const int x = colx(j2);
-            re[j2] = st.p[rowq + x];
-            im[j2] = MODE == 1 ? ra.xi_x[rowq + x] : 0.0;
+            re[j2] = st.p[rowq + 2 * x];
+            im[j2] = MODE == 1 ? ra.xi_x[rowq + 2 * x] : 0.0;
         }
         double rvx0[N2], avx[N2], rinv[N2];
 #pragma unroll
         for (int j2 = 0; j2 < N2; j2++) {
             const int x = colx(j2);
-            rvx0[j2] = st.rvx[rowq + x];
-            avx[j2] = st.a[2][rowq + x];
+            rvx0[j2] = st.rvx[rowq + 2 * x];
+            avx[j2] = st.a[2][rowq + 2 * x];
             rinv[j2] = bg.rhoinv_z[k];
         }
         pin_pre();
@@ -351,7 +346,7 @@ __global__ __launch_bounds__(64) void k_row(Dims d, Bg bg, State st, RowArgs ra,
             rvx = (k == 0 || x == 0 || x == nxr - 1) ? 0.0 : rvx;
             const double v = avx[j2] + ra.bx2 * rvx;
             vx[j2] = v;
-            *(ok(j2) ? &ra.v_x_out[rowq + x] : dump) = v;
+            *(ok(j2) ? &ra.v_x_out[rowq + 2 * x] : dump) = v;
             if (snap && ok(j2))
                 sink.snap[((((size_t)b * sink.nsnap + sslot) * sink.nfield +
                             (sink.adjoint ? 2 : 4)) * nz + k) * nxr + x] = rvx;
@@ -362,14 +357,14 @@ __global__ __launch_bounds__(64) void k_row(Dims d, Bg bg, State st, RowArgs ra,
 #pragma unroll
             for (int j2 = 0; j2 < N2; j2++) {
                 wr[j2] = vx[j2];
-                wi[j2] = ra.v_z[rowq + colx(j2)];
+                wi[j2] = ra.v_z[rowq + 2 * colx(j2)];
             }
             SPARC_FFT_DERIV(wr, wi, t, lds[team], stw, sdm, bg.stretchx);
 #pragma unroll
             for (int j2 = 0; j2 < N2; j2++) {
                 const int x = colx(j2);
-                *(ok(j2) ? &st.dxvx[rowq + x] : dump) = wr[j2];
-                *(ok(j2) ? &st.dxvz[rowq + x] : dump) = wi[j2];
+                *(ok(j2) ? &st.dxvx[rowq + 2 * x] : dump) = wr[j2];
+                *(ok(j2) ? &st.dxvz[rowq + 2 * x] : dump) = wi[j2];
             }
 #pragma unroll
             for (int j2 = 0; j2 < N2; j2++) re[j2] = im[j2];
@@ -397,28 +392,50 @@ __global__ __launch_bounds__(64) void k_row(Dims d, Bg bg, State st, RowArgs ra,
             }
             dx = pml ? d2 : dx;
         }
-        *(ok(j2) ? &st.dxixdx[rowq + x] : dump) = dx;
+        *(ok(j2) ? &st.dxixdx[rowq + 2 * x] : dump) = dx;
     }
 }
 
-// v_x filter of the last step of a run (the next row pass would do it).
-__global__ __launch_bounds__(64) void k_finalize_vx(Dims d, State st, Clock clk, Sink sink)
+// v_x filter of the last step of a run (the next row pass would do it): one
+// lane per point (one per column, walking its rows, took 127 us at 256x300).
+__global__ __launch_bounds__(256) void k_finalize_vx(Dims d, State st, Clock clk, Sink sink)
 {
-    const int x = blockIdx.x * 64 + threadIdx.x;
-    const int b = blockIdx.y;
+    const int x = blockIdx.x * 256 + threadIdx.x, j = blockIdx.y, b = blockIdx.z;
     if (x >= d.nx) return;
     const int nx = d.nx, nz = d.nz;
     const int tp = clock_t_(clk) - 1;
     const int sslot = sink.snap ? out_slot(tp, clk.steps, sink.k0, sink.nsnap) : -1;
-    const bool snap = sslot >= 0;
-    for (int j = 0; j < nz; j++) {
-        const size_t q = ((size_t)b * nz + j) * nx + x;
-        const double v = filter_vars_2d_at(st.vx_unf, q, j, x, nx, nz, d.nh);
-        st.a[2][q] = v;
-        if (snap)
-            sink.snap[((((size_t)b * sink.nsnap + sslot) * sink.nfield +
-                        (sink.adjoint ? 0 : 2)) * nz + j) * nx + x] = v;
+    const size_t fb = (size_t)b * d.nzq * nx;
+    const double v = filter_vars_2d_sel(st.vx_unf + fb, j, x, nx, nz, d.nh);
+    st.a[2][fb + pair_index(nx, j, x)] = v;
+    if (sslot >= 0)
+        sink.snap[((((size_t)b * sink.nsnap + sslot) * sink.nfield + (sink.adjoint ? 0 : 2)) * nz + j) * nx + x] = v;
+}
+
+// The four state fields between their row-pair arrays and plain
+// [4][S][nz][nx] (checkpoints, get_state / set_state): one lane per column of a
+// row pair.
+__global__ __launch_bounds__(256) void k_state_copy(Dims d, State st, double *__restrict__ plain, int load)
+{
+    const int x = blockIdx.x * 256 + threadIdx.x, h = blockIdx.y, f = blockIdx.z / d.S, b = blockIdx.z - f * d.S;
+    if (x >= d.nx) return;
+    double *const q = st.a[f] + (size_t)b * d.nzq * d.nx + pair_index(d.nx, 2 * h, x);
+    double *const p = plain + (((size_t)f * d.S + b) * d.nz + 2 * h) * d.nx + x;
+    const bool two = 2 * h + 1 < d.nz;
+    if (load) {
+        q[0] = p[0];
+        q[1] = two ? p[d.nx] : 0.0;
+    } else {
+        p[0] = q[0];
+        if (two) p[d.nx] = q[1];
     }
+}
+
+// A plain [nz][nx] array to a row-pair array (an odd nz's pad row 0).
+__global__ __launch_bounds__(256) void k_pair_copy(const double *__restrict__ in, double *__restrict__ out, int nx, int nz)
+{
+    const int x = blockIdx.x * 256 + threadIdx.x, k = blockIdx.y;
+    if (x < nx) out[pair_index(nx, k, x)] = k < nz ? in[(size_t)k * nx + x] : 0.0;
 }
 
 __global__ void k_tick(int *tctr, int inc)
@@ -659,11 +676,21 @@ hipError_t launch_row(int mode, const Dims &d, const Bg &bg, const State &s, con
     return hipGetLastError();
 }
 
-hipError_t launch_finalize_vx(const Dims &d, const State &s, const Clock &c, const Sink &sk,
-                              hipStream_t st)
+hipError_t launch_finalize_vx(const Dims &d, const State &s, const Clock &c, const Sink &sk, hipStream_t st)
 {
-    dim3 grid((d.nx + 63) / 64, d.S);
-    hipLaunchKernelGGL(k_finalize_vx, grid, dim3(64), 0, st, d, s, c, sk);
+    hipLaunchKernelGGL(k_finalize_vx, dim3((d.nx + 255) / 256, d.nz, d.S), dim3(256), 0, st, d, s, c, sk);
+    return hipGetLastError();
+}
+
+hipError_t launch_pair_copy(const double *in, double *out, int nx, int nz, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_pair_copy, dim3((nx + 255) / 256, (nz + 1) / 2 * 2), dim3(256), 0, st, in, out, nx, nz);
+    return hipGetLastError();
+}
+
+hipError_t launch_state_copy(const Dims &d, const State &s, double *plain, int load, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_state_copy, dim3((d.nx + 255) / 256, d.nzq / 2, 4 * d.S), dim3(256), 0, st, d, s, plain, load);
     return hipGetLastError();
 }
 

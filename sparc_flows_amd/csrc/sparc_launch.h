@@ -18,17 +18,23 @@ hipError_t launch_row(int mode, const Dims &d, const Bg &bg, const State &s, con
                       const Clock &c, const Sink &sk, hipStream_t st, int wide);
 // Segmented column pass, one lane per (column, segment, field); tc in
 // {1, 2, 4, 8, 16} columns per block, ms = rows per segment, one of
-// SPARC_COLSEG_SIZES.
-#define SPARC_COLSEG_SIZES(X) X(4) X(6) X(8) X(10) X(12) X(16) X(19) X(20) X(24)
+// SPARC_COLSEG_SIZES (even: segments are whole row pairs).
+#define SPARC_COLSEG_SIZES(X) X(4) X(6) X(8) X(10) X(12) X(16) X(18) X(20) X(24)
 hipError_t colseg_init();
-// Whether a column-pass block of tc columns fits: its threads (3 lane groups
-// of at most 128) and its dynamic LDS (after colseg_init, the device maximum).
+// Whether the column pass runs its one-lane form (k_colone) on this batch.
+bool col_one_lane(const Dims &d, int ms);
+// Whether a column-pass block of tc columns fits: its threads (one lane per
+// column and segment, at most 512, or 3 lane groups of at most 128) and its dynamic LDS (after colseg_init, the device maximum).
 bool colsplit_fits(int tc, const Dims &d, const SegTab &sg);
 hipError_t launch_colsplit(int tc, int ms, const Dims &d, const Bg &bg, const DbyCoef &cf, const SegTab &sg,
                            const State &s, const ColArgs &ca, const Src &src, const Clock &c, const Sink &sk,
                            hipStream_t st);
 hipError_t launch_finalize_vx(const Dims &d, const State &s, const Clock &c, const Sink &sk,
                               hipStream_t st);
+// The state fields to (load 0) or from (load 1) a plain [4][S][nz][nx] array.
+hipError_t launch_state_copy(const Dims &d, const State &s, double *plain, int load, hipStream_t st);
+// A plain [nz][nx] array to a row-pair array.
+hipError_t launch_pair_copy(const double *in, double *out, int nx, int nz, hipStream_t st);
 hipError_t launch_tick(int *tctr, int inc, hipStream_t st);
 // sk.norm2 slot of the step at clock c: the sum of v_z^2 of each source.
 hipError_t launch_vz_norm2(const double *vz, int S, size_t n2, const Clock &c, const Sink &sk, hipStream_t st);

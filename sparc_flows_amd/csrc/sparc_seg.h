@@ -116,6 +116,37 @@ SPARC_HD void seg_correct(double (&Y)[MS], int s, int P, int hw, const double *y
     for (int i = 0; i < MS; i++) Y[i] = Y[i] - Lp * tab(3, i) - Fn * tab(4, i);
 }
 
+// The interface rows of one segment by kind: away from the ends of the column
+// the interface inverse repeats from segment to segment, so the column pass
+// keeps the rows of the first E and the last E segments and one interior pair.
+SPARC_HD int seg_band_kind(int s, int P, int E) { return s < E ? s : (s >= P - E ? 2 * E + 1 - (P - s) : E); }
+SPARC_HD int seg_band_kinds(int P, int E) { return 2 * E + 1 < P ? 2 * E + 1 : P; }
+
+// seg_correct from the segment's own pair of rows: rows[0 .. nw), nw = 4 hw + 4,
+// gives L_{s-1} from the end values of segments s-1-hw .. s+hw, rows[nw .. 2 nw)
+// F_{s+1} from those of s+1-hw .. s+2+hw.
+template <int MS, int U = 2, typename Tab>
+SPARC_HD void seg_correct_rows(double (&Y)[MS], int s, int P, int hw, const double *yp, const double *rows, Tab tab)
+{
+    const int nw = 4 * hw + 4;
+    const double *r1 = rows, *y1 = yp + 2 * (s > 0 ? s - 1 : 0);
+    const double *r2 = rows + nw, *y2 = yp + 2 * (s < P - 1 ? s + 1 : P - 1);
+    double a0 = 0.0, a1 = 0.0, b0 = 0.0, b1 = 0.0;
+#pragma unroll U
+    for (int w = 0; w < nw; w += 4) {
+        const Dbl2 pA = ld2(r1 + w), pB = ld2(r1 + w + 2), uA = ld2(y1 + w), uB = ld2(y1 + w + 2);
+        const Dbl2 qA = ld2(r2 + w), qB = ld2(r2 + w + 2), vA = ld2(y2 + w), vB = ld2(y2 + w + 2);
+        a0 += pA.x * uA.x + pB.x * uB.x;
+        a1 += pA.y * uA.y + pB.y * uB.y;
+        b0 += qA.x * vA.x + qB.x * vB.x;
+        b1 += qA.y * vA.y + qB.y * vB.y;
+    }
+    const double Lp = s > 0 ? a0 + a1 : 0.0;
+    const double Fn = s < P - 1 ? b0 + b1 : 0.0;
+#pragma unroll
+    for (int i = 0; i < MS; i++) Y[i] = Y[i] - Lp * tab(3, i) - Fn * tab(4, i);
+}
+
 // Length of one column's end-value buffer: 2P values between 2hw and 2hw+2 zeros.
 inline int yb_len(int P, int hw) { return 2 * P + 4 * hw + 2; }
 
@@ -143,6 +174,18 @@ struct SegTables {
 };
 // false if the interface system is singular.
 bool build_seg_tables(int nz, int m, SegTables &t);
+// The same for the column pass: slots, P, m, nzp, and the interface rows by
+// kind, rows [3][seg_band_kinds][2][4hw+4], with hw from the entries above 1e-19
+// of their row maximum (500 times below the rounding of the sums they enter)
+// and E the smallest for which every interior pair equals the middle one to
+// 1e-18 of its largest entry.
+struct SegRows {
+    int P = 0, m = 0, nzp = 0, hw = 0, E = 0;
+    std::vector<double> slots, rows;
+};
+bool build_seg_rows(int nz, int m, SegRows &t);
+// seg_kind_tables of its slots.
+bool seg_kind_tables(const SegRows &t, std::vector<double> &out);
 
 // Segment kind of segment s of P: 0 the first, 2 the last, 1 any other.
 // Every interior segment has the same tables (the dbyd2 coefficients are

@@ -88,9 +88,9 @@ namespace {
 // The five segment tables of one tridiagonal matrix (sub- and super-diagonals
 // lo, up of N rows, diagonal 1), rows [5][nzp] at tabs, and the exact inverse
 // of its 2P x 2P interface system; widens hw to the largest distance in
-// segments to an entry of the inverse above 1e-24 of its row maximum.
+// segments to an entry of the inverse above cut of its row maximum.
 bool seg_one(int N, int m, const std::vector<double> &lo, const std::vector<double> &up, double *tabs,
-             std::vector<double> &Minv, int &hw)
+             std::vector<double> &Minv, int &hw, double cut = 1e-24)
 {
     const int P = (N + m - 1) / m;
     const int nzp = P * m, n2 = 2 * P;
@@ -134,7 +134,7 @@ bool seg_one(int N, int m, const std::vector<double> &lo, const std::vector<doub
         double rm = 0.0;
         for (int q = 0; q < n2; q++) rm = std::max(rm, std::fabs(Minv[(size_t)k * n2 + q]));
         for (int q = 0; q < n2; q++)
-            if (std::fabs(Minv[(size_t)k * n2 + q]) > 1e-24 * rm) hw = std::max(hw, std::abs(q / 2 - k / 2));
+            if (std::fabs(Minv[(size_t)k * n2 + q]) > cut * rm) hw = std::max(hw, std::abs(q / 2 - k / 2));
     }
     const std::vector<double> *all[5] = {&lowr, &rbl, &gl, &V, &W};
     for (int k = 0; k < 5; k++) std::copy(all[k]->begin(), all[k]->end(), tabs + (size_t)k * nzp);
@@ -191,6 +191,61 @@ bool build_seg_tables(int N, int m, SegTables &t)
     const int W = 4 * hw + 4;
     t.band.assign((size_t)3 * n2 * W, 0.0);
     for (int slot = 0; slot < 3; slot++) band_rows(minv[slot], n2, hw, t.band.data() + (size_t)slot * n2 * W);
+    return true;
+}
+
+bool build_seg_rows(int N, int m, SegRows &t)
+{
+    const int P = (N + m - 1) / m;
+    const int nzp = P * m, n2 = 2 * P;
+    t.P = P;
+    t.m = m;
+    t.nzp = nzp;
+    t.hw = 0;
+    t.slots.assign((size_t)3 * 5 * nzp, 0.0);
+    std::vector<double> minv[3];
+    const int ibcs[3] = {1, 2, 3};
+    for (int slot = 0; slot < 3; slot++) {
+        std::vector<double> lo, up;
+        dbyd2_matrix(N, ibcs[slot], lo, up);
+        if (!seg_one(N, m, lo, up, t.slots.data() + (size_t)5 * slot * nzp, minv[slot], t.hw, 1e-19)) return false;
+    }
+    const int nw = 4 * t.hw + 4;
+    // the two rows of segment s: row 2s-1 around segment s-1, row 2s+2 around s+1
+    auto pair_rows = [&](int slot, int s) {
+        std::vector<double> r((size_t)2 * nw, 0.0);
+        for (int h = 0; h < 2; h++) {
+            const int k = h ? 2 * s + 2 : 2 * s - 1, c = h ? s + 1 : s - 1;
+            if (c < 0 || c >= P) continue;
+            for (int w = 0; w < nw; w++) {
+                const int q = 2 * (c - t.hw) + w;
+                if (q >= 0 && q < n2) r[(size_t)h * nw + w] = minv[slot][(size_t)k * n2 + q];
+            }
+        }
+        return r;
+    };
+    const int mid = P / 2;
+    t.E = 0;
+    for (int slot = 0; slot < 3; slot++) {
+        const std::vector<double> ref = pair_rows(slot, mid);
+        double big = 0.0;
+        for (double v : ref) big = std::max(big, std::fabs(v));
+        for (int s = 0; s < P; s++) {
+            const std::vector<double> r = pair_rows(slot, s);
+            double d = 0.0;
+            for (size_t q = 0; q < r.size(); q++) d = std::max(d, std::fabs(r[q] - ref[q]));
+            if (d > 1e-18 * big) t.E = std::max(t.E, std::min(s, P - 1 - s) + 1);
+        }
+    }
+    const int nk = seg_band_kinds(P, t.E);
+    if (nk == P) t.E = P;                                     // too short a column to repeat: every segment its own
+    t.rows.clear();
+    for (int slot = 0; slot < 3; slot++)
+        for (int k = 0; k < nk; k++) {
+            const int s = t.E == P || k < t.E ? k : (k == t.E ? mid : P - (2 * t.E + 1 - k));
+            const std::vector<double> r = pair_rows(slot, s);
+            t.rows.insert(t.rows.end(), r.begin(), r.end());
+        }
     return true;
 }
 
@@ -251,6 +306,13 @@ void dbyd2_edge_rows(int N2, int ibc, double eb[20])
         eb[10 + 4 - k] = -b;
         eb[15 + 4 - k] = ibc == 1 || ibc == 2 ? -far : 0.0;
     }
+}
+
+bool seg_kind_tables(const SegRows &t, std::vector<double> &out)
+{
+    out.clear();
+    out.reserve((size_t)15 * 3 * t.m);
+    return kind_rows(t.slots.data(), 15, t.P, t.m, out);
 }
 
 bool seg_kind_tables(const SegTables &t, std::vector<double> &out)

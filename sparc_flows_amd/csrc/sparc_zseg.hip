@@ -32,15 +32,6 @@ __device__ __forceinline__ void stg(double *base, unsigned ob, double v)
     *(SPARC_GLOBAL double *)((SPARC_GLOBAL char *)base + ob) = v;
 }
 
-// A block's logical number: the hardware deals consecutive blocks to the eight
-// XCDs in turn; this gives each XCD one contiguous stretch, so that blocks that
-// share 128-byte lines meet in one L2.
-__device__ __forceinline__ unsigned xcd_block(unsigned id, unsigned n)
-{
-    const unsigned q = n >> 3, r = n & 7, x = id & 7;
-    return x * q + min(x, r) + (id >> 3);
-}
-
 // One lane's part of a column: segment s, rows a .. a + MS - 1 of column c.
 struct Lane {
     int c, s, a;
