@@ -80,37 +80,6 @@ __global__ __launch_bounds__(256) void k3_ddy(const double *__restrict__ in, dou
     }
 }
 
-// The y-derivative for any ny that is not a power of two: circ_deriv_row
-// along y on one column pair (x0, x0 + 1) per 64-lane block (nx even, so
-// every pair is 16-byte aligned); cdy holds the derivative's circulant
-// column twice over.  Grid: exactly nplanes * nx/2 blocks.
-template <int N2>
-__global__ __launch_bounds__(64) void k3_ddy_any(const double *__restrict__ in, double *__restrict__ out,
-                                                 int nx, int ny, const double *__restrict__ cdy, double stretch)
-{
-    __shared__ double2 z[64 * N2];
-    __shared__ double cc[128 * N2];
-    for (int q = threadIdx.x; q < 128 * N2; q += 64) cc[q] = q < 2 * ny ? cdy[q] : 0.0;
-    const int t = threadIdx.x, hx = nx >> 1;
-    const long pl = (long)blockIdx.x / hx;
-    const int x0 = 2 * (int)((long)blockIdx.x - pl * hx);
-    const size_t base = (size_t)pl * ny * nx + x0;
-    double re[N2], im[N2];
-#pragma unroll
-    for (int j2 = 0; j2 < N2; j2++) {
-        const int y = min(t + 64 * j2, ny - 1);
-        const double2 v = *(const double2 *)(in + base + (size_t)y * nx);
-        re[j2] = v.x;
-        im[j2] = v.y;
-    }
-    circ_deriv_row<N2>(re, im, t, z, cc, ny, stretch);
-#pragma unroll
-    for (int j2 = 0; j2 < N2; j2++) {
-        const int y = t + 64 * j2;
-        if (y < ny) *(double2 *)(out + base + (size_t)y * nx) = make_double2(re[j2], im[j2]);
-    }
-}
-
 // Forward elimination (dbyd2.f + mtridag.f:96-105) of NC columns of one lane
 // at once, rows 2..nz-3 in chunks of U whose loads are issued together: a
 // lane then has NC * U loads in flight instead of one per dependent step.
@@ -385,18 +354,7 @@ __global__ __launch_bounds__(256) void k3_kern_final(const double *__restrict__ 
 static hipError_t launch_ddy(const double *in, double *out, int nplanes, int nx, int ny, const double2 *tw,
                              const double *dmul, const double *cdy, double stretch, hipStream_t st)
 {
-    if (!nx_has_fft(ny)) {
-        if (ny < 16 || ny > 1024 || (nx & 1)) return hipErrorInvalidValue;
-        const dim3 grid((unsigned)((long)nplanes * (nx / 2)));
-        switch (any_nx_slots(ny)) {
-#define A(N2V)                                                                                           \
-        case N2V: hipLaunchKernelGGL((k3_ddy_any<N2V>), grid, dim3(64), 0, st, in, out, nx, ny, cdy, stretch); break;
-            SPARC_ANY_NX_SLOTS(A)
-#undef A
-        default: return hipErrorInvalidValue;
-        }
-        return hipGetLastError();
-    }
+    if (!nx_has_fft(ny)) return launch_ddy_any(in, out, nplanes, nx, ny, cdy, stretch, st);
 #define L(NYV)                                                                                     \
     {                                                                                              \
         constexpr int BLK = DdyBlock<NYV>::n, TEAMS = BLK / FftShape<NYV>::N1;                     \
@@ -455,7 +413,7 @@ struct sparc3d_handle {
     Tri tri[4]{};
     DevArena bg_mem, st_mem, src_mem;
     const double2 *twx = nullptr, *twy = nullptr;
-    const double *cdx = nullptr, *cdy = nullptr;      // circulant columns [2n] (an n that is not a power of two)
+    const double *cdx = nullptr, *cdy = nullptr;      // circulant columns (an n that is not a power of two)
     const double *dmx = nullptr, *dmy = nullptr, *d_stretch = nullptr, *d_rhoinv = nullptr, *d_rho0 = nullptr,
                  *d_g = nullptr, *d_srcdep = nullptr;
     double *c2rho0 = nullptr, *az = nullptr, *bz = nullptr, *fz = nullptr;   // fz: PML factor of the gradients below
@@ -679,8 +637,7 @@ static int setup3(sparc3d_handle *h)
     const double dimc = 1e6, dimrho = 1e-3, diml = kRsun3, dimc2 = std::pow(dimc, 2.0);
     // x, y spectral tables (initialize.f90:194-225): exp(-2 pi i k/n), i k
     // (zero at the Nyquist bin of an even n), and for an n that is not a
-    // power of two the derivative's circulant column c[m] = -sum_k dm[k]
-    // sin(2 pi (k m mod n)/n), twice over (circ_deriv_row)
+    // power of two the derivative's circulant columns
     auto tables = [&](int n, const double2 **tw, const double **dm, const double **cd) -> int {
         std::vector<double> t(2 * (size_t)n), m(n);
         for (int k = 0; k < n; k++) {
@@ -697,16 +654,7 @@ static int setup3(sparc3d_handle *h)
             const double e = kk < 0 ? 0.0 : (double)kk * norm * 2.0 * kPi3;
             m[k] = 2 * k <= n ? e : -e;
         }
-        std::vector<double> c(2 * (size_t)n, 0.0);
-        if (!nx_has_fft(n)) {
-            std::vector<long double> sn(n);
-            for (int q = 0; q < n; q++) sn[q] = std::sin(2.0L * (long double)kPi3 * q / n);
-            for (int j = 0; j < n; j++) {
-                long double acc = 0.0L;
-                for (int k = 0; k < n; k++) acc -= (long double)m[k] * sn[(int)(((long)k * j) % n)];
-                c[j] = c[j + n] = (double)acc;
-            }
-        }
+        const std::vector<double> c = circ_table(m);
         double *p = nullptr;
         HCHECK3(h, upload(h->bg_mem, &p, t, h->stream));
         *tw = (const double2 *)p;

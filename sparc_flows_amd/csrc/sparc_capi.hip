@@ -146,6 +146,30 @@ static int fail(sparc_handle *h, int code, const std::string &msg)
     return code;
 }
 
+std::vector<double> circ_table(const std::vector<double> &dm)
+{
+    const int n = (int)dm.size();
+    if (nx_has_fft(n)) return {0.0};
+    const CircShape cs = circ_shape(n);
+    std::vector<long double> sn(n), c(n);
+    for (int q = 0; q < n; q++) sn[q] = std::sin(2.0L * 3.14159265358979323846264338327950288L * q / n);
+    for (int m = 0; m < n; m++) {
+        long double acc = 0.0L;
+        for (int k = 0; k < n; k++) acc -= (long double)dm[k] * sn[(int)(((long)k * m) % n)];
+        c[m] = acc;
+    }
+    std::vector<double> t((size_t)cs.nk * cs.plen, 0.0);
+    for (int m = 0; m < cs.len; m++) {
+        if (cs.nk == 1) {
+            t[m] = (double)c[m];
+        } else {
+            t[m] = (double)(0.5L * (c[m] + c[m + cs.len]));
+            t[cs.plen + m] = (double)(0.5L * (c[m] - c[m + cs.len]));
+        }
+    }
+    return t;
+}
+
 // ---------------------------------------------------------------------------
 // dbyd2 coefficients and matrix (dbyd2.f:85-195), float32 scalars widened.
 DbyCoef make_coef(int N2)
@@ -268,10 +292,7 @@ static std::vector<double> dmul_table(const sparc_handle *h)
 
 // The x-derivative's tables: twiddles exp(-2 pi i k / nx) (from the exact
 // octant values where they exist) for the FFT form, and for any other nx the
-// map's first column c[m] = sum_k i dmul[k] exp(2 pi i k m / nx)
-// = -sum_k dmul[k] sin(2 pi (k m mod nx) / nx) (real: dmul is odd in k; the
-// inverse transform's 1/nx is inside eyekx, as in ddx), stored twice over
-// (circ_deriv_row indexes [0, 2 nx) without a wrap).
+// circulant columns.
 static int upload_x_tables(sparc_handle *h)
 {
     const int nx = h->nx;
@@ -285,16 +306,7 @@ static int upload_x_tables(sparc_handle *h)
         tw[2 * k + 1] = s;
     }
     const std::vector<double> dm = dmul_table(h);
-    std::vector<double> cc(2 * (size_t)nx, 0.0);
-    if (!nx_has_fft(nx)) {
-        std::vector<long double> sn(nx);
-        for (int q = 0; q < nx; q++) sn[q] = std::sin(2.0L * (long double)kPi * q / nx);
-        for (int m = 0; m < nx; m++) {
-            long double acc = 0.0L;
-            for (int k = 0; k < nx; k++) acc -= (long double)dm[k] * sn[(int)(((long)k * m) % nx)];
-            cc[m] = cc[m + nx] = (double)acc;
-        }
-    }
+    const std::vector<double> cc = circ_table(dm);
     double *p = nullptr;
     HCHECK(h, upload(h->bg_mem, &p, tw, h->stream));
     h->bg.tw = (const double2 *)p;

@@ -32,6 +32,12 @@ sparc::DbyCoef make_coef(int N2);
 // mtridag.f:96-100): lowr, gam = uppr(j-1)/betad(j-1), 1/betad.
 void make_tri(int N2, int ibc, std::vector<double> &lowr, std::vector<double> &gam,
               std::vector<double> &rbet);
+// Circulant columns (sparc_circ.h) of the derivative of a line whose bin multipliers
+// are dm: the map's first column c[m] = sum_k i dm[k] exp(2 pi i k m / n)
+// = -sum_k dm[k] sin(2 pi (k m mod n) / n) (real: dm is odd in k; the inverse
+// transform's 1/n is inside dm), folded for an even n.  One unused element where n has
+// the FFT form.
+std::vector<double> circ_table(const std::vector<double> &dm);
 // Upload a host vector into a new device buffer of the arena.
 hipError_t upload(DevArena &ar, double **dst, const std::vector<double> &v, hipStream_t st);
 // The z kernels' tables of nz rows (sparc_zseg.h): nset sets, kZSegSets or

@@ -75,7 +75,7 @@ __global__ __launch_bounds__(64) void k_ddz_cols(const double *in, double *out,
 #define SPARC_FFT_DERIV(RE, IM, T, LDS, TW, DM, SX)                                            \
     do {                                                                                       \
         if constexpr (kAny)                                                                    \
-            circ_deriv_row<N2>(RE, IM, T, LDS, sdm, nxr, SX);                                  \
+            circ_deriv_block<N2>(RE, IM, T, LDS, sdm, nxr, SX);                                 \
         else if constexpr (N1 == 32 && N2 == 8)                                                \
             fft_deriv_team_256x32(RE, IM, T, LDS, (LDS) + 8 * 33, TW, DM, SX);                 \
         else if constexpr (N1 == 64 && N2 == 4)                                                \
@@ -84,43 +84,171 @@ __global__ __launch_bounds__(64) void k_ddz_cols(const double *in, double *out,
             fft_deriv_team<N1, N2>(RE, IM, T, LDS, TW, DM, SX);                                \
     } while (0)
 
-// Generic x-derivative (ddx) of nrows real rows of length nx; two rows per
-// FFT team.  NX = nx for a power of two; NX = -N2 for the any-nx form (64
-// lanes, rows up to 64 N2, circ_deriv_row).
-template <int NX, int N1 = (NX < 0 ? 64 : FftShape<(NX < 0 ? 16 : NX)>::N1)>
+// Generic x-derivative (ddx) of nrows real rows of length NX; two rows per
+// FFT team.
+template <int NX>
 __global__ __launch_bounds__(64) void k_ddx_rows(const double *__restrict__ in,
                                                  double *__restrict__ out, int nrows,
                                                  const double2 *__restrict__ tw,
-                                                 const double *__restrict__ dmul, double stretchx,
-                                                 const double *__restrict__ cdx, int nx)
+                                                 const double *__restrict__ dmul, double stretchx)
 {
-    constexpr bool kAny = NX < 0;
-    constexpr int N2 = kAny ? -NX : NX / N1, TEAMS = 64 / N1;
-    const int nxr = kAny ? nx : NX;
+    constexpr int N1 = FftShape<NX>::N1, N2 = FftShape<NX>::N2, TEAMS = 64 / N1;
     __shared__ double2 lds[TEAMS][FftLds<N1, N2>::n];
-    __shared__ double sdm[kAny ? 128 * N2 : 1];
-    if constexpr (kAny) {
-        // visible after circ_deriv_row's first barrier
-        for (int q = threadIdx.x; q < 128 * N2; q += 64) sdm[q] = q < 2 * nxr ? cdx[q] : 0.0;
-    }
     const int team = threadIdx.x / N1, t = threadIdx.x % N1;
     const int r0 = 2 * (blockIdx.x * TEAMS + team), r1 = r0 + 1;
     double re[N2], im[N2];
 #pragma unroll
     for (int j2 = 0; j2 < N2; j2++) {
         const int x = t + N1 * j2;
-        const bool in_row = !kAny || x < nxr;
-        re[j2] = r0 < nrows && in_row ? in[(size_t)r0 * nxr + x] : 0.0;
-        im[j2] = r1 < nrows && in_row ? in[(size_t)r1 * nxr + x] : 0.0;
+        re[j2] = r0 < nrows ? in[(size_t)r0 * NX + x] : 0.0;
+        im[j2] = r1 < nrows ? in[(size_t)r1 * NX + x] : 0.0;
     }
-    SPARC_FFT_DERIV(re, im, t, lds[team], tw, dmul, stretchx);
+    fft_deriv_team<N1, N2>(re, im, t, lds[team], tw, dmul, stretchx);
 #pragma unroll
     for (int j2 = 0; j2 < N2; j2++) {
         const int x = t + N1 * j2;
-        if (kAny && x >= nxr) continue;
-        if (r0 < nrows) out[(size_t)r0 * nxr + x] = re[j2];
-        if (r1 < nrows) out[(size_t)r1 * nxr + x] = im[j2];
+        if (r0 < nrows) out[(size_t)r0 * NX + x] = re[j2];
+        if (r1 < nrows) out[(size_t)r1 * NX + x] = im[j2];
     }
+}
+
+// Derivative of many lines whose length is not a power of two (sparc_circ.h),
+// two lines per team of s.lanes lanes, G teams per block.
+//   AXIS 0: count rows of length n, contiguous; a team takes rows 2 g, 2 g + 1.
+//   AXIS 1: count column pairs (x0, x0 + 1) of [n][nx] planes, nx even, so
+//           every pair is 16-byte aligned.
+// Both directions of global access run with the fastest index over the lanes;
+// the doubled lines and then the results wait in LDS.
+template <int AXIS>
+__global__ __launch_bounds__(256) void k_circ(const double *__restrict__ in, double *__restrict__ out, long count,
+                                              int nx, CircShape s, int G, const double *__restrict__ cd,
+                                              double stretch)
+{
+    extern __shared__ double2 circ_lds[];
+    constexpr int U = 4;                     // elements per lane whose loads are issued together
+    const int t = threadIdx.x;
+    double2 *const E = circ_lds;             // [G][nk][ext]
+    double *const cc = (double *)(E + (size_t)G * s.nk * s.ext);
+    const int per = s.nk * s.ext;
+    const long b0 = (long)xcd_block(blockIdx.x, gridDim.x) * G;     // first pair of the block
+    for (int q = t; q < s.nk * s.plen; q += 256) cc[q] = cd[q];
+    for (int q = t; q < G * s.nk * kCircK; q += 256) {
+        const int e = q / kCircK;
+        E[e * s.ext + q - e * kCircK] = make_double2(0.0, 0.0);
+    }
+    // element e of the block: (line, j) with j fastest (AXIS 0), (j, pair) with the
+    // pair fastest (AXIS 1); advanced by 256 without a division
+    const int fast = AXIS == 0 ? s.len : G, slow = AXIS == 0 ? 2 * G : s.len;
+    const int df = 256 % fast, ds = 256 / fast;
+    auto each = [&](auto &&body) {
+        int f = t % fast, o = t / fast;
+        while (o < slow) {
+            int fs[U], os[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                fs[u] = f;
+                os[u] = o;
+                f += df;
+                o += ds;
+                if (f >= fast) {
+                    f -= fast;
+                    o++;
+                }
+            }
+            body(fs, os);
+        }
+    };
+    // address of element j of line (or pair) i of the block; lines past the end: none
+    auto present = [&](int i) { return AXIS == 0 ? 2 * b0 + i < count : b0 + i < count; };
+    auto base = [&](int i) -> size_t {
+        if (AXIS == 0) return (size_t)(2 * b0 + i) * s.n;
+        const long pair = b0 + i, hx = nx >> 1, pl = pair / hx;
+        return (size_t)pl * s.n * nx + 2 * (size_t)(pair - pl * hx);
+    };
+    const size_t half = AXIS == 0 ? (size_t)s.len : (size_t)s.len * nx;
+    if constexpr (AXIS == 0) {
+        each([&](const int (&fs)[U], const int (&os)[U]) {
+            double a[U], b[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const bool ok = os[u] < slow && present(os[u]);
+                const size_t q = ok ? base(os[u]) + fs[u] : 0;
+                a[u] = ok ? in[q] : 0.0;
+                b[u] = ok && s.nk == 2 ? in[q + half] : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (os[u] >= slow) continue;
+                // line 2 g + c: component c of team g's elements
+                double *e = (double *)(E + (os[u] >> 1) * per) + (os[u] & 1);
+                const double v = s.nk == 2 ? a[u] + b[u] : a[u];
+                e[2 * (kCircK + s.len + fs[u])] = v;
+                e[2 * (kCircK + fs[u])] = v;
+                if (s.nk == 2) {
+                    const double w = a[u] - b[u];
+                    e += 2 * s.ext;
+                    e[2 * (kCircK + s.len + fs[u])] = w;
+                    e[2 * (kCircK + fs[u])] = -w;
+                }
+            }
+        });
+    } else {
+        each([&](const int (&fs)[U], const int (&os)[U]) {
+            double2 a[U], b[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const bool ok = os[u] < slow && present(fs[u]);
+                const size_t q = ok ? base(fs[u]) + (size_t)os[u] * nx : 0;
+                a[u] = ok ? *(const double2 *)(in + q) : make_double2(0.0, 0.0);
+                b[u] = ok && s.nk == 2 ? *(const double2 *)(in + q + half) : make_double2(0.0, 0.0);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (os[u] >= slow) continue;
+                double2 *const e = E + fs[u] * per;
+                if (s.nk == 2) {
+                    circ_put(e, s.len, 0, os[u], make_double2(a[u].x + b[u].x, a[u].y + b[u].y));
+                    circ_put(e + s.ext, s.len, 1, os[u], make_double2(a[u].x - b[u].x, a[u].y - b[u].y));
+                } else {
+                    circ_put(e, s.len, 0, os[u], a[u]);
+                }
+            }
+        });
+    }
+    __syncthreads();
+    const int g = t / s.lanes, l = t - g * s.lanes, kind = l >= s.L ? 1 : 0, x0 = kCircR * (l - kind * s.L);
+    double ar[kCircR], ai[kCircR];
+#pragma unroll
+    for (int r = 0; r < kCircR; r++) ar[r] = ai[r] = 0.0;
+    if (g < G)
+        circ_sum(ar, ai, E + g * per + kind * s.ext + kCircK + s.len + x0, cc + kind * s.plen, 0, s.plen);
+    __syncthreads();
+    if (g < G) {
+#pragma unroll
+        for (int r = 0; r < kCircR; r++)
+            if (x0 + r < s.len) E[g * per + kind * s.ext + x0 + r] = make_double2(ar[r] * stretch, ai[r] * stretch);
+    }
+    __syncthreads();
+    each([&](const int (&fs)[U], const int (&os)[U]) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = AXIS == 0 ? os[u] : fs[u], j = AXIS == 0 ? fs[u] : os[u];
+            if (os[u] >= slow || !present(i)) continue;
+            if constexpr (AXIS == 0) {
+                const double *e = (const double *)(E + (i >> 1) * per) + (i & 1);
+                const size_t q = base(i) + j;
+                const double p = e[2 * j], m = s.nk == 2 ? e[2 * (s.ext + j)] : 0.0;
+                out[q] = p + m;
+                if (s.nk == 2) out[q + half] = p - m;
+            } else {
+                const double2 *const e = E + i * per;
+                const size_t q = base(i) + (size_t)j * nx;
+                const double2 p = e[j], m = s.nk == 2 ? e[s.ext + j] : make_double2(0.0, 0.0);
+                *(double2 *)(out + q) = make_double2(p.x + m.x, p.y + m.y);
+                if (s.nk == 2) *(double2 *)(out + q + half) = make_double2(p.x - m.x, p.y - m.y);
+            }
+        }
+    });
 }
 
 // ---------------------------------------------------------------------------
@@ -134,23 +262,24 @@ __global__ __launch_bounds__(64) void k_ddx_rows(const double *__restrict__ in,
 // four radix-4 stages), which are faster when the pass is latency-bound (one
 // source) and slower when it is bandwidth-bound.
 //
-// NX = -N2: the any-nx form, one row per block of 64 lanes, rows up to
-// 64 N2 (circ_deriv_row); lane slots past nx load column nx-1 and store
+// NX = -N2: the any-nx form, one row per block of 256 lanes, rows up to
+// 256 N2 (circ_deriv_block); lane slots past nx load column nx-1 and store
 // nothing.
-template <int NX, int MODE, int N1 = (NX < 0 ? 64 : FftShape<(NX < 0 ? 16 : NX)>::N1)>
-__global__ __launch_bounds__(64, NX == 256 && N1 == 16 ? 2 : 1) void k_row(Dims d, Bg bg, State st, RowArgs ra, Clock clk, Sink sink)
+template <int NX, int MODE, int N1 = (NX < 0 ? 256 : FftShape<(NX < 0 ? 16 : NX)>::N1)>
+__global__ __launch_bounds__(NX < 0 ? 256 : 64, NX == 256 && N1 == 16 ? 2 : 1) void k_row(Dims d, Bg bg, State st, RowArgs ra, Clock clk, Sink sink)
 {
     constexpr bool kAny = NX < 0;
-    static_assert(!kAny || N1 == 64, "the any-nx form runs one row on 64 lanes");
-    constexpr int N2 = kAny ? -NX : NX / N1, TEAMS = 64 / N1;
+    static_assert(!kAny || N1 == 256, "the any-nx form runs one row on 256 lanes");
+    constexpr int N2 = kAny ? -NX : NX / N1, TEAMS = kAny ? 1 : 64 / N1;
     const int nxr = kAny ? d.nx : NX;
     __shared__ double2 lds[TEAMS][FftLds<N1, N2>::n];
     // twiddles and bin multipliers (any nx: the circulant column) staged in
     // LDS: their reads then never wait behind this pass's global stores
     __shared__ double2 stw[kAny ? 1 : NX];
-    __shared__ double sdm[kAny ? 128 * N2 : NX];
+    __shared__ double sdm[kAny ? CircLds<kAny ? N2 : 1>::c : NX];
     if constexpr (kAny) {
-        for (int q = threadIdx.x; q < 128 * N2; q += 64) sdm[q] = q < 2 * nxr ? bg.cdx[q] : 0.0;
+        const CircShape s = circ_shape(nxr);
+        for (int q = threadIdx.x; q < s.nk * s.plen; q += 256) sdm[q] = bg.cdx[q];
     } else {
         constexpr int NQ = (NX + 63) / 64;
         double2 tv[NQ];
@@ -603,18 +732,9 @@ hipError_t launch_ddx_rows(const double *in, double *out, int nrows, int nx, con
     const int npairs = (nrows + 1) / 2;
     if (!nx_has_fft(nx)) {
         if (nx < 16 || nx > 1024) return hipErrorInvalidValue;
-        // any nx: one row pair per 64-lane block
-        dim3 grid(npairs);
-        switch (any_nx_slots(nx)) {
-#define A(N2V)                                                                                   \
-        case N2V:                                                                                \
-            hipLaunchKernelGGL((k_ddx_rows<-N2V>), grid, dim3(64), 0, st, in, out, nrows, tw, dmul, \
-                               stretchx, cdx, nx);                                              \
-            break;
-            SPARC_ANY_NX_SLOTS(A)
-#undef A
-        default: return hipErrorInvalidValue;
-        }
+        const CircBatch c = circ_batch(nx, 0);
+        hipLaunchKernelGGL((k_circ<0>), dim3((npairs + c.G - 1) / c.G), dim3(256), c.lds, st, in, out, (long)nrows, nx,
+                           c.s, c.G, cdx, stretchx);
         return hipGetLastError();
     }
 #define L(NXV)                                                                              \
@@ -622,10 +742,21 @@ hipError_t launch_ddx_rows(const double *in, double *out, int nrows, int nx, con
         constexpr int TEAMS = 64 / FftShape<NXV>::N1;                                      \
         dim3 grid((npairs + TEAMS - 1) / TEAMS);                                            \
         hipLaunchKernelGGL(k_ddx_rows<NXV>, grid, dim3(64), 0, st, in, out, nrows, tw, dmul, \
-                           stretchx, cdx, nx);                                              \
+                           stretchx);                                                       \
     }
     SPARC_DISPATCH_NX(nx, L)
 #undef L
+    return hipGetLastError();
+}
+
+hipError_t launch_ddy_any(const double *in, double *out, int nplanes, int nx, int ny, const double *cdy,
+                          double stretch, hipStream_t st)
+{
+    if (ny < 16 || ny > 1024 || (nx & 1)) return hipErrorInvalidValue;
+    const CircBatch c = circ_batch(ny, 1);
+    const long pairs = (long)nplanes * (nx / 2);
+    hipLaunchKernelGGL((k_circ<1>), dim3((unsigned)((pairs + c.G - 1) / c.G)), dim3(256), c.lds, st, in, out, pairs, nx,
+                       c.s, c.G, cdy, stretch);
     return hipGetLastError();
 }
 
@@ -648,16 +779,16 @@ hipError_t launch_row(int mode, const Dims &d, const Bg &bg, const State &s, con
     }
     if (!nx_has_fft(d.nx)) {
         if (d.nx < 16 || d.nx > 1024) return hipErrorInvalidValue;
-        // any nx: one row per 64-lane block
+        // any nx: one row per 256-lane block
         dim3 grid(d.S * d.nz);
 #define A(N2V)                                                                                   \
         case N2V:                                                                                \
-            if (mode == 0) hipLaunchKernelGGL((k_row<-N2V, 0, 64>), grid, dim3(64), 0, st, d, bg, s, ra, c, sk); \
-            else if (mode == 1) hipLaunchKernelGGL((k_row<-N2V, 1, 64>), grid, dim3(64), 0, st, d, bg, s, ra, c, sk); \
-            else hipLaunchKernelGGL((k_row<-N2V, 2, 64>), grid, dim3(64), 0, st, d, bg, s, ra, c, sk); \
+            if (mode == 0) hipLaunchKernelGGL((k_row<-N2V, 0, 256>), grid, dim3(256), 0, st, d, bg, s, ra, c, sk); \
+            else if (mode == 1) hipLaunchKernelGGL((k_row<-N2V, 1, 256>), grid, dim3(256), 0, st, d, bg, s, ra, c, sk); \
+            else hipLaunchKernelGGL((k_row<-N2V, 2, 256>), grid, dim3(256), 0, st, d, bg, s, ra, c, sk); \
             break;
-        switch (any_nx_slots(d.nx)) {
-            SPARC_ANY_NX_SLOTS(A)
+        switch ((d.nx + 255) / 256) {
+            A(1) A(2) A(3) A(4)
         default: return hipErrorInvalidValue;
         }
 #undef A

@@ -12,6 +12,10 @@ hipError_t launch_ddz_cols(const double *in, double *out, int ncols, int nz, int
 // the circulant product (cdx, Bg::cdx's layout) for any other nx in [16, 1024].
 hipError_t launch_ddx_rows(const double *in, double *out, int nrows, int nx, const double2 *tw,
                            const double *dmul, const double *cdx, double stretchx, hipStream_t st);
+// y-derivative of nplanes [ny][nx] planes for an ny in [16, 1024] that is not a power
+// of two (nx even).
+hipError_t launch_ddy_any(const double *in, double *out, int nplanes, int nx, int ny, const double *cdy,
+                          double stretch, hipStream_t st);
 // Row pass; at nx = 256 wide = 1 runs 32 lanes per row (two rows per wave),
 // wide = 2 runs 64 lanes per row (one row per wave).
 hipError_t launch_row(int mode, const Dims &d, const Bg &bg, const State &s, const RowArgs &ra,
