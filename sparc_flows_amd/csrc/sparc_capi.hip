@@ -1771,7 +1771,7 @@ int sparc_discrete_gradient(sparc_handle *h, int maxtime, const double *gvz_dev,
     c.steps = h->steps;
     c.orow = h->o_rad;
     auto done = [&](int r) { (void)hipStreamSynchronize(h->stream); ar.release(); return r; };
-    int r = discrete_matrices(h, ar, c, 2 * h->S);
+    int r = discrete_matrices(h, ar, c, 3 * h->S);
     if (r) return done(r);
     DiscreteWork w{};
     const size_t S = h->S;
@@ -1781,10 +1781,9 @@ int sparc_discrete_gradient(sparc_handle *h, int maxtime, const double *gvz_dev,
     w.NST = 4 * w.SN + 2 * w.PZ1 + 2 * w.PX1;
     const int nseg = (maxtime + C) / C;
     struct B { double **p; size_t n; } bufs[] = {
-        {&w.U, w.NST}, {&w.Unext, w.NST}, {&w.Y, w.NST}, {&w.R, w.NST}, {&w.acc, w.NST}, {&w.Rb, w.NST},
-        {&w.Yb, w.NST}, {&w.lam, w.NST}, {&w.ck, (size_t)nseg * w.NST}, {&w.seg, (size_t)C * w.NST},
+        {&w.U, w.NST}, {&w.Unext, w.NST}, {&w.Y, w.NST}, {&w.acc, w.NST}, {&w.Rb, w.NST}, {&w.lam, w.NST}, {&w.ck, (size_t)nseg * w.NST}, {&w.seg, (size_t)C * w.NST},
         {&w.Dst, 25 * w.SN}, {&w.Dscr, 5 * w.SN}, {&w.T0, w.SN}, {&w.T1, w.SN}, {&w.T2, w.SN}, {&w.T3, w.SN},
-        {&w.GZ, w.SN}, {&w.DGZ, w.SN}, {&w.RHOB, w.SN}, {&w.XZP, w.SN}, {&w.DXB, w.SN}, {&w.DZB, w.SN},
+        {&w.GZ, w.SN}, {&w.DGZ, w.SN}, {&w.XZP, w.SN}, {&w.DXB, w.SN}, {&w.DZB, w.SN},
         {&w.DZ3B, w.SN}, {&w.DDXB, w.SN}, {&w.FX, 3 * w.SN}, {&w.DFX, 3 * w.SN}, {&w.FZ, 2 * w.SN},
         {&w.DFZ, 2 * w.SN}, {&w.PB, S * h->nx}};
     for (const B &b : bufs) {

@@ -22,7 +22,15 @@
 //     forward stage (k_fwd_b, k_fwd_c) and of its transpose (k_adj_a,
 //     k_adj_b, k_adj_c), the z filter and its transpose.
 // The forward stages here are unfused and recomputed from the trajectory; they
-// agree with the fused solver to rounding.
+// agree with the fused solver to rounding.  Bound: HBM and the launches (7 to 16 us
+// each).  A forward stage is six launches and a transposed one seven: the pointwise
+// kernels write the next stage's input or the accumulated adjoint themselves, and
+// derivatives of different fields share a launch.  With a pass of its own for every
+// update and accumulation a step of 8 sources at 256 x 300 took 415 us forward and
+// 620 transposed; here 310 and 500.
+#include <algorithm>
+#include <utility>
+
 #include "sparc_device.h"
 #include "sparc_launch.h"
 
@@ -86,23 +94,32 @@ __global__ void k_colsum_w(const double *__restrict__ in, const double *__restri
     out[q] = s;
 }
 
-// Geometry of a point q of an [S][nz][nx] field: source, row, column, its
-// z-PML row (-1 outside the layers) and x-PML column (-1 outside).
+// Geometry of point r of one source's [nz][nx] field: row, column, its z-PML
+// row (-1 outside the layers) and x-PML column (-1 outside).
 struct Pt {
     int b, k, i, pj, ci;
 };
-__device__ __forceinline__ Pt point(size_t q, const Dims &d)
+__device__ __forceinline__ Pt point(int b, unsigned r, const Dims &d)
 {
     Pt p;
-    const size_t n2 = (size_t)d.nz * d.nx;
-    p.b = (int)(q / n2);
-    const int r = (int)(q - (size_t)p.b * n2);
-    p.k = r / d.nx;
-    p.i = r - p.k * d.nx;
+    p.b = b;
+    p.k = (int)(r / (unsigned)d.nx);
+    p.i = (int)r - p.k * d.nx;
     p.pj = p.k < d.npmlbot ? p.k : (p.k >= d.nz - d.npmltop ? d.npmlbot + (p.k - (d.nz - d.npmltop)) : -1);
     p.ci = p.i < d.nh ? p.i : (p.i >= d.nx - d.nh ? d.nh + (p.i - (d.nx - d.nh)) : -1);
     return p;
 }
+// The pointwise kernels' grid: blocks of 256 points of a source in x, sources in y
+// (each point costs one 32-bit division; with flat 64-bit indices over all sources the
+// divisions bound the filters, 45 us a launch at 8 x 256 x 300).
+inline dim3 grid2(const Dims &d)
+{
+    return dim3((unsigned)((d.nz * d.nx + 255) / 256), (unsigned)(d.S < 65535 ? d.S : 65535));
+}
+#define FOR_POINTS(d, r, b)                                                                        \
+    const unsigned r = blockIdx.x * 256u + threadIdx.x, n2_ = (unsigned)d.nz * (unsigned)d.nx;     \
+    if (r >= n2_) return;                                                                          \
+    for (int b = blockIdx.y; b < d.S; b += gridDim.y)
 
 // Full-state views: a [4][S][nz][nx], pz [2][S][nzpml][nx], px [2][S][nz][nph].
 struct Views {
@@ -113,236 +130,273 @@ __device__ __forceinline__ size_t pxi(const Dims &d, const Pt &p) { return ((siz
 
 // Forward stage, first pointwise part (physics2d.f90:957-998, :1043): z-PML of
 // dxi_z/dz, x-PML of dxi_x/dx, div, p, rho'.  dzxi includes the kept last
-// row (:954).  Writes DIV, P, RHO and the RHS of psivz, psivx.
-__global__ void k_fwd_b(Dims d, Bg bg, Views v, const double *__restrict__ Y, const double *__restrict__ dxxi,
-                        const double *__restrict__ dzxi, double *__restrict__ DIV, double *__restrict__ P,
-                        double *__restrict__ RHO, double *__restrict__ R)
+// row (:954).  Writes DIV, P, RHO and psivz, psivx of the next stage's
+// input Yn = U + beta * RHS (step.f90:60-62), where every element is read only at
+// its own point before: Yn may be Y.
+__global__ __launch_bounds__(256) void k_fwd_b(Dims d, Bg bg, Views v, const double *Y,
+                                               const double *__restrict__ dxxi, const double *__restrict__ dzxi,
+                                               double *__restrict__ DIV, double *__restrict__ P,
+                                               double *__restrict__ RHO, const double *U, double beta, double *Yn)
 {
-    const size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (q >= v.SN) return;
-    const Pt p = point(q, d);
-    const size_t r2 = (size_t)p.k * d.nx + p.i;
-    const double *ypz = Y + 4 * v.SN, *ypx = ypz + 2 * v.PZ1;
-    double *rpz = R + 4 * v.SN, *rpx = rpz + 2 * v.PZ1;
-    double dz = dzxi[q], dx = dxxi[q];
-    if (p.pj >= 0) {
-        const size_t e = pzi(d, p), c = (size_t)p.pj * d.nx + p.i;
-        const double psi = ypz[e];
-        rpz[e] = bg.az[c] * dz + bg.bz[c] * psi;
-        dz = dz + psi;
+    FOR_POINTS(d, r2, b)
+    {
+        const Pt p = point(b, r2, d);
+        const size_t q = (size_t)b * n2_ + r2, pz = 4 * v.SN, px = pz + 2 * v.PZ1;
+        double dz = dzxi[q], dx = dxxi[q];
+        if (p.pj >= 0) {
+            const size_t e = pz + pzi(d, p), c = (size_t)p.pj * d.nx + p.i;
+            const double psi = Y[e];
+            Yn[e] = U[e] + beta * (bg.az[c] * dz + bg.bz[c] * psi);
+            dz = dz + psi;
+        }
+        if (p.ci >= 0) {
+            const size_t e = px + pxi(d, p), c = (size_t)p.k * d.nph + p.ci;
+            const double psi = Y[e];
+            dx = dx + psi;
+            Yn[e] = U[e] + beta * (bg.ax[c] * dx + bg.bx[c] * psi);
+        }
+        const double div = dx + dz, xiz = Y[v.SN + q];
+        DIV[q] = div;
+        P[q] = -(bg.c2rho0[r2] * div) - bg.gp0[r2] * xiz;
+        RHO[q] = -(bg.rho0[r2] * div) - bg.gr0[r2] * xiz;
     }
-    if (p.ci >= 0) {
-        const size_t e = pxi(d, p), c = (size_t)p.k * d.nph + p.ci;
-        const double psi = ypx[e];
-        dx = dx + psi;
-        rpx[e] = bg.ax[c] * dx + bg.bx[c] * psi;
-    }
-    const double div = dx + dz, xiz = Y[v.SN + q];
-    DIV[q] = div;
-    P[q] = -(bg.c2rho0[r2] * div) - bg.gp0[r2] * xiz;
-    RHO[q] = -(bg.rho0[r2] * div) - bg.gr0[r2] * xiz;
 }
 
 // Forward stage, second pointwise part (physics2d.f90:1003-1092): PMLs of the
 // pressure gradient, RHS v_x, v_z, xi, the source of time t, the flow terms,
-// the zeroed rows and columns.  DV = [dvx/dx, dvz/dx, dvx/dz, dvz/dz].
-__global__ void k_fwd_c(Dims d, Bg bg, Views v, Src src, int t, const double *__restrict__ Y,
-                        const double *__restrict__ gpx_in, const double *__restrict__ gpz_in,
-                        const double *__restrict__ RHO, const double *__restrict__ DV, double *__restrict__ R)
+// the zeroed rows and columns, and the next stage's input Yn = U + beta * RHS.
+// DV = [dvx/dx, dvz/dx, dvx/dz, dvz/dz].  Yn may be Y, as in k_fwd_b.
+__global__ __launch_bounds__(256) void k_fwd_c(Dims d, Bg bg, Views v, Src src, int t, const double *Y,
+                                               const double *__restrict__ gpx_in, const double *__restrict__ gpz_in,
+                                               const double *__restrict__ RHO, const double *__restrict__ DV,
+                                               const double *U, double beta, double *Yn)
 {
-    const size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (q >= v.SN) return;
-    const Pt p = point(q, d);
-    const size_t r2 = (size_t)p.k * d.nx + p.i;
-    const double *ypz = Y + 4 * v.SN, *ypx = ypz + 2 * v.PZ1;
-    double *rpz = R + 4 * v.SN, *rpx = rpz + 2 * v.PZ1;
-    double gpx = gpx_in[q], gpz = gpz_in[q];
-    if (p.ci >= 0) {
-        const size_t e = v.PX1 + pxi(d, p), c = (size_t)p.k * d.nph + p.ci;
-        const double psi = ypx[e];
-        gpx = gpx + psi;
-        rpx[e] = bg.ax[c] * gpx + bg.bx[c] * psi;
-    }
-    if (p.pj >= 0) {
-        const size_t e = v.PZ1 + pzi(d, p), c = (size_t)p.pj * d.nx + p.i;
-        const double psi = ypz[e];
-        rpz[e] = bg.az[c] * gpz + bg.bz[c] * psi;
-        gpz = gpz + psi;
-    }
-    double rvx = -bg.rhoinv[r2] * gpx;
-    double rvz = -bg.rhoinv[r2] * (gpz + RHO[q] * bg.g[p.k]);
-    double rxx = Y[2 * v.SN + q], rxz = Y[3 * v.SN + q];
-    if (t <= src.limit) {                                   // :1051-1061
-        const double fs = (t >= 0 && t < src.nfwd) ? src.fwd[t] : 0.0;
-        if (src.mode == 1 && p.k == src.row)
-            rvz += src.vr[(size_t)p.b * d.nx + p.i] * fs * src.delta_width / bg.rho0_src[p.i];
-        else if (src.mode == 3)
-            rvz += src.vr[(size_t)p.b * d.nx + p.i] * fs * src.zprof[p.k];
-    }
-    rvx = rvx - 2.0 * bg.v0x[r2] * DV[q];                   // :1065-1079
-    rvx = rvx - 2.0 * bg.v0z[r2] * DV[2 * v.SN + q];
-    rvz = rvz - 2.0 * bg.v0x[r2] * DV[v.SN + q];
-    rvz = rvz - 2.0 * bg.v0z[r2] * DV[3 * v.SN + q];
-    const bool zero = p.k == 0 || p.i == 0 || p.i == d.nx - 1;  // :1083-1092
-    R[q] = zero ? 0.0 : rxx;
-    R[v.SN + q] = zero ? 0.0 : rxz;
-    R[2 * v.SN + q] = zero ? 0.0 : rvx;
-    R[3 * v.SN + q] = zero ? 0.0 : rvz;
-}
-
-// out = U + beta R over the whole state (n doubles); beta 0 copies.
-__global__ void k_axpy(const double *__restrict__ U, const double *__restrict__ R, double beta,
-                       double *__restrict__ out, size_t n)
-{
-    const size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (q < n) out[q] = U[q] + beta * R[q];
-}
-
-// acc += Yb, Rb = beta Yb
-__global__ void k_accum(double *__restrict__ acc, double *__restrict__ Rb, const double *__restrict__ Yb,
-                        double beta, size_t n)
-{
-    const size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    const double y = Yb[q];
-    acc[q] += y;
-    Rb[q] = beta * y;
-}
-
-// One of the filtered rows of FILTER_VARS_2D (physics2d.f90:509-556):
-// rows 5..nz-6 (0-based) take the 11-point filter, rows nz-5..nz-2 the
-// two-point mean, for columns nh-1 .. nx-nh.
-__device__ __constant__ double kFC[6] = {0.75390625, 0.41015625, -0.234375, 0.087890625, -0.01953125,
-                                         0.001953125};
-
-// a_new = filter(U + dt R) on the 4 fields, pz/px += dt R (the last stage's
-// update, step.f90:107-112); A = out state.
-__global__ void k_update_filter(Dims d, Views v, const double *__restrict__ U, const double *__restrict__ R,
-                                double dt, double *__restrict__ A)
-{
-    const size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    const size_t n4 = 4 * v.SN, nall = n4 + 2 * v.PZ1 + 2 * v.PX1;
-    if (q >= nall) return;
-    if (q >= n4) { A[q] = U[q] + dt * R[q]; return; }
-    const size_t f = q / v.SN, qq = q - f * v.SN;
-    const Pt p = point(qq, d);
-    const size_t base = f * v.SN + ((size_t)p.b * d.nz) * d.nx + p.i;
-    auto u = [&](int k) { const size_t e = base + (size_t)k * d.nx; return U[e] + dt * R[e]; };
-    double val = u(p.k);
-    if (p.i >= d.nh - 1 && p.i <= d.nx - d.nh && p.k >= 5 && p.k <= d.nz - 2) {
-        if (p.k <= d.nz - 6) {
-            val = kFC[0] * u(p.k);
-            for (int m = 1; m <= 5; m++) val += 0.5 * kFC[m] * (u(p.k - m) + u(p.k + m));
-        } else {
-            val = 0.5 * (u(p.k + 1) + u(p.k - 1));
+    FOR_POINTS(d, r2, b)
+    {
+        const Pt p = point(b, r2, d);
+        const size_t q = (size_t)b * n2_ + r2, pz = 4 * v.SN + v.PZ1, px = 4 * v.SN + 2 * v.PZ1 + v.PX1;
+        double gpx = gpx_in[q], gpz = gpz_in[q];
+        if (p.ci >= 0) {
+            const size_t e = px + pxi(d, p), c = (size_t)p.k * d.nph + p.ci;
+            const double psi = Y[e];
+            gpx = gpx + psi;
+            Yn[e] = U[e] + beta * (bg.ax[c] * gpx + bg.bx[c] * psi);
         }
+        if (p.pj >= 0) {
+            const size_t e = pz + pzi(d, p), c = (size_t)p.pj * d.nx + p.i;
+            const double psi = Y[e];
+            Yn[e] = U[e] + beta * (bg.az[c] * gpz + bg.bz[c] * psi);
+            gpz = gpz + psi;
+        }
+        double rvx = -bg.rhoinv[r2] * gpx;
+        double rvz = -bg.rhoinv[r2] * (gpz + RHO[q] * bg.g[p.k]);
+        const double rxx = Y[2 * v.SN + q], rxz = Y[3 * v.SN + q];
+        if (t <= src.limit) {                                   // :1051-1061
+            const double fs = (t >= 0 && t < src.nfwd) ? src.fwd[t] : 0.0;
+            if (src.mode == 1 && p.k == src.row)
+                rvz += src.vr[(size_t)b * d.nx + p.i] * fs * src.delta_width / bg.rho0_src[p.i];
+            else if (src.mode == 3)
+                rvz += src.vr[(size_t)b * d.nx + p.i] * fs * src.zprof[p.k];
+        }
+        rvx = rvx - 2.0 * bg.v0x[r2] * DV[q];                   // :1065-1079
+        rvx = rvx - 2.0 * bg.v0z[r2] * DV[2 * v.SN + q];
+        rvz = rvz - 2.0 * bg.v0x[r2] * DV[v.SN + q];
+        rvz = rvz - 2.0 * bg.v0z[r2] * DV[3 * v.SN + q];
+        const bool zero = p.k == 0 || p.i == 0 || p.i == d.nx - 1;  // :1083-1092
+        Yn[q] = U[q] + beta * (zero ? 0.0 : rxx);
+        Yn[v.SN + q] = U[v.SN + q] + beta * (zero ? 0.0 : rxz);
+        Yn[2 * v.SN + q] = U[2 * v.SN + q] + beta * (zero ? 0.0 : rvx);
+        Yn[3 * v.SN + q] = U[3 * v.SN + q] + beta * (zero ? 0.0 : rvz);
     }
-    A[q] = val;
 }
 
-// Transpose of the filter on the 4 fields (pz, px copied): out = F^T lam.
-__global__ void k_filter_T(Dims d, Views v, const double *__restrict__ lam, double *__restrict__ out)
+// FILTER_VARS_2D (physics2d.f90:509-556): rows 5..nz-6 (0-based) take the
+// 11-point filter, rows nz-5..nz-2 the two-point mean, for columns nh-1 .. nx-nh.
+// One lane filters kFR rows of a column of one field, from a window of kFR + 10 rows:
+// 2.25 loads a row in place of 11.  us per launch at 8 x 256 x 300, one lane a
+// point with 64-bit index arithmetic -> here: 45 -> 11, transposed 44 -> 15.
+constexpr int kFR = 8;
+__device__ __forceinline__ double kfc(int m)
 {
-    const size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    const size_t n4 = 4 * v.SN, nall = n4 + 2 * v.PZ1 + 2 * v.PX1;
-    if (q >= nall) return;
-    if (q >= n4) { out[q] = lam[q]; return; }
-    const size_t f = q / v.SN, qq = q - f * v.SN;
-    const Pt p = point(qq, d);
-    const size_t base = f * v.SN + ((size_t)p.b * d.nz) * d.nx + p.i;
-    const int j = p.k, nz = d.nz;
-    const bool xin = p.i >= d.nh - 1 && p.i <= d.nx - d.nh;
-    if (!xin) { out[q] = lam[q]; return; }
-    double val = (j >= 5 && j <= nz - 2) ? 0.0 : lam[q];    // rows the filter replaces
-    for (int k = max(5, j - 5); k <= min(nz - 6, j + 5); k++) {
-        const int m = abs(k - j);
-        val += (m == 0 ? kFC[0] : 0.5 * kFC[m]) * lam[base + (size_t)k * d.nx];
+    constexpr double c[6] = {0.75390625, 0.41015625, -0.234375, 0.087890625, -0.01953125, 0.001953125};
+    return c[m];
+}
+inline dim3 grid_filter(const Dims &d)
+{
+    return dim3((unsigned)(((d.nz + kFR - 1) / kFR * d.nx + 255) / 256), (unsigned)std::min(4 * (long)d.S, 65535L));
+}
+// The window of the lane's rows in each of the 4 S columns of fields, and the PML
+// variables behind them element by element: body(field base, first row, column,
+// window), tail(element).
+template <class Body, class Tail>
+__device__ __forceinline__ void filter_walk(const Dims &d, const Views &v, const double *__restrict__ in, Body &&body,
+                                            Tail &&tail)
+{
+    const size_t n4 = 4 * v.SN, nall = n4 + 2 * v.PZ1 + 2 * v.PX1, total = (size_t)gridDim.x * gridDim.y * 256;
+    for (size_t q = n4 + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x; q < nall; q += total) tail(q);
+    const unsigned id = blockIdx.x * 256u + threadIdx.x;
+    const int g = (int)(id / (unsigned)d.nx), x = (int)id - g * d.nx, j0 = g * kFR;
+    if (j0 >= d.nz) return;
+    for (int fb = blockIdx.y; fb < 4 * d.S; fb += gridDim.y) {
+        const size_t base = (size_t)fb * d.nz * d.nx + x;
+        double w[kFR + 10];
+#pragma unroll
+        for (int u = 0; u < kFR + 10; u++) w[u] = in[base + (size_t)min(max(j0 - 5 + u, 0), d.nz - 1) * d.nx];
+        body(base, j0, x, w);
     }
-    for (int k = max(nz - 5, j - 1); k <= min(nz - 2, j + 1); k++)
-        if (abs(k - j) == 1) val += 0.5 * lam[base + (size_t)k * d.nx];
-    out[q] = val;
+}
+
+// A = filter(Y) on the 4 fields of the last stage's update (step.f90:107-112),
+// the PML variables copied.
+__global__ __launch_bounds__(256) void k_filter(Dims d, Views v, const double *__restrict__ Y, double *__restrict__ A)
+{
+    filter_walk(d, v, Y,
+        [&](size_t base, int j0, int x, const double (&w)[kFR + 10]) {
+            const bool xin = x >= d.nh - 1 && x <= d.nx - d.nh;
+#pragma unroll
+            for (int i = 0; i < kFR; i++) {
+                const int k = j0 + i;
+                if (k >= d.nz) break;
+                double val = w[i + 5];
+                if (xin && k >= 5 && k <= d.nz - 2) {
+                    if (k <= d.nz - 6) {
+                        val = kfc(0) * val;
+#pragma unroll
+                        for (int m = 1; m <= 5; m++) val += 0.5 * kfc(m) * (w[i + 5 - m] + w[i + 5 + m]);
+                    } else {
+                        val = 0.5 * (w[i + 6] + w[i + 4]);
+                    }
+                }
+                A[base + (size_t)k * d.nx] = val;
+            }
+        },
+        [&](size_t q) { A[q] = Y[q]; });
+}
+
+// Transpose of the filter on the 4 fields (pz, px copied): acc = F^T lam, and
+// the last stage's RHS adjoint Rb = dt acc.
+__global__ __launch_bounds__(256) void k_filter_T(Dims d, Views v, const double *__restrict__ lam, double dt,
+                                                  double *__restrict__ acc, double *__restrict__ Rb)
+{
+    filter_walk(d, v, lam,
+        [&](size_t base, int j0, int x, const double (&w)[kFR + 10]) {
+            const int nz = d.nz;
+            const bool xin = x >= d.nh - 1 && x <= d.nx - d.nh;
+#pragma unroll
+            for (int i = 0; i < kFR; i++) {
+                const int j = j0 + i;
+                if (j >= nz) break;
+                double val = w[i + 5];
+                if (xin) {
+                    if (j >= 5 && j <= nz - 2) val = 0.0;          // rows the filter replaces
+#pragma unroll
+                    for (int m = -5; m <= 5; m++) {
+                        const int k = j + m;
+                        if (k >= 5 && k <= nz - 6) val += (m == 0 ? kfc(0) : 0.5 * kfc(m < 0 ? -m : m)) * w[i + 5 + m];
+                    }
+                    if (j - 1 >= nz - 5 && j - 1 <= nz - 2) val += 0.5 * w[i + 4];
+                    if (j + 1 >= nz - 5 && j + 1 <= nz - 2) val += 0.5 * w[i + 6];
+                }
+                acc[base + (size_t)j * d.nx] = val;
+                Rb[base + (size_t)j * d.nx] = dt * val;
+            }
+        },
+        [&](size_t q) {
+            const double val = lam[q];
+            acc[q] = val;
+            Rb[q] = dt * val;
+        });
+}
+
+// The adjoint y of one element of a stage's input: into the adjoint of the step's
+// start, and times beta the RHS adjoint of the stage before.
+__device__ __forceinline__ void accumulate(double *acc, double *Rb, size_t e, double y, double beta)
+{
+    acc[e] += y;
+    Rb[e] = beta * y;
 }
 
 // Transpose of k_fwd_c's RHS (and of the flow terms' inputs):
 // FX = [-2 v0x Rvx, -2 v0x Rvz, adjoint of dp/dx], FZ = [-2 v0z Rvx,
-// -2 v0z Rvz], GZ = adjoint of the raw dp/dz, RHOB = adjoint of rho';
-// writes the adjoints of psi_gradp_x and psip into Yb.
-__global__ void k_adj_a(Dims d, Bg bg, Views v, const double *__restrict__ Rb, double *__restrict__ FX,
-                        double *__restrict__ FZ, double *__restrict__ GZ, double *__restrict__ RHOB,
-                        double *__restrict__ Yb)
+// -2 v0z Rvz], GZ = adjoint of the raw dp/dz; accumulates the adjoints of
+// psi_gradp_x and psip.  The three adjoint kernels read and then replace Rb at
+// their own points only, each its own elements.
+__global__ __launch_bounds__(256) void k_adj_a(Dims d, Bg bg, Views v, double *__restrict__ Rb,
+                                               double *__restrict__ acc, double beta, double *__restrict__ FX,
+                                               double *__restrict__ FZ, double *__restrict__ GZ)
 {
-    const size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (q >= v.SN) return;
-    const Pt p = point(q, d);
-    const size_t r2 = (size_t)p.k * d.nx + p.i;
-    const bool zero = p.k == 0 || p.i == 0 || p.i == d.nx - 1;
-    const double rvx = zero ? 0.0 : Rb[2 * v.SN + q], rvz = zero ? 0.0 : Rb[3 * v.SN + q];
-    const double *rpz = Rb + 4 * v.SN, *rpx = rpz + 2 * v.PZ1;
-    double *ypz = Yb + 4 * v.SN, *ypx = ypz + 2 * v.PZ1;
-    FX[q] = -2.0 * bg.v0x[r2] * rvx;
-    FX[v.SN + q] = -2.0 * bg.v0x[r2] * rvz;
-    FZ[q] = -2.0 * bg.v0z[r2] * rvx;
-    FZ[v.SN + q] = -2.0 * bg.v0z[r2] * rvz;
-    double gpx = -bg.rhoinv[r2] * rvx;
-    if (p.ci >= 0) {
-        const size_t e = v.PX1 + pxi(d, p), c = (size_t)p.k * d.nph + p.ci;
-        const double tot = gpx + bg.ax[c] * rpx[e];
-        ypx[e] = tot + bg.bx[c] * rpx[e];
-        gpx = tot;
+    FOR_POINTS(d, r2, b)
+    {
+        const Pt p = point(b, r2, d);
+        const size_t q = (size_t)b * n2_ + r2;
+        const bool zero = p.k == 0 || p.i == 0 || p.i == d.nx - 1;
+        const double rvx = zero ? 0.0 : Rb[2 * v.SN + q], rvz = zero ? 0.0 : Rb[3 * v.SN + q];
+        FX[q] = -2.0 * bg.v0x[r2] * rvx;
+        FX[v.SN + q] = -2.0 * bg.v0x[r2] * rvz;
+        FZ[q] = -2.0 * bg.v0z[r2] * rvx;
+        FZ[v.SN + q] = -2.0 * bg.v0z[r2] * rvz;
+        double gpx = -bg.rhoinv[r2] * rvx;
+        if (p.ci >= 0) {
+            const size_t e = 4 * v.SN + 2 * v.PZ1 + v.PX1 + pxi(d, p), c = (size_t)p.k * d.nph + p.ci;
+            const double r = Rb[e], tot = gpx + bg.ax[c] * r;
+            accumulate(acc, Rb, e, tot + bg.bx[c] * r, beta);
+            gpx = tot;
+        }
+        FX[2 * v.SN + q] = gpx;
+        double gpz = -bg.rhoinv[r2] * rvz;
+        if (p.pj >= 0) {
+            const size_t e = 4 * v.SN + v.PZ1 + pzi(d, p), c = (size_t)p.pj * d.nx + p.i;
+            const double r = Rb[e];
+            accumulate(acc, Rb, e, gpz + bg.bz[c] * r, beta);
+            gpz = gpz + bg.az[c] * r;
+        }
+        GZ[q] = gpz;
     }
-    FX[2 * v.SN + q] = gpx;
-    double gpz = -bg.rhoinv[r2] * rvz;
-    RHOB[q] = -bg.rhoinv[r2] * bg.g[p.k] * rvz;
-    if (p.pj >= 0) {
-        const size_t e = v.PZ1 + pzi(d, p), c = (size_t)p.pj * d.nx + p.i;
-        ypz[e] = gpz + bg.bz[c] * rpz[e];
-        gpz = gpz + bg.az[c] * rpz[e];
-    }
-    GZ[q] = gpz;
 }
 
 // Second transposed part: v adjoints, p adjoint, div adjoint through both
 // PMLs of the displacement derivatives, the gradient contributions of this
 // stage: G = [d/d(c^2 rho0), d/dv0x, d/dv0z] += pairs with the stage's
 // forward quantities D = [div, dvx/dx, dvz/dx, dvx/dz, dvz/dz].
-__global__ void k_adj_b(Dims d, Bg bg, Views v, const double *__restrict__ Rb, const double *__restrict__ DFX,
-                        const double *__restrict__ DFZ, const double *__restrict__ DGZ,
-                        const double *__restrict__ RHOB, const double *__restrict__ D, double *__restrict__ Yb,
-                        double *__restrict__ XZP, double *__restrict__ DXB, double *__restrict__ DZB,
-                        double *__restrict__ G)
+__global__ __launch_bounds__(256) void k_adj_b(Dims d, Bg bg, Views v, double *__restrict__ Rb,
+                                               double *__restrict__ acc, double beta, const double *__restrict__ DFX,
+                                               const double *__restrict__ DFZ, const double *__restrict__ DGZ,
+                                               const double *__restrict__ D, double *__restrict__ XZP,
+                                               double *__restrict__ DXB, double *__restrict__ DZB,
+                                               double *__restrict__ G)
 {
-    const size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (q >= v.SN) return;
-    const Pt p = point(q, d);
-    const size_t r2 = (size_t)p.k * d.nx + p.i;
-    const bool zero = p.k == 0 || p.i == 0 || p.i == d.nx - 1;
-    const double rxx = zero ? 0.0 : Rb[q], rxz = zero ? 0.0 : Rb[v.SN + q];
-    const double rvx = zero ? 0.0 : Rb[2 * v.SN + q], rvz = zero ? 0.0 : Rb[3 * v.SN + q];
-    const double *rpz = Rb + 4 * v.SN, *rpx = rpz + 2 * v.PZ1;
-    double *ypz = Yb + 4 * v.SN, *ypx = ypz + 2 * v.PZ1;
-    Yb[2 * v.SN + q] = -DFX[q] + DFZ[q] + rxx;                 // dx^T = -dx
-    Yb[3 * v.SN + q] = -DFX[v.SN + q] + DFZ[v.SN + q] + rxz;
-    const double pb = -DFX[2 * v.SN + q] + DGZ[q];
-    const double rb = RHOB[q];
-    const double divb = -bg.rho0[r2] * rb - bg.c2rho0[r2] * pb;
-    XZP[q] = -bg.gr0[r2] * rb - bg.gp0[r2] * pb;
-    double dxb = divb, dzb = divb;
-    if (p.ci >= 0) {
-        const size_t e = pxi(d, p), c = (size_t)p.k * d.nph + p.ci;
-        const double tot = divb + bg.ax[c] * rpx[e];
-        ypx[e] = tot + bg.bx[c] * rpx[e];
-        dxb = tot;
+    FOR_POINTS(d, r2, b)
+    {
+        const Pt p = point(b, r2, d);
+        const size_t q = (size_t)b * n2_ + r2;
+        const bool zero = p.k == 0 || p.i == 0 || p.i == d.nx - 1;
+        const double rxx = zero ? 0.0 : Rb[q], rxz = zero ? 0.0 : Rb[v.SN + q];
+        const double rvx = zero ? 0.0 : Rb[2 * v.SN + q], rvz = zero ? 0.0 : Rb[3 * v.SN + q];
+        accumulate(acc, Rb, 2 * v.SN + q, -DFX[q] + DFZ[q] + rxx, beta);           // dx^T = -dx
+        accumulate(acc, Rb, 3 * v.SN + q, -DFX[v.SN + q] + DFZ[v.SN + q] + rxz, beta);
+        const double pb = -DFX[2 * v.SN + q] + DGZ[q];
+        const double rb = -bg.rhoinv[r2] * bg.g[p.k] * rvz;                        // adjoint of rho'
+        const double divb = -bg.rho0[r2] * rb - bg.c2rho0[r2] * pb;
+        XZP[q] = -bg.gr0[r2] * rb - bg.gp0[r2] * pb;
+        double dxb = divb, dzb = divb;
+        if (p.ci >= 0) {
+            const size_t e = 4 * v.SN + 2 * v.PZ1 + pxi(d, p), c = (size_t)p.k * d.nph + p.ci;
+            const double r = Rb[e], tot = divb + bg.ax[c] * r;
+            accumulate(acc, Rb, e, tot + bg.bx[c] * r, beta);
+            dxb = tot;
+        }
+        if (p.pj >= 0) {
+            const size_t e = 4 * v.SN + pzi(d, p), c = (size_t)p.pj * d.nx + p.i;
+            const double r = Rb[e];
+            accumulate(acc, Rb, e, divb + bg.bz[c] * r, beta);
+            dzb = divb + bg.az[c] * r;
+        }
+        DXB[q] = dxb;
+        DZB[q] = dzb;
+        G[q] += -pb * D[q];
+        G[v.SN + q] += -2.0 * (rvx * D[v.SN + q] + rvz * D[2 * v.SN + q]);
+        G[2 * v.SN + q] += -2.0 * (rvx * D[3 * v.SN + q] + rvz * D[4 * v.SN + q]);
     }
-    if (p.pj >= 0) {
-        const size_t e = pzi(d, p), c = (size_t)p.pj * d.nx + p.i;
-        ypz[e] = divb + bg.bz[c] * rpz[e];
-        dzb = divb + bg.az[c] * rpz[e];
-    }
-    DXB[q] = dxb;
-    DZB[q] = dzb;
-    G[q] += -pb * D[q];
-    G[v.SN + q] += -2.0 * (rvx * D[v.SN + q] + rvz * D[2 * v.SN + q]);
-    G[2 * v.SN + q] += -2.0 * (rvx * D[3 * v.SN + q] + rvz * D[4 * v.SN + q]);
 }
 
 // The kept last row of dxi_z/dz is -dxi_x/dx unstretch (:954): its adjoint
@@ -356,14 +410,15 @@ __global__ void k_adj_preset(const double *__restrict__ pb, double *__restrict__
     DXB[((size_t)b * nz + nz - 1) * nx + x] += -unstretch_last * pb[q];
 }
 
-// Yb xi_x = -dx(DXB), Yb xi_z = XZP + Dz3^T DZB
-__global__ void k_adj_c(Views v, const double *__restrict__ DDXB, const double *__restrict__ XZP,
-                        const double *__restrict__ DZ3B, double *__restrict__ Yb)
+// The displacement's adjoints: xi_x = -dx(DXB), xi_z = XZP + Dz3^T DZB
+__global__ __launch_bounds__(256) void k_adj_c(Views v, const double *__restrict__ DDXB,
+                                               const double *__restrict__ XZP, const double *__restrict__ DZ3B,
+                                               double *__restrict__ Rb, double *__restrict__ acc, double beta)
 {
     const size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
     if (q >= v.SN) return;
-    Yb[q] = -DDXB[q];
-    Yb[v.SN + q] = XZP[q] + DZ3B[q];
+    accumulate(acc, Rb, q, -DDXB[q], beta);
+    accumulate(acc, Rb, v.SN + q, XZP[q] + DZ3B[q], beta);
 }
 
 // lam[vz][b][o_rad][x] += gvz[b][k][x]
@@ -429,76 +484,129 @@ static ZDer zder_args(const DiscreteCtx &c, const double *in, double *out, int n
     return a;
 }
 
+// A second group of fields in the launch of a.
+static void zder_second(ZDer &a, const double *in, double *out, int nbatch, int ibc)
+{
+    a.in2 = in;
+    a.out2 = out;
+    a.nbatch2 = nbatch;
+    a.ibc2 = ibc;
+    if (a.transposed) dbyd2_edge_rows(a.nz, ibc, a.eb2);
+}
+
 bool discrete_segmented(const DiscreteCtx &c, int nbatch)
 {
     return zder_fits(zder_args(c, nullptr, nullptr, nbatch, 1, true), c.zseg);
 }
 
-// out = Dz_ibc in (ibc 1..3), the kept last row of ibc 3 preScale * pre[b *
-// preStride + x] (0 when pre is null), kept first row of ibc 2 0.
-static hipError_t dz(const DiscreteCtx &c, const double *in, double *out, int nbatch, int ibc, const double *pre,
-                     size_t preStride, double preScale)
+// One group of fields of a z-derivative: out = Dz_ibc in (or its transpose) of
+// nbatch fields, ibc 1..3.
+struct ZGroup {
+    const double *in;
+    double *out;
+    int nbatch, ibc;
+};
+
+// out = Dz_ibc in, the kept last row of ibc 3 preScale * pre[b * preStride + x]
+// (0 when pre is null; for the first group), kept first row of ibc 2 0; g2 (may
+// be null) a second group in the same launch.
+static hipError_t dz(const DiscreteCtx &c, const ZGroup &g, const ZGroup *g2, const double *pre, size_t preStride,
+                     double preScale)
 {
-    ZDer a = zder_args(c, in, out, nbatch, ibc, false);
-    if (discrete_segmented(c, nbatch)) {
+    ZDer a = zder_args(c, g.in, g.out, g.nbatch, g.ibc, false);
+    if (discrete_segmented(c, g.nbatch + (g2 ? g2->nbatch : 0))) {
         a.pre = pre;
         a.pre_stride = preStride;
         a.pre_scale = preScale;
         a.zero_kept = 1;
+        if (g2) zder_second(a, g2->in, g2->out, g2->nbatch, g2->ibc);
         return launch_zder(a, c.zseg, c.stream);
     }
-    dim3 grid((c.d.nx + kTX - 1) / kTX, (c.d.nz + kTJ - 1) / kTJ, nbatch);
-    hipLaunchKernelGGL(k_dz_dense, grid, dim3(256), 0, c.stream, in, out, c.d.nz, c.d.nx, c.M[ibc - 1],
-                       pre ? c.vN3 : nullptr, pre, preStride, preScale);
-    return hipGetLastError();
+    for (const ZGroup *k : {&g, g2}) {
+        if (!k) continue;
+        dim3 grid((c.d.nx + kTX - 1) / kTX, (c.d.nz + kTJ - 1) / kTJ, k->nbatch);
+        const double *const kp = k == &g ? pre : nullptr;
+        hipLaunchKernelGGL(k_dz_dense, grid, dim3(256), 0, c.stream, k->in, k->out, c.d.nz, c.d.nx, c.M[k->ibc - 1],
+                           kp ? c.vN3 : nullptr, kp, preStride, preScale);
+        DCHK(hipGetLastError());
+    }
+    return hipSuccess;
 }
 
 // out = Dz_ibc^T in (ibc 1..3, kept rows 0); prebar (may be null) gets the
-// adjoint of ibc 3's kept last row [nbatch][nx].
-static hipError_t dz_T(const DiscreteCtx &c, const double *in, double *out, int nbatch, int ibc, double *prebar)
+// adjoint of ibc 3's kept last row [nbatch][nx]; g2 as in dz.
+static hipError_t dz_T(const DiscreteCtx &c, const ZGroup &g, const ZGroup *g2, double *prebar)
 {
-    ZDer a = zder_args(c, in, out, nbatch, ibc, true);
-    if (discrete_segmented(c, nbatch)) {
+    ZDer a = zder_args(c, g.in, g.out, g.nbatch, g.ibc, true);
+    if (discrete_segmented(c, g.nbatch + (g2 ? g2->nbatch : 0))) {
         a.prebar = prebar;
+        a.prebar_stride = (size_t)c.d.nx;
+        if (g2) zder_second(a, g2->in, g2->out, g2->nbatch, g2->ibc);
         return launch_zder(a, c.zseg, c.stream);
     }
     if (prebar) {
-        hipLaunchKernelGGL(k_colsum_w, grid1((size_t)nbatch * c.d.nx), dim3(256), 0, c.stream, in, c.vN3, prebar,
-                           c.d.nz, c.d.nx, nbatch);
+        hipLaunchKernelGGL(k_colsum_w, grid1((size_t)g.nbatch * c.d.nx), dim3(256), 0, c.stream, g.in, c.vN3, prebar,
+                           c.d.nz, c.d.nx, g.nbatch);
         DCHK(hipGetLastError());
     }
-    dim3 grid((c.d.nx + kTX - 1) / kTX, (c.d.nz + kTJ - 1) / kTJ, nbatch);
-    hipLaunchKernelGGL(k_dz_dense, grid, dim3(256), 0, c.stream, in, out, c.d.nz, c.d.nx, c.MT[ibc - 1], nullptr,
-                       nullptr, 0, 0.0);
+    for (const ZGroup *k : {&g, g2}) {
+        if (!k) continue;
+        dim3 grid((c.d.nx + kTX - 1) / kTX, (c.d.nz + kTJ - 1) / kTJ, k->nbatch);
+        hipLaunchKernelGGL(k_dz_dense, grid, dim3(256), 0, c.stream, k->in, k->out, c.d.nz, c.d.nx, c.MT[k->ibc - 1],
+                           nullptr, nullptr, 0, 0.0);
+        DCHK(hipGetLastError());
+    }
+    return hipSuccess;
+}
+
+// Dz3^T of the dxi_z/dz adjoint DZB, and the adjoint of its kept last row
+// (-dxi_x/dx unstretch, physics2d.f90:954) into the last row of DXB: by the
+// segmented solve itself, or by a column sum.
+static hipError_t dz3_T(const DiscreteCtx &c, const DiscreteWork &w)
+{
+    const Dims &d = c.d;
+    if (discrete_segmented(c, d.S)) {
+        ZDer a = zder_args(c, w.DZB, w.DZ3B, d.S, 3, true);
+        a.prebar = w.DXB + (size_t)(d.nz - 1) * d.nx;
+        a.prebar_stride = (size_t)d.nz * d.nx;
+        a.prebar_add = -c.unstretch_last;
+        return launch_zder(a, c.zseg, c.stream);
+    }
+    DCHK(dz_T(c, {w.DZB, w.DZ3B, d.S, 3}, nullptr, w.PB));
+    hipLaunchKernelGGL(k_adj_preset, grid1((size_t)d.S * d.nx), dim3(256), 0, c.stream, w.PB, w.DXB, d.nz, d.nx, d.S,
+                       c.unstretch_last);
     return hipGetLastError();
 }
 
-static hipError_t ddx(const DiscreteCtx &c, const double *in, double *out, int nrows)
+static hipError_t ddx(const DiscreteCtx &c, const double *in, double *out, int nrows, const double *in2 = nullptr,
+                      double *out2 = nullptr, int nrows2 = 0)
 {
-    return launch_ddx_rows(in, out, nrows, c.d.nx, c.bg.tw, c.bg.dmul, c.bg.cdx, c.bg.stretchx, c.stream);
+    return launch_ddx_rows2(in, out, nrows, in2, out2, nrows2, c.d.nx, c.bg.tw, c.bg.dmul, c.bg.cdx, c.bg.stretchx,
+                            c.stream);
 }
 
-// One forward RHS evaluation of the stage state Y at time t: R (full state)
-// and the stage quantities D = [div, dvx/dx, dvz/dx, dvx/dz, dvz/dz].
-static hipError_t fwd_rhs(const DiscreteCtx &c, const DiscreteWork &w, const double *Y, int t, double *R,
-                          double *D)
+// One forward stage: the next stage's input Yn = U + beta * RHS(Y, t) (Yn may be Y,
+// not U) and the stage quantities D = [div, dvx/dx, dvz/dx, dvx/dz, dvz/dz].
+static hipError_t fwd_stage(const DiscreteCtx &c, const DiscreteWork &w, const double *Y, int t, const double *U,
+                            double beta, double *Yn, double *D)
 {
     const Dims &d = c.d;
     const Views v{w.SN, w.PZ1, w.PX1};
     const int S = d.S;
-    // dxi_x/dx, dv_x/dx, dv_z/dx
-    DCHK(ddx(c, Y, w.T0, S * d.nz));
-    DCHK(ddx(c, Y + 2 * w.SN, D + w.SN, 2 * S * d.nz));
-    // dxi_z/dz (ibc 3, kept last row -dxi_x/dx unstretch), dv_x/dz, dv_z/dz (ibc 1)
-    DCHK(dz(c, Y + w.SN, w.T1, S, 3, w.T0 + (size_t)(d.nz - 1) * d.nx, (size_t)d.nz * d.nx, -c.unstretch_last));
-    DCHK(dz(c, Y + 2 * w.SN, D + 3 * w.SN, 2 * S, 1, nullptr, 0, 0.0));
-    hipLaunchKernelGGL(k_fwd_b, grid1(w.SN), dim3(256), 0, c.stream, d, c.bg, v, Y, w.T0, w.T1, D, w.T2, w.T3, R);
+    // dxi_x/dx; dv_x/dx, dv_z/dx
+    DCHK(ddx(c, Y, w.T0, S * d.nz, Y + 2 * w.SN, D + w.SN, 2 * S * d.nz));
+    // dxi_z/dz (ibc 3, kept last row -dxi_x/dx unstretch); dv_x/dz, dv_z/dz (ibc 1)
+    const ZGroup vel{Y + 2 * w.SN, D + 3 * w.SN, 2 * S, 1};
+    DCHK(dz(c, {Y + w.SN, w.T1, S, 3}, &vel, w.T0 + (size_t)(d.nz - 1) * d.nx, (size_t)d.nz * d.nx,
+            -c.unstretch_last));
+    hipLaunchKernelGGL(k_fwd_b, grid2(d), dim3(256), 0, c.stream, d, c.bg, v, Y, w.T0, w.T1, D, w.T2, w.T3, U, beta,
+                       Yn);
     DCHK(hipGetLastError());
     // dp/dx, dp/dz (ibc 2, its first row 0)
     DCHK(ddx(c, w.T2, w.T0, S * d.nz));
-    DCHK(dz(c, w.T2, w.T1, S, 2, nullptr, 0, 0.0));
-    hipLaunchKernelGGL(k_fwd_c, grid1(w.SN), dim3(256), 0, c.stream, d, c.bg, v, c.src, t, Y, w.T0, w.T1, w.T3,
-                       D + w.SN, R);
+    DCHK(dz(c, {w.T2, w.T1, S, 2}, nullptr, nullptr, 0, 0.0));
+    hipLaunchKernelGGL(k_fwd_c, grid2(d), dim3(256), 0, c.stream, d, c.bg, v, c.src, t, Y, w.T0, w.T1, w.T3,
+                       D + w.SN, U, beta, Yn);
     return hipGetLastError();
 }
 
@@ -507,23 +615,19 @@ static hipError_t fwd_rhs(const DiscreteCtx &c, const DiscreteWork &w, const dou
 static hipError_t fwd_step(const DiscreteCtx &c, const DiscreteWork &w, const double *U, int t, double *Unew,
                            double *Dst)
 {
-    for (int s = 0; s < 5; s++) {
-        hipLaunchKernelGGL(k_axpy, grid1(w.NST), dim3(256), 0, c.stream, U, w.R, s == 0 ? 0.0 : c.betas[s], w.Y,
-                           w.NST);
-        DCHK(hipGetLastError());
-        DCHK(fwd_rhs(c, w, w.Y, t, w.R, Dst ? Dst + (size_t)s * 5 * w.SN : w.Dscr));
-    }
-    const Views v{w.SN, w.PZ1, w.PX1};
-    hipLaunchKernelGGL(k_update_filter, grid1(w.NST), dim3(256), 0, c.stream, c.d, v, U, w.R, c.deltat, Unew);
+    for (int s = 0; s < 5; s++)
+        DCHK(fwd_stage(c, w, s == 0 ? U : w.Y, t, U, s < 4 ? c.betas[s + 1] : c.deltat, w.Y,
+                       Dst ? Dst + (size_t)s * 5 * w.SN : w.Dscr));
+    hipLaunchKernelGGL(k_filter, grid_filter(c.d), dim3(256), 0, c.stream, c.d, Views{w.SN, w.PZ1, w.PX1}, w.Y, Unew);
     return hipGetLastError();
 }
 
 // Transpose of one step at time t: lam (adjoint of the state after the step)
-// -> adjoint of U_t, accumulating the gradient into G.  Dkept: the step's
-// stage quantities [5][5][SN] kept by the segment recompute, or null to
+// -> acc, the adjoint of U_t, accumulating the gradient into G.  Dkept: the
+// step's stage quantities [5][5][SN] kept by the segment recompute, or null to
 // recompute them from U here.
-static hipError_t bwd_step(const DiscreteCtx &c, const DiscreteWork &w, const double *U, int t, double *lam,
-                           double *G, const double *Dkept)
+static hipError_t bwd_step(const DiscreteCtx &c, const DiscreteWork &w, const double *U, int t, const double *lam,
+                           double *acc, double *G, const double *Dkept)
 {
     const Dims &d = c.d;
     const Views v{w.SN, w.PZ1, w.PX1};
@@ -533,32 +637,24 @@ static hipError_t bwd_step(const DiscreteCtx &c, const DiscreteWork &w, const do
         DCHK(fwd_step(c, w, U, t, w.Unext, w.Dst));          // the stage quantities of this step
         Dst = w.Dst;
     }
-    hipLaunchKernelGGL(k_filter_T, grid1(w.NST), dim3(256), 0, c.stream, d, v, lam, w.acc);
-    DCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_axpy, grid1(w.NST), dim3(256), 0, c.stream, w.acc, w.acc, c.deltat - 1.0, w.Rb, w.NST);
+    hipLaunchKernelGGL(k_filter_T, grid_filter(d), dim3(256), 0, c.stream, d, v, lam, c.deltat, acc, w.Rb);
     DCHK(hipGetLastError());
     for (int s = 4; s >= 0; s--) {
-        hipLaunchKernelGGL(k_adj_a, grid1(w.SN), dim3(256), 0, c.stream, d, c.bg, v, w.Rb, w.FX, w.FZ, w.GZ, w.RHOB,
-                           w.Yb);
+        const double beta = s > 0 ? c.betas[s] : 0.0;
+        hipLaunchKernelGGL(k_adj_a, grid2(d), dim3(256), 0, c.stream, d, c.bg, v, w.Rb, acc, beta, w.FX, w.FZ, w.GZ);
         DCHK(hipGetLastError());
         DCHK(ddx(c, w.FX, w.DFX, 3 * S * d.nz));
-        DCHK(dz_T(c, w.FZ, w.DFZ, 2 * S, 1, nullptr));
-        DCHK(dz_T(c, w.GZ, w.DGZ, S, 2, nullptr));
-        hipLaunchKernelGGL(k_adj_b, grid1(w.SN), dim3(256), 0, c.stream, d, c.bg, v, w.Rb, w.DFX, w.DFZ, w.DGZ,
-                           w.RHOB, Dst + (size_t)s * 5 * w.SN, w.Yb, w.XZP, w.DXB, w.DZB, G);
+        const ZGroup gradp{w.GZ, w.DGZ, S, 2};
+        DCHK(dz_T(c, {w.FZ, w.DFZ, 2 * S, 1}, &gradp, nullptr));
+        hipLaunchKernelGGL(k_adj_b, grid2(d), dim3(256), 0, c.stream, d, c.bg, v, w.Rb, acc, beta, w.DFX, w.DFZ, w.DGZ,
+                           Dst + (size_t)s * 5 * w.SN, w.XZP, w.DXB, w.DZB, G);
         DCHK(hipGetLastError());
-        DCHK(dz_T(c, w.DZB, w.DZ3B, S, 3, w.PB));
-        hipLaunchKernelGGL(k_adj_preset, grid1((size_t)S * d.nx), dim3(256), 0, c.stream, w.PB, w.DXB, d.nz, d.nx,
-                           S, c.unstretch_last);
-        DCHK(hipGetLastError());
+        DCHK(dz3_T(c, w));
         DCHK(ddx(c, w.DXB, w.DDXB, S * d.nz));
-        hipLaunchKernelGGL(k_adj_c, grid1(w.SN), dim3(256), 0, c.stream, v, w.DDXB, w.XZP, w.DZ3B, w.Yb);
-        DCHK(hipGetLastError());
-        hipLaunchKernelGGL(k_accum, grid1(w.NST), dim3(256), 0, c.stream, w.acc, w.Rb, w.Yb,
-                           s > 0 ? c.betas[s] : 0.0, w.NST);
+        hipLaunchKernelGGL(k_adj_c, grid1(w.SN), dim3(256), 0, c.stream, v, w.DDXB, w.XZP, w.DZ3B, w.Rb, acc, beta);
         DCHK(hipGetLastError());
     }
-    return hipMemcpyAsync(lam, w.acc, w.NST * sizeof(double), hipMemcpyDeviceToDevice, c.stream);
+    return hipSuccess;
 }
 
 hipError_t discrete_gradient(const DiscreteCtx &c, const DiscreteWork &w, int maxtime, int interval,
@@ -568,16 +664,20 @@ hipError_t discrete_gradient(const DiscreteCtx &c, const DiscreteWork &w, int ma
     const int S = d.S;
     const int C = interval;
     const int nseg = (maxtime + C) / C;                       // segments start at 0, C, 2C, ...
-    // forward pass from the zero state, keeping the state at every segment start
-    DCHK(launch_fill(w.U, w.NST, 0.0, c.stream));
-    for (int t = 0; t <= maxtime; t++) {
+    // forward pass from the zero state, keeping the state at every segment
+    // start; the last segment's own steps are left to its recompute
+    double *U = w.U, *Un = w.Unext;
+    DCHK(launch_fill(U, w.NST, 0.0, c.stream));
+    for (int t = 0; t <= (nseg - 1) * C; t++) {
         if (t % C == 0)
-            DCHK(hipMemcpyAsync(w.ck + (size_t)(t / C) * w.NST, w.U, w.NST * sizeof(double),
-                                hipMemcpyDeviceToDevice, c.stream));
-        DCHK(fwd_step(c, w, w.U, t, w.Unext, nullptr));
-        DCHK(hipMemcpyAsync(w.U, w.Unext, w.NST * sizeof(double), hipMemcpyDeviceToDevice, c.stream));
+            DCHK(hipMemcpyAsync(w.ck + (size_t)(t / C) * w.NST, U, w.NST * sizeof(double), hipMemcpyDeviceToDevice,
+                                c.stream));
+        if (t == (nseg - 1) * C) break;
+        DCHK(fwd_step(c, w, U, t, Un, nullptr));
+        std::swap(U, Un);
     }
-    DCHK(launch_fill(w.lam, w.NST, 0.0, c.stream));
+    double *lam = w.lam, *acc = w.acc;
+    DCHK(launch_fill(lam, w.NST, 0.0, c.stream));
     DCHK(launch_fill(G, 3 * w.SN, 0.0, c.stream));
     for (int j = nseg - 1; j >= 0; j--) {
         const int t0 = j * C, t1 = std::min(maxtime, t0 + C - 1);
@@ -593,12 +693,13 @@ hipError_t discrete_gradient(const DiscreteCtx &c, const DiscreteWork &w, int ma
                           w.Dseg ? w.Dseg + (size_t)(t - t0) * D1 : nullptr));
         for (int t = t1; t >= t0; t--) {
             if (t % c.steps == 0) {                            // output k after step t
-                hipLaunchKernelGGL(k_inject, grid1((size_t)S * d.nx), dim3(256), 0, c.stream, w.lam, gvz,
-                                   t / c.steps, nt, c.orow, d.nz, d.nx, S, w.SN);
+                hipLaunchKernelGGL(k_inject, grid1((size_t)S * d.nx), dim3(256), 0, c.stream, lam, gvz, t / c.steps, nt,
+                                   c.orow, d.nz, d.nx, S, w.SN);
                 DCHK(hipGetLastError());
             }
-            DCHK(bwd_step(c, w, w.seg + (size_t)(t - t0) * w.NST, t, w.lam, G,
+            DCHK(bwd_step(c, w, w.seg + (size_t)(t - t0) * w.NST, t, lam, acc, G,
                           w.Dseg ? w.Dseg + (size_t)(t - t0) * D1 : nullptr));
+            std::swap(lam, acc);
         }
     }
     return hipSuccess;
@@ -613,7 +714,7 @@ hipError_t discrete_flow_chain(const DiscreteCtx &c, const DiscreteWork &w, cons
     const int n2 = d.nz * d.nx;
     hipLaunchKernelGGL(k_flow_in, grid1(w.SN), dim3(256), 0, c.stream, v, n2, rho0, G, w.FX, w.FZ);
     DCHK(hipGetLastError());
-    DCHK(dz_T(c, w.FX, w.DFX, d.S, 1, nullptr));   // Dz1^T (Gx / rho0)
+    DCHK(dz_T(c, {w.FX, w.DFX, d.S, 1}, nullptr, nullptr));                  // Dz1^T (Gx / rho0)
     DCHK(ddx(c, w.FZ, w.DFZ, d.S * d.nz));                                   // dx (Gz / rho0)
     hipLaunchKernelGGL(k_flow_out, grid1(w.SN), dim3(256), 0, c.stream, v, n2, rho0, c2, psi, scale, dimc, G,
                        w.DFX, w.DFZ, gpsi, gc);
@@ -625,8 +726,8 @@ hipError_t discrete_apply(const DiscreteCtx &c, const double *in, double *out, i
 {
     // which: 0..2 Dz of ibc 1..3, 3..5 their transposes
     if (which < 0 || which > 5) return hipErrorInvalidValue;
-    return which < 3 ? dz(c, in, out, nbatch, which + 1, nullptr, 0, 0.0)
-                     : dz_T(c, in, out, nbatch, which - 2, which == 5 ? presetN_bar : nullptr);
+    return which < 3 ? dz(c, {in, out, nbatch, which + 1}, nullptr, nullptr, 0, 0.0)
+                     : dz_T(c, {in, out, nbatch, which - 2}, nullptr, which == 5 ? presetN_bar : nullptr);
 }
 
 }  // namespace sparc

@@ -84,45 +84,60 @@ __global__ __launch_bounds__(64) void k_ddz_cols(const double *in, double *out,
             fft_deriv_team<N1, N2>(RE, IM, T, LDS, TW, DM, SX);                                \
     } while (0)
 
-// Generic x-derivative (ddx) of nrows real rows of length NX; two rows per
-// FFT team.
+// Rows of a batch in two arrays: n of the first, then m of the second.
+struct RowSets {
+    const double *in, *in2;
+    double *out, *out2;
+    int n, m;
+    __device__ __forceinline__ int count() const { return n + m; }
+    __device__ __forceinline__ const double *src(int r, int nx) const
+    {
+        return r < n ? in + (size_t)r * nx : in2 + (size_t)(r - n) * nx;
+    }
+    __device__ __forceinline__ double *dst(int r, int nx) const
+    {
+        return r < n ? out + (size_t)r * nx : out2 + (size_t)(r - n) * nx;
+    }
+};
+
+// Generic x-derivative (ddx) of real rows of length NX; two rows per FFT team.
 template <int NX>
-__global__ __launch_bounds__(64) void k_ddx_rows(const double *__restrict__ in,
-                                                 double *__restrict__ out, int nrows,
-                                                 const double2 *__restrict__ tw,
+__global__ __launch_bounds__(64) void k_ddx_rows(RowSets rs, const double2 *__restrict__ tw,
                                                  const double *__restrict__ dmul, double stretchx)
 {
     constexpr int N1 = FftShape<NX>::N1, N2 = FftShape<NX>::N2, TEAMS = 64 / N1;
     __shared__ double2 lds[TEAMS][FftLds<N1, N2>::n];
     const int team = threadIdx.x / N1, t = threadIdx.x % N1;
     const int r0 = 2 * (blockIdx.x * TEAMS + team), r1 = r0 + 1;
+    const int nrows = rs.count();
+    const double *const i0 = rs.src(min(r0, nrows - 1), NX), *const i1 = rs.src(min(r1, nrows - 1), NX);
     double re[N2], im[N2];
 #pragma unroll
     for (int j2 = 0; j2 < N2; j2++) {
         const int x = t + N1 * j2;
-        re[j2] = r0 < nrows ? in[(size_t)r0 * NX + x] : 0.0;
-        im[j2] = r1 < nrows ? in[(size_t)r1 * NX + x] : 0.0;
+        re[j2] = i0[x];
+        im[j2] = i1[x];
     }
     fft_deriv_team<N1, N2>(re, im, t, lds[team], tw, dmul, stretchx);
+    double *const o0 = rs.dst(min(r0, nrows - 1), NX), *const o1 = rs.dst(min(r1, nrows - 1), NX);
 #pragma unroll
     for (int j2 = 0; j2 < N2; j2++) {
         const int x = t + N1 * j2;
-        if (r0 < nrows) out[(size_t)r0 * NX + x] = re[j2];
-        if (r1 < nrows) out[(size_t)r1 * NX + x] = im[j2];
+        if (r0 < nrows) o0[x] = re[j2];
+        if (r1 < nrows) o1[x] = im[j2];
     }
 }
 
 // Derivative of many lines whose length is not a power of two (sparc_circ.h),
 // two lines per team of s.lanes lanes, G teams per block.
-//   AXIS 0: count rows of length n, contiguous; a team takes rows 2 g, 2 g + 1.
-//   AXIS 1: count column pairs (x0, x0 + 1) of [n][nx] planes, nx even, so
-//           every pair is 16-byte aligned.
+//   AXIS 0: count rows of length n; a team takes rows 2 g, 2 g + 1.
+//   AXIS 1: count column pairs (x0, x0 + 1) of [n][nx] planes (of the first array),
+//           nx even, so every pair is 16-byte aligned.
 // Both directions of global access run with the fastest index over the lanes;
 // the doubled lines and then the results wait in LDS.
 template <int AXIS>
-__global__ __launch_bounds__(256) void k_circ(const double *__restrict__ in, double *__restrict__ out, long count,
-                                              int nx, CircShape s, int G, const double *__restrict__ cd,
-                                              double stretch)
+__global__ __launch_bounds__(256) void k_circ(RowSets rs, long count, int nx, CircShape s, int G,
+                                              const double *__restrict__ cd, double stretch)
 {
     extern __shared__ double2 circ_lds[];
     constexpr int U = 4;                     // elements per lane whose loads are issued together
@@ -161,7 +176,6 @@ __global__ __launch_bounds__(256) void k_circ(const double *__restrict__ in, dou
     // address of element j of line (or pair) i of the block; lines past the end: none
     auto present = [&](int i) { return AXIS == 0 ? 2 * b0 + i < count : b0 + i < count; };
     auto base = [&](int i) -> size_t {
-        if (AXIS == 0) return (size_t)(2 * b0 + i) * s.n;
         const long pair = b0 + i, hx = nx >> 1, pl = pair / hx;
         return (size_t)pl * s.n * nx + 2 * (size_t)(pair - pl * hx);
     };
@@ -172,9 +186,9 @@ __global__ __launch_bounds__(256) void k_circ(const double *__restrict__ in, dou
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const bool ok = os[u] < slow && present(os[u]);
-                const size_t q = ok ? base(os[u]) + fs[u] : 0;
-                a[u] = ok ? in[q] : 0.0;
-                b[u] = ok && s.nk == 2 ? in[q + half] : 0.0;
+                const double *const in = rs.src(ok ? (int)(2 * b0) + os[u] : 0, s.n) + (ok ? fs[u] : 0);
+                a[u] = ok ? in[0] : 0.0;
+                b[u] = ok && s.nk == 2 ? in[half] : 0.0;
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
@@ -199,8 +213,8 @@ __global__ __launch_bounds__(256) void k_circ(const double *__restrict__ in, dou
             for (int u = 0; u < U; u++) {
                 const bool ok = os[u] < slow && present(fs[u]);
                 const size_t q = ok ? base(fs[u]) + (size_t)os[u] * nx : 0;
-                a[u] = ok ? *(const double2 *)(in + q) : make_double2(0.0, 0.0);
-                b[u] = ok && s.nk == 2 ? *(const double2 *)(in + q + half) : make_double2(0.0, 0.0);
+                a[u] = ok ? *(const double2 *)(rs.in + q) : make_double2(0.0, 0.0);
+                b[u] = ok && s.nk == 2 ? *(const double2 *)(rs.in + q + half) : make_double2(0.0, 0.0);
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
@@ -236,16 +250,16 @@ __global__ __launch_bounds__(256) void k_circ(const double *__restrict__ in, dou
             if (os[u] >= slow || !present(i)) continue;
             if constexpr (AXIS == 0) {
                 const double *e = (const double *)(E + (i >> 1) * per) + (i & 1);
-                const size_t q = base(i) + j;
+                double *const out = rs.dst((int)(2 * b0) + i, s.n) + j;
                 const double p = e[2 * j], m = s.nk == 2 ? e[2 * (s.ext + j)] : 0.0;
-                out[q] = p + m;
-                if (s.nk == 2) out[q + half] = p - m;
+                out[0] = p + m;
+                if (s.nk == 2) out[half] = p - m;
             } else {
                 const double2 *const e = E + i * per;
                 const size_t q = base(i) + (size_t)j * nx;
                 const double2 p = e[j], m = s.nk == 2 ? e[s.ext + j] : make_double2(0.0, 0.0);
-                *(double2 *)(out + q) = make_double2(p.x + m.x, p.y + m.y);
-                if (s.nk == 2) *(double2 *)(out + q + half) = make_double2(p.x - m.x, p.y - m.y);
+                *(double2 *)(rs.out + q) = make_double2(p.x + m.x, p.y + m.y);
+                if (s.nk == 2) *(double2 *)(rs.out + q + half) = make_double2(p.x - m.x, p.y - m.y);
             }
         }
     });
@@ -726,23 +740,30 @@ hipError_t launch_vz_norm2(const double *vz, int S, size_t n2, const Clock &c, c
     return hipGetLastError();
 }
 
-hipError_t launch_ddx_rows(const double *in, double *out, int nrows, int nx, const double2 *tw,
-                           const double *dmul, const double *cdx, double stretchx, hipStream_t st)
+hipError_t launch_ddx_rows(const double *in, double *out, int nrows, int nx, const double2 *tw, const double *dmul,
+                           const double *cdx, double stretchx, hipStream_t st)
 {
-    const int npairs = (nrows + 1) / 2;
+    return launch_ddx_rows2(in, out, nrows, nullptr, nullptr, 0, nx, tw, dmul, cdx, stretchx, st);
+}
+
+hipError_t launch_ddx_rows2(const double *in, double *out, int nrows, const double *in2, double *out2, int nrows2,
+                            int nx, const double2 *tw, const double *dmul, const double *cdx, double stretchx,
+                            hipStream_t st)
+{
+    const RowSets rs{in, in2, out, out2, nrows, nrows2};
+    const int npairs = (nrows + nrows2 + 1) / 2;
     if (!nx_has_fft(nx)) {
         if (nx < 16 || nx > 1024) return hipErrorInvalidValue;
         const CircBatch c = circ_batch(nx, 0);
-        hipLaunchKernelGGL((k_circ<0>), dim3((npairs + c.G - 1) / c.G), dim3(256), c.lds, st, in, out, (long)nrows, nx,
-                           c.s, c.G, cdx, stretchx);
+        hipLaunchKernelGGL((k_circ<0>), dim3((npairs + c.G - 1) / c.G), dim3(256), c.lds, st, rs, (long)(nrows + nrows2),
+                           nx, c.s, c.G, cdx, stretchx);
         return hipGetLastError();
     }
 #define L(NXV)                                                                              \
     {                                                                                       \
         constexpr int TEAMS = 64 / FftShape<NXV>::N1;                                      \
         dim3 grid((npairs + TEAMS - 1) / TEAMS);                                            \
-        hipLaunchKernelGGL(k_ddx_rows<NXV>, grid, dim3(64), 0, st, in, out, nrows, tw, dmul, \
-                           stretchx);                                                       \
+        hipLaunchKernelGGL(k_ddx_rows<NXV>, grid, dim3(64), 0, st, rs, tw, dmul, stretchx);     \
     }
     SPARC_DISPATCH_NX(nx, L)
 #undef L
@@ -755,8 +776,8 @@ hipError_t launch_ddy_any(const double *in, double *out, int nplanes, int nx, in
     if (ny < 16 || ny > 1024 || (nx & 1)) return hipErrorInvalidValue;
     const CircBatch c = circ_batch(ny, 1);
     const long pairs = (long)nplanes * (nx / 2);
-    hipLaunchKernelGGL((k_circ<1>), dim3((unsigned)((pairs + c.G - 1) / c.G)), dim3(256), c.lds, st, in, out, pairs, nx,
-                       c.s, c.G, cdy, stretch);
+    hipLaunchKernelGGL((k_circ<1>), dim3((unsigned)((pairs + c.G - 1) / c.G)), dim3(256), c.lds, st,
+                       RowSets{in, nullptr, out, nullptr, 0, 0}, pairs, nx, c.s, c.G, cdy, stretch);
     return hipGetLastError();
 }
 

@@ -12,6 +12,10 @@ hipError_t launch_ddz_cols(const double *in, double *out, int ncols, int nz, int
 // the circulant product (cdx, Bg::cdx's layout) for any other nx in [16, 1024].
 hipError_t launch_ddx_rows(const double *in, double *out, int nrows, int nx, const double2 *tw,
                            const double *dmul, const double *cdx, double stretchx, hipStream_t st);
+// The same of two sets of rows in one launch (nrows2 may be 0).
+hipError_t launch_ddx_rows2(const double *in, double *out, int nrows, const double *in2, double *out2, int nrows2,
+                            int nx, const double2 *tw, const double *dmul, const double *cdx, double stretchx,
+                            hipStream_t st);
 // y-derivative of nplanes [ny][nx] planes for an ny in [16, 1024] that is not a power
 // of two (nx even).
 hipError_t launch_ddy_any(const double *in, double *out, int nplanes, int nx, int ny, const double *cdy,
@@ -71,11 +75,11 @@ struct DiscreteCtx {
 };
 struct DiscreteWork {
     size_t SN, PZ1, PX1, NST;      // one [S][nz][nx] field, one pz field, one px field, a full state
-    double *U, *Unext, *Y, *R, *acc, *Rb, *Yb, *lam;          // NST each
+    double *U, *Unext, *Y, *acc, *Rb, *lam;                   // NST each
     double *ck, *seg;                                         // segment starts, one segment of states
     double *Dst, *Dscr;                                       // [5][5][SN], [5][SN]
     double *Dseg;                                             // [interval][5][5][SN] or null
-    double *T0, *T1, *T2, *T3, *GZ, *DGZ, *RHOB, *XZP, *DXB, *DZB, *DZ3B, *DDXB;   // SN each
+    double *T0, *T1, *T2, *T3, *GZ, *DGZ, *XZP, *DXB, *DZB, *DZ3B, *DDXB;   // SN each
     double *FX, *DFX, *FZ, *DFZ;                              // 3, 3, 2, 2 SN
     double *PB;                                               // [S][nx]
 };

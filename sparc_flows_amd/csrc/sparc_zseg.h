@@ -31,11 +31,19 @@ struct ZDer {
     const double *pre;
     size_t pre_stride;
     double pre_scale;
-    // transposed (ibc 1..3, kept rows 0): eb from dbyd2_edge_rows; prebar
-    // [nbatch][ncols] gets the adjoint of ibc 3's kept last row (may be null)
+    // transposed (ibc 1..3, kept rows 0): eb from dbyd2_edge_rows; prebar[b *
+    // prebar_stride + column] gets the adjoint of ibc 3's kept last row (may be null), or
+    // prebar_add times it added where that is not 0
     int transposed;
     double eb[20];
     double *prebar;
+    size_t prebar_stride;
+    double prebar_add;
+    // a second set of nbatch2 fields (0: none) of another ibc, without pre and prebar
+    const double *in2;
+    double *out2;
+    int nbatch2, ibc2;
+    double eb2[20];
 };
 // Whether the segmented form takes it: tables, and 32-bit offsets in a field.
 bool zder_fits(const ZDer &a, const ZSeg &sg);

@@ -100,7 +100,12 @@ __global__ __launch_bounds__(512) void k_zder(ZDer z, ZSeg sg)
     double *const tile = yb + NC * LY + 2 * NC;             // filter, transpose: [nzp] rows of NC, two more before and after
     const int tid = threadIdx.x, nthr = blockDim.x, nz = z.nz;
     const int c0 = (int)blockIdx.x * NC + tid % NC;
-    const size_t fo = (size_t)blockIdx.y * nz * z.ncols;
+    const bool two = (int)blockIdx.y >= z.nbatch;           // the second set of fields
+    const int ibc = two ? z.ibc2 : z.ibc, fb = (int)blockIdx.y - (two ? z.nbatch : 0);
+    const size_t fo = (size_t)fb * nz * z.ncols;
+    const double *const in = (two ? z.in2 : z.in) + fo;
+    double *const oc = (two ? z.out2 : z.out) + fo;
+    const double *const pre = two ? nullptr : z.pre;
     Lane ln;
     ln.c = tid % NC;
     ln.s = min(tid / NC, P - 1);
@@ -118,16 +123,16 @@ __global__ __launch_bounds__(512) void k_zder(ZDer z, ZSeg sg)
     double win[MS + 6], e[5], p0 = 0.0, pN = 0.0;
     if (TR) {
 #pragma unroll
-        for (int i = 0; i < MS; i++) Y[i] = ldg(z.in + fo, ln.row(ln.a + i));
+        for (int i = 0; i < MS; i++) Y[i] = ldg(in, ln.row(ln.a + i));
     } else {
-        load_window<MS>(z.in + fo, ln, win, e);
-        if (z.ibc == 2 && !z.zero_kept) p0 = ldg(z.out + fo, ln.row(0));
-        if (z.ibc == 3 && (z.pre || !z.zero_kept))
-            pN = z.pre ? z.pre_scale * z.pre[(size_t)blockIdx.y * z.pre_stride + (ln.col >> 3)]
-                       : ldg(z.out + fo, ln.row(nz - 1));
+        load_window<MS>(in, ln, win, e);
+        if (ibc == 2 && !z.zero_kept) p0 = ldg(oc, ln.row(0));
+        if (ibc == 3 && (pre || !z.zero_kept))
+            pN = pre ? z.pre_scale * pre[(size_t)fb * z.pre_stride + (ln.col >> 3)]
+                       : ldg(oc, ln.row(nz - 1));
     }
     zero_lds(yb, NC * LY, tid, nthr);
-    stage_lds(lds, sg.img + (size_t)(TR ? 3 + z.ibc : z.ibc) * nset, nset, tid, nthr);
+    stage_lds(lds, sg.img + (size_t)(TR ? 3 + ibc : ibc) * nset, nset, tid, nthr);
     if (TR && tid < 2 * NC) {                               // zero rows around the tile
         tile[tid - 2 * NC] = 0.0;
         tile[nzp * NC + tid] = 0.0;
@@ -139,7 +144,7 @@ __global__ __launch_bounds__(512) void k_zder(ZDer z, ZSeg sg)
 #pragma unroll
         for (int i = 0; i < MS; i++) Y[i] = ln.a + i < nz ? Y[i] * st[i] : 0.0;
     } else {
-        seg_rhs<MS>([&](int k) { return win[k]; }, e, Y, ln.a, nz, ln.first, ln.last, z.ibc, p0, pN, sg.c1, sg.c2,
+        seg_rhs<MS>([&](int k) { return win[k]; }, e, Y, ln.a, nz, ln.first, ln.last, ibc, p0, pN, sg.c1, sg.c2,
                     sg.cb);
     }
     seg_solve<MS>(Y, tab);
@@ -150,7 +155,6 @@ __global__ __launch_bounds__(512) void k_zder(ZDer z, ZSeg sg)
     }
     __syncthreads();
     seg_correct<MS>(Y, ln.s, P, hw, yc, band, tab);
-    double *const oc = z.out + fo;
     if (!TR) {
 #pragma unroll
         for (int i = 0; i < MS; i++) Y[i] = Y[i] * st[i];
@@ -172,13 +176,15 @@ __global__ __launch_bounds__(512) void k_zder(ZDer z, ZSeg sg)
             const bool edge = TR && (j < 2 || (j >= nz - 2 && j < nz));
             tile[j * NC + ln.c] = edge || j >= nz ? 0.0 : Y[i];
             if (edge) ed[er * NC + ln.c] = Y[i];
-            if (TR && z.prebar && z.ibc == 3 && j == nz - 1 && ln.act)
-                z.prebar[(size_t)blockIdx.y * z.ncols + c0] = Y[i];
+            if (TR && z.prebar && !two && ibc == 3 && j == nz - 1 && ln.act) {
+                double *const pb = z.prebar + (size_t)fb * z.prebar_stride + c0;
+                *pb = z.prebar_add != 0.0 ? *pb + z.prebar_add * Y[i] : Y[i];
+            }
         }
     }
     __syncthreads();
     if (!ln.act) return;
-    const double *const t = tile + ln.c;
+    const double *const t = tile + ln.c, *const eb = two ? z.eb2 : z.eb;
 #pragma unroll
     for (int i = 0; i < MS; i++) {
         const int j = ln.a + i;
@@ -187,8 +193,8 @@ __global__ __launch_bounds__(512) void k_zder(ZDer z, ZSeg sg)
         if (TR) {
             v = sg.c1 * (t[(j - 1) * NC] - t[(j + 1) * NC]) + sg.c2 * (t[(j - 2) * NC] - t[(j + 2) * NC]);
             const int k = j < 5 ? j : j - nz + 5;
-            if (j < 5) v += z.eb[k] * ed[ln.c] + z.eb[5 + k] * ed[NC + ln.c];
-            if (j >= nz - 5) v += z.eb[10 + j - nz + 5] * ed[2 * NC + ln.c] + z.eb[15 + j - nz + 5] * ed[3 * NC + ln.c];
+            if (j < 5) v += eb[k] * ed[ln.c] + eb[5 + k] * ed[NC + ln.c];
+            if (j >= nz - 5) v += eb[10 + j - nz + 5] * ed[2 * NC + ln.c] + eb[15 + j - nz + 5] * ed[3 * NC + ln.c];
         } else if (j == 0 || j == nz - 1) {
             v = Y[i];
         } else if (j <= 4 || j >= nz - 5) {                // FILTER_VAR_Z (kernels.f90:891-928)
@@ -218,14 +224,14 @@ int lanes(int cols, int P) { return (cols * P + 63) / 64 * 64; }
 
 bool zder_fits(const ZDer &a, const ZSeg &sg)
 {
-    return sg.img && sg.P <= kZSegP && (size_t)a.nz * a.ncols < ((size_t)1 << 28) && a.nbatch <= 65535 &&
+    return sg.img && sg.P <= kZSegP && (size_t)a.nz * a.ncols < ((size_t)1 << 28) && a.nbatch + a.nbatch2 <= 65535 &&
            zder_lds(a, sg) <= 160 * 1024;
 }
 
 hipError_t launch_zder(const ZDer &a, const ZSeg &sg, hipStream_t st)
 {
     const size_t shm = zder_lds(a, sg);
-    const dim3 grid((unsigned)((a.ncols + kZdCols - 1) / kZdCols), (unsigned)a.nbatch), block(lanes(kZdCols, sg.P));
+    const dim3 grid((unsigned)((a.ncols + kZdCols - 1) / kZdCols), (unsigned)(a.nbatch + a.nbatch2)), block(lanes(kZdCols, sg.P));
 #define L(M)                                                                                     \
     if (sg.m == M) {                                                                             \
         const void *k = a.transposed ? (const void *)k_zder<M, true> : (const void *)k_zder<M, false>; \
