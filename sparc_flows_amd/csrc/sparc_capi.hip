@@ -1249,14 +1249,13 @@ int sparc_step(sparc_handle *h, int t)
     return SPARC_OK;
 }
 
-// Row-pass team width for nx = 256: the narrowest form whose waves still
-// reach every compute unit -- 64 lanes per row (one row per wave) when the
-// 32-lane form (two rows per wave) would leave compute units idle, else 32
-// lanes when the 16-lane form (four rows per wave) would, else 16 lanes.
-// Measured for one source: 32 lanes 10 % and 64 lanes a further 3 % faster
-// gradients; for 16 sources the 16-lane form is 2 % faster than 32 lanes.
-// (Timing a few steps with each width at set-up chose the 32-lane form for
-// 16 sources too.)  SPARC_ROW_WIDE (0, 1 or 2) forces the choice.
+// Row-pass team width for nx = 256: 16 lanes per row (four rows per wave) where that
+// still gives every SIMD a wave, else 32 lanes, and 64 lanes (one row per wave)
+// where 32 would leave half of the SIMDs idle.  us per launch at nz = 300 on 16 / 32
+// / 64 lanes: 1 source 14.1 / 10.7 / 10.0, 2 sources 15.2 / 12.4 / 11.8, 4 sources
+// 16.9 / 12.9 / 13.1, 8 sources 18.8 / 16.6 / 17.6, 16 sources 24.4 / 24.9 / 28.3
+// (first pass of a step 26.4 / 27.9 / 30.9).  SPARC_ROW_WIDE (0, 1 or 2) forces the
+// choice.
 static int tune_rows(sparc_handle *h)
 {
     h->row_wide = 0;
@@ -1270,7 +1269,7 @@ static int tune_rows(sparc_handle *h)
     HCHECK(h, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     const long rows = (long)h->S * h->nz;
     const long waves16 = (rows + 3) / 4, waves32 = (rows + 1) / 2;
-    h->row_wide = waves32 < ncu ? 2 : (waves16 < ncu ? 1 : 0);
+    h->row_wide = waves32 < 2 * ncu ? 2 : (waves16 < 4 * ncu ? 1 : 0);
     return SPARC_OK;
 }
 
