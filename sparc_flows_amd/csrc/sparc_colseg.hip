@@ -72,7 +72,8 @@ inline size_t colsplit_lds_bytes(int tc, const SegTab &sg, int nzpml)
 // (16 bytes).  With plain rows the pass was bound by the L1's one access per
 // clock: at TC = 2 a wave instruction touched 32 lines for 16 bytes each, 21 000
 // accesses per block, 9 of its 14 us (one source at 256x300; 21.1 us a launch
-// between events, now 17.2; 128x150 17.3 -> 15.8).
+// between events, then 17.2, and 16.9 with the source off the first solve's path and
+// shared windows of end values; 128x150 17.3 -> 15.8 -> 15.1).
 //
 // Loads and stores at a 32-bit byte offset from a wave-uniform base address:
 // the compiler then uses the SGPR-base + VGPR-offset addressing form, with no
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(384) void k_colsplit(Dims d, Bg bg, DbyCoef cf, Seg
     const int nstaged = (3 * nband + kZS * 3 * MS + kZF * nzp + kCB + kPL * nzpml * TC + nzp + 1) & ~1;
     const int LY = n2P + 4 * sg.hw + 2, hw2 = 2 * sg.hw;
     double *const yb0 = lds_dyn + nstaged;             // [4][TC][LY] end values: field groups 0-2, d p/dz
-    double *const wl = yb0 + 4 * TC * LY;              // [TC][nzp] group-1 part of RHS v_z,
+    double *const wl = yb0 + 4 * TC * LY;              // [TC][nzp] group 1's part of RHS v_z,
                                                        // then [TC][nzp] group 0's part, [TC][nzp] p
     const int tid = threadIdx.x, G = blockDim.x / 3;
     const int f = __builtin_amdgcn_readfirstlane(tid / G);   // the field group: one per wave
@@ -193,7 +194,6 @@ __global__ __launch_bounds__(384) void k_colsplit(Dims d, Bg bg, DbyCoef cf, Seg
         win[k + 1] = v.y;
     }
     const double topv = f == 0 ? ldb(st.topbc, (b * nx + x) * 8) : 0.0;
-    const double r0src = f == 0 ? ldb(bg.rho0_src, x * 8) : 1.0;   // the source lanes' rho0 at the source row
     double e[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     if (lastseg) {
 #pragma unroll
@@ -281,22 +281,6 @@ __global__ __launch_bounds__(384) void k_colsplit(Dims d, Bg bg, DbyCoef cf, Seg
         }
     }
     __syncthreads();
-    // source value of this column at its injection row (physics2d.f90:1051-1061)
-    double srcv = 0.0;
-    const int isrc = src.row - a;
-    if (f == 0 && act && isrc >= 0 && isrc < MS && time <= src.limit) {
-        if (src.mode == 1) {
-            // both loads issued before either is used (clamped time index)
-            double fsr = src.fwd[min(max(time, 0), max(src.nfwd - 1, 0))];
-            double vrx = src.vr[b * nx + x];
-            asm volatile("" : "+v"(fsr), "+v"(vrx));
-            const double fs = (time >= 0 && time < src.nfwd) ? fsr : 0.0;
-            srcv = vrx * fs * src.delta_width / r0src;
-        } else if (src.mode == 2) {
-            srcv = lagrange_forcing(src, b, x, nx, time) * src.delta_width / r0src;
-        }
-    }
-    const double pamp = (f == 0 && act) ? profile_amp(src, b, x, nx, a, MS, time) : 0.0;
     const int slot_f = f == 0 ? 2 : 0;                 // dbyd2 table set: ibc 3 or ibc 1
     double Y[MS], own[MS];
     const double *const cbt = cbl;                      // LDS: read only by the end segments' lanes
@@ -313,7 +297,7 @@ __global__ __launch_bounds__(384) void k_colsplit(Dims d, Bg bg, DbyCoef cf, Seg
     if (act)
         seg_correct_rows<MS>(Y, s, P, sg.hw, ybf + c * LY, mvs + (f == 0 ? 2 * nband : 0), gtab);
 
-    double *const w0 = wl + (TC + c) * nzp + a;       // group 0: -rho'/rho0 g + source
+    double *const w0 = wl + (TC + c) * nzp + a;       // group 0: -rho'/rho0 g
     double *const pcol = wl + (2 * TC + c) * nzp;     // p of this column (group 0)
     if (f == 0) {
         // z-PML (:957-967), divergence, p and rho' (:990-998, :1043)
@@ -355,9 +339,10 @@ __global__ __launch_bounds__(384) void k_colsplit(Dims d, Bg bg, DbyCoef cf, Seg
                 const double div = pa[i] + dz;
                 pv[i] = -(pb[i] * div) - gp0 * xiz;
                 const double rho = -(r0 * div) - gr0 * xiz;
-                double bzv = -rinv * (rho * gz);
-                if (src.mode == 3) bzv = bzv + pamp * zpl[j];
-                bv[i] = (i == isrc) ? bzv + srcv : bzv;
+                bv[i] = -rinv * (rho * gz);
+                // one row after the other: with all rows' table reads in flight the 10-row
+                // form spilled
+                asm volatile("" : "+v"(bv[i]), "+v"(pv[i]) :: "memory");
             }
         };
         if (segpml) epi(std::true_type{});
@@ -372,8 +357,12 @@ __global__ __launch_bounds__(384) void k_colsplit(Dims d, Bg bg, DbyCoef cf, Seg
             }
         }
     } else {
-        // group 1: flow part of RHS v_z (:1073-1077) to LDS, xi_z update;
-        // group 2: RHS v_x flow part (:1067-1071), xi_x update
+        // group 1: source and flow part of RHS v_z (:1051-1061, :1073-1077) to LDS,
+        // xi_z update; group 2: RHS v_x flow part (:1067-1071), xi_x update.  The
+        // source's loads and the adjoint's interpolation (seven divisions) stand here
+        // because group 0's epilogue takes 1.2 us longer than this one (before the
+        // first solve every wave of the block waited for them), and after the updates
+        // because their operands then need no registers any more.
         double r1[MS], r2[MS];                         // the xi update; group 1 its part of RHS v_z, group 2 RHS v_x
 #pragma unroll
         for (int i = 0; i < MS; i++) {
@@ -389,9 +378,30 @@ __global__ __launch_bounds__(384) void k_colsplit(Dims d, Bg bg, DbyCoef cf, Seg
             put2(X, i, r1[i], r1[i + 1]);
             if (f == 2) put2(st.rvx, i, r2[i], r2[i + 1]);
         }
+        double srcv = 0.0, pamp = 0.0;
+        const int isrc = src.row - a;
+        if (f == 1 && act && time <= src.limit) {
+            if (src.mode == 3) {
+                pamp = profile_amp(src, b, x, nx, a, MS, time);
+            } else if (isrc >= 0 && isrc < MS) {
+                if (src.mode == 1) {
+                    // the loads issued before any is used (clamped time index)
+                    double fsr = src.fwd[min(max(time, 0), max(src.nfwd - 1, 0))];
+                    double vrx = src.vr[b * nx + x], r0 = ldb(bg.rho0_src, x * 8);
+                    asm volatile("" : "+v"(fsr), "+v"(vrx), "+v"(r0));
+                    const double fs = (time >= 0 && time < src.nfwd) ? fsr : 0.0;
+                    srcv = vrx * fs * src.delta_width / r0;
+                } else if (src.mode == 2) {
+                    srcv = lagrange_forcing(src, b, x, nx, time) * src.delta_width / ldb(bg.rho0_src, x * 8);
+                }
+            }
+        }
         if (f == 1 && act) {
 #pragma unroll
-            for (int i = 0; i < MS; i++) wl[c * nzp + a + i] = r2[i];
+            for (int i = 0; i < MS; i++) {
+                if (src.mode == 3) r2[i] = r2[i] + pamp * zpl[a + i];
+                wl[c * nzp + a + i] = (i == isrc) ? r2[i] + srcv : r2[i];
+            }
         }
     }
 
@@ -513,9 +523,10 @@ __global__ __launch_bounds__(384) void k_colsplit(Dims d, Bg bg, DbyCoef cf, Seg
 // enough columns to fill the chip twice.  Bound: registers (244 at MS = 6, two
 // waves per SIMD; MS = 8 spills a little, longer segments more than they gain)
 // and HBM, 128 B per point.  us per launch, lane groups -> here: 16 sources at
-// 256x300 67 -> 51 (3.1 TB/s), 8 sources 37 -> 29, 6 sources 36 -> 27; 4 sources
-// (307 000 points) 21 -> 24, 16 at 128x150 (307 000) 20 -> 23: the line between
-// the forms lies at 450 000 points.
+// 256x300 67 -> 51, 8 sources 37 -> 29, 6 sources 36 -> 27; 4 sources (307 000
+// points) 21 -> 24, 16 at 128x150 (307 000) 20 -> 23: the line between the forms
+// lies at 450 000 points.  With shared windows of end values 16 sources take 47
+// (3.3 TB/s) and 8 take 27, the lane groups' 16 at 128x150 19.
 constexpr size_t kOneLanePoints = 450000;
 constexpr int kCA = 9;      // epilogue inputs of a row pair
 struct PairIn {

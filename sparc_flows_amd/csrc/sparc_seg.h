@@ -124,22 +124,29 @@ SPARC_HD int seg_band_kinds(int P, int E) { return 2 * E + 1 < P ? 2 * E + 1 : P
 
 // seg_correct from the segment's own pair of rows: rows[0 .. nw), nw = 4 hw + 4,
 // gives L_{s-1} from the end values of segments s-1-hw .. s+hw, rows[nw .. 2 nw)
-// F_{s+1} from those of s+1-hw .. s+2+hw.
+// F_{s+1} from those of s+1-hw .. s+2+hw.  The two windows of end values are four
+// elements apart, so each is read once (six 16-byte LDS reads for eight products
+// of pairs; with a window each, eight: the reads bound this phase of the column
+// pass).  The end segments' window reaches two elements before and after the
+// column's buffer: the caller's LDS holds something there, and the sum it enters is
+// not used.
 template <int MS, int U = 2, typename Tab>
 SPARC_HD void seg_correct_rows(double (&Y)[MS], int s, int P, int hw, const double *yp, const double *rows, Tab tab)
 {
     const int nw = 4 * hw + 4;
-    const double *r1 = rows, *y1 = yp + 2 * (s > 0 ? s - 1 : 0);
-    const double *r2 = rows + nw, *y2 = yp + 2 * (s < P - 1 ? s + 1 : P - 1);
+    const double *r1 = rows, *r2 = rows + nw, *y = yp + 2 * (s - 1);
     double a0 = 0.0, a1 = 0.0, b0 = 0.0, b1 = 0.0;
+    Dbl2 uA = ld2(y), uB = ld2(y + 2);
 #pragma unroll U
     for (int w = 0; w < nw; w += 4) {
-        const Dbl2 pA = ld2(r1 + w), pB = ld2(r1 + w + 2), uA = ld2(y1 + w), uB = ld2(y1 + w + 2);
-        const Dbl2 qA = ld2(r2 + w), qB = ld2(r2 + w + 2), vA = ld2(y2 + w), vB = ld2(y2 + w + 2);
+        const Dbl2 pA = ld2(r1 + w), pB = ld2(r1 + w + 2), qA = ld2(r2 + w), qB = ld2(r2 + w + 2);
+        const Dbl2 vA = ld2(y + w + 4), vB = ld2(y + w + 6);
         a0 += pA.x * uA.x + pB.x * uB.x;
         a1 += pA.y * uA.y + pB.y * uB.y;
         b0 += qA.x * vA.x + qB.x * vB.x;
         b1 += qA.y * vA.y + qB.y * vB.y;
+        uA = vA;
+        uB = vB;
     }
     const double Lp = s > 0 ? a0 + a1 : 0.0;
     const double Fn = s < P - 1 ? b0 + b1 : 0.0;
