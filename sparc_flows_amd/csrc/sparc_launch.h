@@ -27,7 +27,7 @@ hipError_t launch_row(int mode, const Dims &d, const Bg &bg, const State &s, con
 // Segmented column pass, one lane per (column, segment, field); tc in
 // {1, 2, 4, 8, 16} columns per block, ms = rows per segment, one of
 // SPARC_COLSEG_SIZES (even: segments are whole row pairs).
-#define SPARC_COLSEG_SIZES(X) X(4) X(6) X(8) X(10) X(12) X(16) X(18) X(20) X(24)
+#define SPARC_COLSEG_SIZES(X) X(4) X(6) X(8) X(10) X(12) X(16) X(20) X(22) X(24)
 hipError_t colseg_init();
 // Whether the column pass runs its one-lane form (k_colone) on this batch.
 bool col_one_lane(const Dims &d, int ms);

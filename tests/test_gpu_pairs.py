@@ -59,3 +59,25 @@ def test_run_snapshots_and_state_round_trip(nx, nz, nsrc):
     assert torch.equal(s.state(), state)
     s.step(maxtime + 1)
     assert torch.equal(s.state(), a)
+
+
+@pytest.mark.parametrize("nz", [121, 482, 721, 722, 758, 841, 1024])
+@pytest.mark.parametrize("nsrc", [1, 24])
+def test_depths_that_only_long_segments_cut(nz, nsrc):
+    """Depths whose last segment would hold fewer than three rows at every length up
+    to 12 (at 721 and 722: at every length but 22), and the deepest: 6 steps of one
+    source and of a batch against the oracle, 1e-11."""
+    p, bg, c2d, psi = small_case(nx=32, nz=nz, npml=10, nph=4)
+    xs = list(np.linspace(-12.0, 12.0, nsrc))
+    s = Sparc(p, bg, nsrc=nsrc, c2d=c2d, psi=psi)
+    s.set_forward_sources(xs, 30)
+    s.reset()
+    for t in range(6):
+        s.step(t)
+    state = s.state().cpu().numpy()
+    for b in {0, nsrc - 1}:
+        o = oracle.Oracle(p, bg, c2d=c2d, psi=psi)
+        o.set_forward_source(xs[b], 30)
+        for t in range(6):
+            o.step(t)
+        assert rel_l2(state[:, b], o.state()) < 1e-11, (s.query("colseg_ms"), s.query("colseg_tc"))
