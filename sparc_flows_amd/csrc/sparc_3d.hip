@@ -264,31 +264,43 @@ __global__ __launch_bounds__(256) void k3_zv(Z3 z)
 
 // FILTER_VARS_3D_HORIZ_PML (physics.f90:855-878) on the six fields, rows
 // npmlbot+1 .. nz-npmltop, in place from a register window of the unfiltered
-// column.
+// column: rows j0-5 .. j0+U+4 of a chunk, the next chunk's U rows in flight
+// meanwhile (they lie above every row the chunk stores).  Bound: HBM at 256x256
+// columns, latency below, where one row in flight per lane left the chip waiting.
+// us per launch, one row in flight -> 8: 128x128x150 76 -> 43, 96x90x100 30 -> 16,
+// 64x64x80 26 -> 13; 256x256x300 322 -> 336 (5.6 TB/s; 16 rows the same, 4 rows 335
+// and 49 at 128x128x150).
 __global__ __launch_bounds__(256) void k3_filter(double *a, int nxy, int nz, int nb, int nt)
 {
+    constexpr int U = 8;
     const long id = (long)blockIdx.x * 256 + threadIdx.x;
     if (id >= 6L * nxy) return;
     const int f = (int)(id / nxy), c = (int)(id - (long)f * nxy);
     const size_t s = (size_t)nxy;
     double *A = a + (size_t)f * nz * s + c;
-    double w[11];                       // w[k] = a(j - 5 + k) at filtered row j
+    auto row = [&](int j) { const double v = A[(size_t)min(j, nz - 1) * s]; return j < nz ? v : 0.0; };
+    double w[U + 10];                   // w[k] = a(j0 - 5 + k)
 #pragma unroll
-    for (int k = 0; k < 11; k++) w[k] = A[(size_t)(nb - 5 + k) * s];
+    for (int k = 0; k < U + 10; k++) w[k] = row(nb - 5 + k);
     const double c0 = 0.75390625, c1 = 0.41015625, c2 = -0.234375, c3 = 0.087890625,
                  c4 = -0.01953125, c5 = 0.001953125;
-    for (int j = nb; j < nz - nt; j++) {
-        double v = c0 * w[5] + 0.5 * c1 * (w[4] + w[6]);
-        v = v + 0.5 * c2 * (w[3] + w[7]);
-        v = v + 0.5 * c3 * (w[2] + w[8]);
-        v = v + 0.5 * c4 * (w[1] + w[9]);
-        v = v + 0.5 * c5 * (w[0] + w[10]);
-        const int jn = j + 6;
-        const double un = jn < nz ? A[(size_t)jn * s] : 0.0;
-        A[(size_t)j * s] = v;
+    for (int j0 = nb; j0 < nz - nt; j0 += U) {
+        double un[U];
 #pragma unroll
-        for (int k = 0; k < 10; k++) w[k] = w[k + 1];
-        w[10] = un;
+        for (int u = 0; u < U; u++) un[u] = row(j0 + U + 5 + u);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            double v = c0 * w[u + 5] + 0.5 * c1 * (w[u + 4] + w[u + 6]);
+            v = v + 0.5 * c2 * (w[u + 3] + w[u + 7]);
+            v = v + 0.5 * c3 * (w[u + 2] + w[u + 8]);
+            v = v + 0.5 * c4 * (w[u + 1] + w[u + 9]);
+            v = v + 0.5 * c5 * (w[u] + w[u + 10]);
+            if (j0 + u < nz - nt) A[(size_t)(j0 + u) * s] = v;
+        }
+#pragma unroll
+        for (int k = 0; k < 10; k++) w[k] = w[k + U];
+#pragma unroll
+        for (int u = 0; u < U; u++) w[10 + u] = un[u];
     }
 }
 
