@@ -22,12 +22,12 @@
 //     forward stage (k_fwd_b, k_fwd_c) and of its transpose (k_adj_a,
 //     k_adj_b, k_adj_c), the z filter and its transpose.
 // The forward stages here are unfused and recomputed from the trajectory; they
-// agree with the fused solver to rounding.  Bound: HBM and the launches (7 to 16 us
+// agree with the fused solver to rounding.  Bound: HBM and the launches (6 to 29 us
 // each).  A forward stage is six launches and a transposed one seven: the pointwise
 // kernels write the next stage's input or the accumulated adjoint themselves, and
 // derivatives of different fields share a launch.  With a pass of its own for every
 // update and accumulation a step of 8 sources at 256 x 300 took 415 us forward and
-// 620 transposed; here 310 and 500.
+// 620 transposed; here 317 and 455.
 #include <algorithm>
 #include <utility>
 
