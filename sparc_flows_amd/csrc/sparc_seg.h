@@ -1,11 +1,12 @@
 // sparc_seg.h -- the segmented (SPIKE) form of dbyd2 (dbyd2.f:8-200,
-// mtridag.f:95-112) that the column pass runs, one segment per lane: the
-// segment's right-hand side, its local Thomas solve and the interface
+// mtridag.f:95-112) that the column pass and the z kernels run, one segment per
+// lane: the segment's right-hand side, its local Thomas solve and the interface
 // correction, plus the host construction of their tables.
 //
-// The three templates are the kernel's own code (k_colsplit includes this
-// header); the same source also compiles as host C++, so that the algorithm
-// is checked on the CPU against the oracle's dbyd2 for every segment length.
+// The templates are the kernels' own code: k_colsplit and k_colone correct with
+// seg_correct_rows, the kernels of sparc_zseg.hip with seg_correct.  The same source
+// also compiles as host C++, so that both are checked on the CPU against the oracle's
+// dbyd2 (tests/seg_rows_emul.cpp) for every segment length.
 #pragma once
 
 #include <vector>
@@ -169,7 +170,9 @@ void dbyd2_coefs(int N2, double &c1, double &c2, double cb[kCB]);
 void dbyd2_matrix(int N2, int ibc, std::vector<double> &lowr, std::vector<double> &uppr);
 
 // Tables of the segmented solve for nz rows cut into segments of m rows
-// (P = ceil(nz/m), nzp = P*m, the last segment padded with identity rows).
+// (P = ceil(nz/m), nzp = P*m, the last segment padded with identity rows), with
+// every interface row: the form that the rows by kind below are compared with on the
+// CPU; no kernel reads it.
 // slots: [3][5][nzp], for ibc 1, 2, 3: lowr, rbl, gl (Thomas factors restarted
 // at each segment start), V, W (the spikes: the segment's response to the row
 // above and below it).  band: [3][2P][4hw+4], rows of the exact inverse of the
@@ -215,7 +218,9 @@ constexpr int kZSegP = 32;
 constexpr int kZSegMax3 = 16;
 // The shortest of them that cuts nz rows into at most kZSegP segments (half as
 // many up to nz = 160, where blocks of twice the columns then fit) whose last
-// holds at least 3 real rows; 0 if there is none (nz > 1024).
+// holds at least 3 real rows; 0 if there is none: nz > 1024, and 673, 674, 897, 898,
+// 929, 930, 961, 962, 993 and 994.  Lengths above kZSegMax3 leave the 3D passes to the
+// one-lane sweeps: nz > 512, and 337, 338, 449, 450, 465, 466, 481, 482, 497 and 498.
 int zseg_length(int nz);
 // The device image of nset matrices, one after the other: the banded
 // interface inverse [2P][4hw+4], then the segment tables [5][3][m] by kind,

@@ -94,7 +94,8 @@ __device__ __forceinline__ int pml_index(int j, int nz, int nb, int nt)
 }
 
 // Whether the segmented passes take this grid: segments of at most kZSegMax3
-// rows (nz <= 512) and a field of less than 2^31 bytes (32-bit byte offsets).
+// rows (every nz up to 512 but the ten that zseg_length names) and a field of less
+// than 2^31 bytes (32-bit byte offsets).
 bool zseg3_fits(const Z3 &z, const ZSeg &sg);
 hipError_t launch_zp_seg(const Z3 &z, const ZSeg &sg, hipStream_t st);
 hipError_t launch_zv_seg(const Z3 &z, const ZSeg &sg, hipStream_t st);
