@@ -468,8 +468,7 @@ def main():
         # times the single-source bytes, more than the 256 MB MALL holds
         bms = bpipe.fwd.profile_kernels(200)
         bach = bytes_per_pt["col"] * npts * args.batch / (bms["col"] * 1e-3) / 1e9
-        # the form a batch of this size takes (csrc/sparc_colseg.hip, col_one_lane)
-        bform = "k_colone" if bpipe.fwd.query("colseg_ms") <= 8 and npts * args.batch >= 450000 else "k_colsplit"
+        bform = "k_colone" if bpipe.fwd.query("colseg_one") else "k_colsplit"
         btraffic = measured_traffic(bform, bpipe.fwd.query("colseg_ms"), bpipe.fwd.query("colseg_p"),
                                     bpipe.fwd.query("colseg_tc"), args.batch)
         batched = {"sources": args.batch, "s_per_gradient": bsec, "finite": bfinite,

@@ -70,7 +70,8 @@ const char *sparc_last_error(const sparc_handle *h);
 int sparc_set_stream(sparc_handle *h, void *hip_stream);
 /* Integer / double facts of the handle: "e_rad", "o_rad", "steps",
  * "cadforcing_step", "forcing_length", "nsrc", "nx", "nz", "nzpml", "nph",
- * "colseg_tc", "colseg_ms", "colseg_p", "colseg_hw" (column-pass launch shape) / "deltat",
+ * "colseg_tc", "colseg_ms", "colseg_p", "colseg_hw" (column-pass launch shape),
+ * "colseg_one" (1: one lane per segment for all fields) / "deltat",
  * "stretchx", "delta_width", "beta2".."beta5". */
 int sparc_query_int(const sparc_handle *h, const char *name, int *value);
 int sparc_query_double(const sparc_handle *h, const char *name, double *value);

@@ -987,6 +987,7 @@ int sparc_query_int(const sparc_handle *h, const char *name, int *v)
     else if (n == "colseg_tc") *v = h->seg_tc;
     else if (n == "row_wide") *v = h->row_wide;
     else if (n == "colseg_ms") *v = h->seg_ms;
+    else if (n == "colseg_one") *v = col_one_lane(h->d, h->seg, h->seg_tc);
     else if (n == "colseg_p") *v = h->seg.P;
     else if (n == "colseg_hw") *v = h->seg.hw;
     else return SPARC_E_ARG;

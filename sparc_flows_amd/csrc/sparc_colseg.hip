@@ -14,6 +14,7 @@
 // segment's end values through LDS, and the exact correction
 // y - L_{s-1} V - F_{s+1} W.  Loads use clamped row indices and 32-bit byte
 // offsets from wave-uniform bases; stores of padding rows are masked off.
+#include <algorithm>
 #include <type_traits>
 
 #include "sparc_device.h"
@@ -527,7 +528,20 @@ __global__ __launch_bounds__(384) void k_colsplit(Dims d, Bg bg, DbyCoef cf, Seg
 // points) 21 -> 24, 16 at 128x150 (307 000) 20 -> 23: the line between the forms
 // lies at 450 000 points.  With shared windows of end values 16 sources take 47
 // (3.3 TB/s) and 8 take 27, the lane groups' 16 at 128x150 19.
+//
+// It also wants many blocks on a compute unit: a lane group's wave does about a third of
+// a one-lane wave's work, so where the tables' LDS, and not the registers, bounds the
+// blocks of a unit, the lane groups have three times the waves.  The form runs where a
+// unit holds at least three of its blocks for one of the lane groups', and above 128
+// lanes, where the lane groups do not fit.  us per launch at the best shape of each form,
+// lane groups / one lane: 64 sources of 100x100 47 / 63, 16 of 250x150 52 / 67, 8 of
+// 255x300 64 / 89, 100 of 256x60 74 / 78, 400 of 300x60 551 / 604; 8 of 1000x100 52 / 45,
+// 60 of 150x60 86 / 68, 1000 of 17x40 214 / 160, 16 of 256x300 70 / 50.  Over 48 grids the
+// best shape under this rule is 0.1 % (at most 1.9 %) behind the best of both forms; lines
+// at 2 or 4 in place of 3 cost up to 10 % and 26 %.
 constexpr size_t kOneLanePoints = 450000;
+constexpr int kOneLaneBlocks = 3;
+constexpr int kWavesPerUnit = 8;   // both forms: two waves per SIMD by registers
 constexpr int kCA = 9;      // epilogue inputs of a row pair
 struct PairIn {
     dpair v[kCA];           // d xi_x/dx, c^2 rho0, d v_z/dx, d v_x/dx, v0x, v0z, xi_z base, xi_z, v_z
@@ -823,12 +837,6 @@ __global__ __launch_bounds__(512) void k_colone(Dims d, Bg bg, DbyCoef cf, SegTa
 // Segment lengths of the one-lane form: longer ones do not fit its registers.
 #define SPARC_COLONE_SIZES(X) X(4) X(6) X(8)
 
-// The form that a batch takes.
-bool col_one_lane(const Dims &d, int ms)
-{
-    return ms <= 8 && (size_t)d.S * d.nx * d.nz >= kOneLanePoints;
-}
-
 inline size_t colone_lds_bytes(int tc, const SegTab &sg)
 {
     const size_t img = ((size_t)3 * sg.nk * 2 * (4 * sg.hw + 4) + (size_t)kZS * 3 * sg.m + (size_t)kZF * sg.nzp + kCB + 1) &
@@ -838,6 +846,21 @@ inline size_t colone_lds_bytes(int tc, const SegTab &sg)
 
 namespace {
 int g_lds_max = 64 * 1024;   // dynamic LDS a block may use on this device
+// Blocks of so many waves and bytes of LDS that a compute unit holds.
+int resident(int waves, size_t lds)
+{
+    return std::min((int)((size_t)g_lds_max / lds), kWavesPerUnit / waves);
+}
+}  // namespace
+
+// The form that a batch takes with blocks of tc columns.
+bool col_one_lane(const Dims &d, const SegTab &sg, int tc)
+{
+    if (sg.m > 8 || (size_t)d.S * d.nx * d.nz < kOneLanePoints) return false;
+    const int waves = (tc * sg.P + 63) / 64;
+    if (waves > 2) return true;                      // more than the lane groups' 128 lanes
+    return resident(waves, colone_lds_bytes(tc, sg)) >=
+           kOneLaneBlocks * resident(3 * waves, colsplit_lds_bytes(tc, sg, d.nzpml));
 }
 
 // Raises every instantiation's dynamic-LDS limit to the device's maximum per
@@ -878,7 +901,7 @@ namespace sparc {
 
 bool colsplit_fits(int tc, const Dims &d, const SegTab &sg)
 {
-    if (col_one_lane(d, sg.m))
+    if (col_one_lane(d, sg, tc))
         return d.nx % tc == 0 && tc * sg.P <= 512 && colone_lds_bytes(tc, sg) <= (size_t)g_lds_max;
     return d.nx % tc == 0 && (tc * sg.P + 63) / 64 <= 2 &&
            colsplit_lds_bytes(tc, sg, d.nzpml) <= (size_t)g_lds_max;
@@ -890,7 +913,7 @@ hipError_t launch_colsplit(int tc, int ms, const Dims &d, const Bg &bg, const Db
 {
     if ((tc != 1 && tc != 2 && tc != 4 && tc != 8 && tc != 16) || d.nx % tc || sg.m != ms || sg.P > kSegMax)
         return hipErrorInvalidValue;
-    if (col_one_lane(d, ms)) {
+    if (col_one_lane(d, sg, tc)) {
         const size_t shm = colone_lds_bytes(tc, sg);
         if (tc * sg.P > 512 || shm > (size_t)g_lds_max) return hipErrorInvalidValue;
         const dim3 grid(d.nx / tc, d.S), block((tc * sg.P + 63) / 64 * 64);

@@ -29,10 +29,12 @@ hipError_t launch_row(int mode, const Dims &d, const Bg &bg, const State &s, con
 // SPARC_COLSEG_SIZES (even: segments are whole row pairs).
 #define SPARC_COLSEG_SIZES(X) X(4) X(6) X(8) X(10) X(12) X(16) X(20) X(22) X(24)
 hipError_t colseg_init();
-// Whether the column pass runs its one-lane form (k_colone) on this batch.
-bool col_one_lane(const Dims &d, int ms);
+// Whether the column pass runs its one-lane form (k_colone) on this batch with blocks
+// of tc columns.
+bool col_one_lane(const Dims &d, const SegTab &sg, int tc);
 // Whether a column-pass block of tc columns fits: its threads (one lane per
-// column and segment, at most 512, or 3 lane groups of at most 128) and its dynamic LDS (after colseg_init, the device maximum).
+// column and segment, at most 512, or 3 lane groups of at most 128) and its dynamic
+// LDS (after colseg_init, the device maximum).
 bool colsplit_fits(int tc, const Dims &d, const SegTab &sg);
 hipError_t launch_colsplit(int tc, int ms, const Dims &d, const Bg &bg, const DbyCoef &cf, const SegTab &sg,
                            const State &s, const ColArgs &ca, const Src &src, const Clock &c, const Sink &sk,
