@@ -96,47 +96,47 @@ __device__ __forceinline__ void circ_sum(double (&ar)[kCircR], double (&ai)[kCir
     }
 }
 
-// One line per block of 256 lanes (the row pass): lane t holds z[t + 256 j2],
-// j2 < N2, 256 N2 >= n; slots past n carry nothing and get garbage.  With
-// one line per block the m range is split as well, over as many groups of
-// lanes as fit (at most 4), and their sums are added through LDS.
-template <int N2> struct CircLds {
-    static constexpr int raw = 256 * N2;
+// One line per block of B lanes (the row pass): lane t holds z[t + B j2], j2 < N2,
+// B N2 >= n; slots past n carry nothing and get garbage.  With one line per block
+// the m range is split as well, over as many groups of lanes as fit (at most 4), and
+// their sums are added through LDS.
+template <int B, int N2> struct CircLds {
+    static constexpr int raw = B * N2;
     // doubled lines (even: 2 (n + 15), odd: 2 n + 15), or the partial sums
-    // (splits n, at most 1280 elements: splits <= 256 / ceil(n / 5))
-    static constexpr int work = 512 * N2 + 30 > 1280 ? 512 * N2 + 30 : 1280;
+    // (splits n, at most 5 B elements: splits <= B / ceil(n / 5))
+    static constexpr int work = 2 * B * N2 + 30 > 5 * B ? 2 * B * N2 + 30 : 5 * B;
     static constexpr int n = raw + work;
-    static constexpr int c = 256 * N2 + 20;      // the table
+    static constexpr int c = B * N2 + 20;        // the table
 };
 
-// z: CircLds<N2>::n elements; cc: the table.  Every lane of the block must call this
-// (it contains block barriers).
-template <int N2>
+// z: CircLds<B, N2>::n elements; cc: the table.  Every lane of the block must call
+// this (it contains block barriers).
+template <int B, int N2>
 __device__ __forceinline__ void circ_deriv_block(double (&re)[N2], double (&im)[N2], int t, double2 *z,
                                                  const double *cc, int n, double stretch)
 {
     const CircShape s = circ_shape(n);
-    double2 *const work = z + CircLds<N2>::raw;
+    double2 *const work = z + CircLds<B, N2>::raw;
 #pragma unroll
     for (int j2 = 0; j2 < N2; j2++) {
-        const int x = t + 256 * j2;
+        const int x = t + B * j2;
         if (x < n) z[x] = make_double2(re[j2], im[j2]);
     }
     __syncthreads();
-    for (int q = t; q < kCircK * s.nk; q += 256) work[q < kCircK ? q : s.ext + q - kCircK] = make_double2(0.0, 0.0);
-    for (int j = t; j < s.len; j += 256) {
+    for (int q = t; q < kCircK * s.nk; q += B) work[q < kCircK ? q : s.ext + q - kCircK] = make_double2(0.0, 0.0);
+    for (int j = t; j < s.len; j += B) {
         const double2 a = z[j];
         if (s.nk == 1) {
             circ_put(work, s.len, 0, j, a);
         } else {
-            const double2 b = z[j + s.len];
-            circ_put(work, s.len, 0, j, make_double2(a.x + b.x, a.y + b.y));
-            circ_put(work + s.ext, s.len, 1, j, make_double2(a.x - b.x, a.y - b.y));
+            const double2 o = z[j + s.len];
+            circ_put(work, s.len, 0, j, make_double2(a.x + o.x, a.y + o.y));
+            circ_put(work + s.ext, s.len, 1, j, make_double2(a.x - o.x, a.y - o.y));
         }
     }
     __syncthreads();
     // group of lanes g = split, then product, then output block
-    const int ns = min(4, 256 / s.lanes), chunks = s.plen / kCircK;
+    const int ns = min(4, B / s.lanes), chunks = s.plen / kCircK;
     const int g = t / s.lanes, l = t - g * s.lanes, kind = l >= s.L ? 1 : 0, x0 = kCircR * (l - kind * s.L);
     double ar[kCircR], ai[kCircR];
 #pragma unroll
@@ -153,7 +153,7 @@ __device__ __forceinline__ void circ_deriv_block(double (&re)[N2], double (&im)[
     __syncthreads();
 #pragma unroll
     for (int j2 = 0; j2 < N2; j2++) {
-        const int x = t + 256 * j2;
+        const int x = t + B * j2;
         if (x < n) {
             const int hi = s.nk == 2 && x >= s.len, j = hi ? x - s.len : x;
             double pr = 0.0, pi = 0.0, qr = 0.0, qi = 0.0;

@@ -534,11 +534,10 @@ __device__ __forceinline__ void fft_deriv_team_256x64(double (&re)[4], double (&
 template <int N1, int N2> struct FftLds { static constexpr int n = N2 * (N1 + 1); };
 template <> struct FftLds<32, 8> { static constexpr int n = 2 * 8 * 33; };
 template <> struct FftLds<64, 4> { static constexpr int n = 2 * 264; };
-template <int N2> struct FftLds<256, N2> { static constexpr int n = CircLds<N2>::n; };   // any-nx form
 
 // Factorization N1 x N2 of the power-of-two row lengths (N1 >= N2).  Any
 // other nx runs the circulant form (sparc_circ.h), a kernel template argument
-// NX = -N2: rows of at most 256 N2 on 256 lanes.
+// NX = -N2: rows of at most N1 N2 points on N1 lanes, N1 = 64 or 256.
 template <int NX> struct FftShape;
 template <> struct FftShape<16> { static constexpr int N1 = 4, N2 = 4; };
 template <> struct FftShape<32> { static constexpr int N1 = 8, N2 = 4; };

@@ -15,6 +15,8 @@
 //
 // A step is R1 C1 R(1|2) C2 R(2|3) C3 R(3|4) C4 R(4|5) C5 R5; the v_x filter of
 // the previous step is applied on the fly by the next R1 (or by k_finalize_vx).
+#include <type_traits>
+
 #include "sparc_device.h"
 #include "sparc_launch.h"
 
@@ -75,7 +77,7 @@ __global__ __launch_bounds__(64) void k_ddz_cols(const double *in, double *out,
 #define SPARC_FFT_DERIV(RE, IM, T, LDS, TW, DM, SX)                                            \
     do {                                                                                       \
         if constexpr (kAny)                                                                    \
-            circ_deriv_block<N2>(RE, IM, T, LDS, sdm, nxr, SX);                                 \
+            circ_deriv_block<N1, N2>(RE, IM, T, LDS, sdm, nxr, SX);                             \
         else if constexpr (N1 == 32 && N2 == 8)                                                \
             fft_deriv_team_256x32(RE, IM, T, LDS, (LDS) + 8 * 33, TW, DM, SX);                 \
         else if constexpr (N1 == 64 && N2 == 4)                                                \
@@ -276,24 +278,24 @@ __global__ __launch_bounds__(256) void k_circ(RowSets rs, long count, int nx, Ci
 // four radix-4 stages), which are faster when the pass is latency-bound (one
 // source) and slower when it is bandwidth-bound.
 //
-// NX = -N2: the any-nx form, one row per block of 256 lanes, rows up to
-// 256 N2 (circ_deriv_block); lane slots past nx load column nx-1 and store
+// NX = -N2: the any-nx form, one row per block of N1 lanes (64 or 256), rows up to
+// N1 N2 (circ_deriv_block); lane slots past nx load column nx-1 and store
 // nothing.
 template <int NX, int MODE, int N1 = (NX < 0 ? 256 : FftShape<(NX < 0 ? 16 : NX)>::N1)>
-__global__ __launch_bounds__(NX < 0 ? 256 : 64, NX == 256 && N1 == 16 ? 2 : 1) void k_row(Dims d, Bg bg, State st, RowArgs ra, Clock clk, Sink sink)
+__global__ __launch_bounds__(NX < 0 ? N1 : 64, NX == 256 && N1 == 16 ? 2 : 1) void k_row(Dims d, Bg bg, State st, RowArgs ra, Clock clk, Sink sink)
 {
     constexpr bool kAny = NX < 0;
-    static_assert(!kAny || N1 == 256, "the any-nx form runs one row on 256 lanes");
+    static_assert(!kAny || N1 == 64 || N1 == 256, "the any-nx form runs one row on 64 or 256 lanes");
     constexpr int N2 = kAny ? -NX : NX / N1, TEAMS = kAny ? 1 : 64 / N1;
     const int nxr = kAny ? d.nx : NX;
-    __shared__ double2 lds[TEAMS][FftLds<N1, N2>::n];
+    __shared__ double2 lds[TEAMS][std::conditional_t<kAny, CircLds<N1, N2>, FftLds<N1, N2>>::n];
     // twiddles and bin multipliers (any nx: the circulant column) staged in
     // LDS: their reads then never wait behind this pass's global stores
     __shared__ double2 stw[kAny ? 1 : NX];
-    __shared__ double sdm[kAny ? CircLds<kAny ? N2 : 1>::c : NX];
+    __shared__ double sdm[kAny ? CircLds<N1, N2>::c : NX];
     if constexpr (kAny) {
         const CircShape s = circ_shape(nxr);
-        for (int q = threadIdx.x; q < s.nk * s.plen; q += 256) sdm[q] = bg.cdx[q];
+        for (int q = threadIdx.x; q < s.nk * s.plen; q += N1) sdm[q] = bg.cdx[q];
     } else {
         constexpr int NQ = (NX + 63) / 64;
         double2 tv[NQ];
@@ -781,6 +783,16 @@ hipError_t launch_ddy_any(const double *in, double *out, int nplanes, int nx, in
     return hipGetLastError();
 }
 
+// Lanes per row of the any-nx form.  256 lanes split the sum of a short row four ways,
+// which is faster while every row has a compute unit's SIMDs to itself; with more than
+// four rows a unit most of those lanes only hold back other rows, and rows of up to 128
+// points take one wave each.  us per launch (stage pass) on 256 / 64 lanes: nx = 48, 600
+// rows 9.0 / 9.0, 1440 13.8 / 10.2, 24 000 133 / 50; nx = 121, 960 14.8 / 16.9, 1440
+// 20.7 / 17.9, 24 000 216 / 135.  Longer odd rows want the split for longer: nx = 191,
+// 1440 27.8 / 31.6, 2400 40 / 42; nx = 255, 2400 52 / 53.
+constexpr int kShortRow = 128, kManyRows = 4 * 256;
+static int any_row_lanes(const Dims &d) { return d.nx <= kShortRow && (long)d.S * d.nz > kManyRows ? 64 : 256; }
+
 hipError_t launch_row(int mode, const Dims &d, const Bg &bg, const State &s, const RowArgs &ra,
                       const Clock &c, const Sink &sk, hipStream_t st, int wide)
 {
@@ -800,16 +812,17 @@ hipError_t launch_row(int mode, const Dims &d, const Bg &bg, const State &s, con
     }
     if (!nx_has_fft(d.nx)) {
         if (d.nx < 16 || d.nx > 1024) return hipErrorInvalidValue;
-        // any nx: one row per 256-lane block
+        // any nx: one row per block
         dim3 grid(d.S * d.nz);
-#define A(N2V)                                                                                   \
-        case N2V:                                                                                \
-            if (mode == 0) hipLaunchKernelGGL((k_row<-N2V, 0, 256>), grid, dim3(256), 0, st, d, bg, s, ra, c, sk); \
-            else if (mode == 1) hipLaunchKernelGGL((k_row<-N2V, 1, 256>), grid, dim3(256), 0, st, d, bg, s, ra, c, sk); \
-            else hipLaunchKernelGGL((k_row<-N2V, 2, 256>), grid, dim3(256), 0, st, d, bg, s, ra, c, sk); \
+#define A(N1V, N2V)                                                                              \
+        case N1V * 16 + N2V:                                                                     \
+            if (mode == 0) hipLaunchKernelGGL((k_row<-N2V, 0, N1V>), grid, dim3(N1V), 0, st, d, bg, s, ra, c, sk); \
+            else if (mode == 1) hipLaunchKernelGGL((k_row<-N2V, 1, N1V>), grid, dim3(N1V), 0, st, d, bg, s, ra, c, sk); \
+            else hipLaunchKernelGGL((k_row<-N2V, 2, N1V>), grid, dim3(N1V), 0, st, d, bg, s, ra, c, sk); \
             break;
-        switch ((d.nx + 255) / 256) {
-            A(1) A(2) A(3) A(4)
+        const int lanes = any_row_lanes(d);
+        switch (lanes * 16 + (d.nx + lanes - 1) / lanes) {
+            A(64, 1) A(64, 2) A(256, 1) A(256, 2) A(256, 3) A(256, 4)
         default: return hipErrorInvalidValue;
         }
 #undef A
