@@ -135,18 +135,19 @@ __global__ __launch_bounds__(64) void k_ddx_rows(RowSets rs, const double2 *__re
 //   AXIS 0: count rows of length n; a team takes rows 2 g, 2 g + 1.
 //   AXIS 1: count column pairs (x0, x0 + 1) of [n][nx] planes (of the first array),
 //           nx even, so every pair is 16-byte aligned.
+// SPLIT: ns groups of lanes a pair share its sum (circ_batch).
 // Both directions of global access run with the fastest index over the lanes;
 // the doubled lines and then the results wait in LDS.
-template <int AXIS>
-__global__ __launch_bounds__(256) void k_circ(RowSets rs, long count, int nx, CircShape s, int G,
+template <int AXIS, bool SPLIT>
+__global__ __launch_bounds__(256) void k_circ(RowSets rs, long count, int nx, CircShape s, int G, int ns,
                                               const double *__restrict__ cd, double stretch)
 {
     extern __shared__ double2 circ_lds[];
     constexpr int U = 4;                     // elements per lane whose loads are issued together
     const int t = threadIdx.x;
-    double2 *const E = circ_lds;             // [G][nk][ext]
-    double *const cc = (double *)(E + (size_t)G * s.nk * s.ext);
+    double2 *const E = circ_lds;             // [G][nk][ext]; the sums later, [ns][G][nk][ext]
     const int per = s.nk * s.ext;
+    double *const cc = (double *)(E + (size_t)(SPLIT ? ns : 1) * G * per);
     const long b0 = (long)xcd_block(blockIdx.x, gridDim.x) * G;     // first pair of the block
     for (int q = t; q < s.nk * s.plen; q += 256) cc[q] = cd[q];
     for (int q = t; q < G * s.nk * kCircK; q += 256) {
@@ -232,19 +233,37 @@ __global__ __launch_bounds__(256) void k_circ(RowSets rs, long count, int nx, Ci
         });
     }
     __syncthreads();
-    const int g = t / s.lanes, l = t - g * s.lanes, kind = l >= s.L ? 1 : 0, x0 = kCircR * (l - kind * s.L);
+    // group of lanes gp = split, then pair
+    const int gp = t / s.lanes, l = t - gp * s.lanes, kind = l >= s.L ? 1 : 0, x0 = kCircR * (l - kind * s.L);
+    const int sp = SPLIT ? gp / G : 0, g = gp - sp * G;
+    const bool on = SPLIT ? sp < ns : g < G;
     double ar[kCircR], ai[kCircR];
 #pragma unroll
     for (int r = 0; r < kCircR; r++) ar[r] = ai[r] = 0.0;
-    if (g < G)
-        circ_sum(ar, ai, E + g * per + kind * s.ext + kCircK + s.len + x0, cc + kind * s.plen, 0, s.plen);
-    __syncthreads();
-    if (g < G) {
-#pragma unroll
-        for (int r = 0; r < kCircR; r++)
-            if (x0 + r < s.len) E[g * per + kind * s.ext + x0 + r] = make_double2(ar[r] * stretch, ai[r] * stretch);
+    if (on) {
+        const int chunks = s.plen / kCircK;
+        circ_sum(ar, ai, E + g * per + kind * s.ext + kCircK + s.len + x0, cc + kind * s.plen,
+                 SPLIT ? kCircK * (sp * chunks / ns) : 0, SPLIT ? kCircK * ((sp + 1) * chunks / ns) : s.plen);
     }
     __syncthreads();
+    if (on) {
+#pragma unroll
+        for (int r = 0; r < kCircR; r++)
+            if (x0 + r < s.len) E[gp * per + kind * s.ext + x0 + r] = make_double2(ar[r] * stretch, ai[r] * stretch);
+    }
+    __syncthreads();
+    if constexpr (SPLIT) {                    // the splits' sums into the first's
+        for (int q = t; q < G * per; q += 256) {
+            double2 v = E[q];
+            for (int k = 1; k < ns; k++) {
+                const double2 w = E[k * G * per + q];
+                v.x += w.x;
+                v.y += w.y;
+            }
+            E[q] = v;
+        }
+        __syncthreads();
+    }
     each([&](const int (&fs)[U], const int (&os)[U]) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
@@ -756,9 +775,10 @@ hipError_t launch_ddx_rows2(const double *in, double *out, int nrows, const doub
     const int npairs = (nrows + nrows2 + 1) / 2;
     if (!nx_has_fft(nx)) {
         if (nx < 16 || nx > 1024) return hipErrorInvalidValue;
-        const CircBatch c = circ_batch(nx, 0);
-        hipLaunchKernelGGL((k_circ<0>), dim3((npairs + c.G - 1) / c.G), dim3(256), c.lds, st, rs, (long)(nrows + nrows2),
-                           nx, c.s, c.G, cdx, stretchx);
+        const CircBatch c = circ_batch(nx, 0, npairs);
+        auto *const k = c.ns > 1 ? &k_circ<0, true> : &k_circ<0, false>;
+        hipLaunchKernelGGL(k, dim3((npairs + c.G - 1) / c.G), dim3(256), c.lds, st, rs, (long)(nrows + nrows2), nx, c.s,
+                           c.G, c.ns, cdx, stretchx);
         return hipGetLastError();
     }
 #define L(NXV)                                                                              \
@@ -776,10 +796,11 @@ hipError_t launch_ddy_any(const double *in, double *out, int nplanes, int nx, in
                           double stretch, hipStream_t st)
 {
     if (ny < 16 || ny > 1024 || (nx & 1)) return hipErrorInvalidValue;
-    const CircBatch c = circ_batch(ny, 1);
     const long pairs = (long)nplanes * (nx / 2);
-    hipLaunchKernelGGL((k_circ<1>), dim3((unsigned)((pairs + c.G - 1) / c.G)), dim3(256), c.lds, st,
-                       RowSets{in, nullptr, out, nullptr, 0, 0}, pairs, nx, c.s, c.G, cdy, stretch);
+    const CircBatch c = circ_batch(ny, 1, pairs);
+    auto *const k = c.ns > 1 ? &k_circ<1, true> : &k_circ<1, false>;
+    hipLaunchKernelGGL(k, dim3((unsigned)((pairs + c.G - 1) / c.G)), dim3(256), c.lds, st,
+                       RowSets{in, nullptr, out, nullptr, 0, 0}, pairs, nx, c.s, c.G, c.ns, cdy, stretch);
     return hipGetLastError();
 }
 
