@@ -265,14 +265,11 @@ __global__ __launch_bounds__(256) void k3_zv(Z3 z)
 // FILTER_VARS_3D_HORIZ_PML (physics.f90:855-878) on the six fields, rows
 // npmlbot+1 .. nz-npmltop, in place from a register window of the unfiltered
 // column: rows j0-5 .. j0+U+4 of a chunk, the next chunk's U rows in flight
-// meanwhile (they lie above every row the chunk stores).  Bound: HBM at 256x256
-// columns, latency below, where one row in flight per lane left the chip waiting.
-// us per launch, one row in flight -> 8: 128x128x150 76 -> 43, 96x90x100 30 -> 16,
-// 64x64x80 26 -> 13; 256x256x300 322 -> 336 (5.6 TB/s; 16 rows the same, 4 rows 335
-// and 49 at 128x128x150).
+// meanwhile (they lie above every row the chunk stores).  Bound: HBM where the
+// columns fill the chip, latency where they do not (launch_filter).
+template <int U>
 __global__ __launch_bounds__(256) void k3_filter(double *a, int nxy, int nz, int nb, int nt)
 {
-    constexpr int U = 8;
     const long id = (long)blockIdx.x * 256 + threadIdx.x;
     if (id >= 6L * nxy) return;
     const int f = (int)(id / nxy), c = (int)(id - (long)f * nxy);
@@ -393,8 +390,19 @@ static hipError_t launch_zv(const Z3 &z, hipStream_t st)
 
 static hipError_t launch_filter(double *a, int nxy, int nz, int nb, int nt, hipStream_t st)
 {
-    const long n = 6L * nxy;
-    hipLaunchKernelGGL(k3_filter, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, nxy, nz, nb, nt);
+    // A chip of 256 compute units holds 2048 blocks of the one-row form.  While its last
+    // round of blocks is nearly full the pass is bound by HBM, which serves one row in
+    // flight per lane better than eight; a thinner round (the whole launch of a small grid,
+    // or the tail of a large one) waits for latency.  us per launch on one row / eight, by
+    // the last round's fill: 128x128x150 (0.19) 87 / 42, 384x256x200 (0.13) 385 / 323,
+    // 224x224x300 (0.57) 253 / 246, 240x240x200 (0.66) 185 / 190, 250x250x300 (0.72)
+    // 327 / 355, 256x256x300 (0.75) 319 / 333, 512x512x100 (1) 390 / 425; two or four
+    // rows lie between, or at the eight's.
+    constexpr long kRound = 2048;
+    const long blocks = (6L * nxy + 255) / 256, last = (blocks - 1) % kRound + 1;
+    const dim3 grid((unsigned)blocks);
+    if (3 * last >= 2 * kRound) hipLaunchKernelGGL(k3_filter<1>, grid, dim3(256), 0, st, a, nxy, nz, nb, nt);
+    else hipLaunchKernelGGL(k3_filter<8>, grid, dim3(256), 0, st, a, nxy, nz, nb, nt);
     return hipGetLastError();
 }
 
