@@ -559,19 +559,24 @@ hipError_t launch_zp_seg(const Z3 &z, const ZSeg &sg, hipStream_t st)
 
 hipError_t launch_zv_seg(const Z3 &z, const ZSeg &sg, hipStream_t st)
 {
-    // 32 columns (256 bytes of each row) while they fill the 256 compute units
-    // and 512 threads: 143 us against 183 with 16 at 128x128x150, 68 against 63
-    // at 96x90x100
-    const int nc = sg.P <= kZSegP / 2 && z.nxy >= 32 * 256 ? 32 : 16;
+    // 32 columns (256 bytes of each row) where they fill the 256 compute units and
+    // 512 threads, but not at four rows a segment, whose registers let a unit hold
+    // three blocks of 16 columns and one of 32.  us on 16 / 32 columns: 128x128x150
+    // 164 / 141, x100 149 / 106; 100x100x150 118 / 112, x100 77 / 74; 90x91x100 46 / 43;
+    // four rows (nz = 60): 64x64 25 / 34, 96x90 52 / 65, 128x112 64 / 68, 160x160 143 / 154,
+    // 192x192 205 / 204.  32 lose elsewhere where their last round of blocks is nearly
+    // empty or the grid is large: 96x90x100 (270 blocks) 64 / 68, 160x160x150 226 / 251,
+    // 256x256x150 527 / 542 (x100 427 / 389).
+    const int nc = sg.P <= kZSegP / 2 && sg.m > 4 && z.nxy >= 32 * 256 ? 32 : 16;
     const size_t shm = zv_lds(sg, nc);
     const dim3 grid((unsigned)((z.nxy + nc - 1) / nc)), block(lanes(nc, sg.P));
 #define L(M)                                                                                 \
     if (sg.m == M) {                                                                         \
-        const void *k = nc == 32 ? (const void *)k3_zv_seg<M, 32> : (const void *)k3_zv_seg<M, 16>; \
-        const hipError_t e = allow_lds(k, shm);                                              \
+        constexpr int W = M > 4 ? 32 : 16;                                                   \
+        auto *const k = nc == 32 ? &k3_zv_seg<M, W> : &k3_zv_seg<M, 16>;                     \
+        const hipError_t e = allow_lds((const void *)k, shm);                                \
         if (e != hipSuccess) return e;                                                       \
-        if (nc == 32) hipLaunchKernelGGL((k3_zv_seg<M, 32>), grid, block, shm, st, z, sg);   \
-        else hipLaunchKernelGGL((k3_zv_seg<M, 16>), grid, block, shm, st, z, sg);            \
+        hipLaunchKernelGGL(k, grid, block, shm, st, z, sg);                                  \
         return hipGetLastError();                                                            \
     }
     SPARC_ZSEG_SIZES(L)

@@ -16,6 +16,7 @@ import tests.test_gpu_zseg as zseg  # noqa: E402
 
 @pytest.mark.parametrize("nx,ny,nz,npml", [
     (16, 17, 78, 6), (18, 17, 108, 11), (16, 16, 128, 12), (16, 17, 121, 12), (18, 17, 241, 13), (96, 90, 301, 12),
-    (128, 128, 121, 12), (128, 130, 141, 12)])
+    (128, 128, 121, 12), (128, 130, 141, 12), (128, 66, 78, 6), (96, 90, 108, 11), (100, 96, 126, 12), (96, 90, 150, 13),
+    (96, 90, 62, 6)])
 def test_two_steps_match_oracle(nx, ny, nz, npml):
     zseg.test_two_steps_match_oracle(nx, ny, nz, npml)
