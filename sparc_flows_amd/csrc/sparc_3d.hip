@@ -832,7 +832,11 @@ static int setup3(sparc3d_handle *h)
     HCHECK3(h, m.alloc(&h->RG, N));
     HCHECK3(h, m.alloc(&h->DXP, N));
     HCHECK3(h, m.alloc(&h->DYP, N));
-    HCHECK3(h, m.alloc(&h->W, 4 * N));   // one block per chain of the Zv pass
+    // the one-lane sweeps' values: one block per chain of k3_zv, or, where the z passes
+    // run segmented, one for z-derivatives of more fields than a launch's grid holds
+    Z3 zfit{};
+    zfit.N = N;
+    HCHECK3(h, m.alloc(&h->W, zseg3_fits(zfit, h->zseg) ? N : 4 * N));
     HCHECK3(h, hipMemsetAsync(h->a, 0, 6 * N * sizeof(double), h->stream));
     HCHECK3(h, hipMemsetAsync(h->scr, 0, 6 * N * sizeof(double), h->stream));
     HCHECK3(h, hipMemsetAsync(h->pml, 0, 2 * h->np * sizeof(double), h->stream));

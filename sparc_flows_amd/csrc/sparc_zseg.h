@@ -54,7 +54,7 @@ namespace d3 {
 // Arguments of the two z passes of a 3D stage.
 struct Z3 {
     const double *B;            // Zp: xi_z; Zv: v_x (v_y, v_z follow at +N, +2N)
-    double *W;                  // one-lane sweeps: forward-sweep values, one [nz][nxy] block per chain
+    double *W;                  // one-lane sweeps only: forward-sweep values, one [nz][nxy] block per chain
     size_t N;                   // points per field
     int nxy, nz, nb, nt;
     const double *stretch;      // [nz]
