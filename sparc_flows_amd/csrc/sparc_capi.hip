@@ -220,7 +220,6 @@ hipError_t upload(DevArena &ar, double **dst, const std::vector<double> &v, hipS
     return hipMemcpyAsync(*dst, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice, st);
 }
 
-// GPU z-derivative of [nb][nz][ncols] host data (used by the set-up).
 hipError_t upload_zseg(DevArena &ar, ZSeg *out, int nz, int nset, hipStream_t st)
 {
     *out = ZSeg{};
@@ -239,6 +238,7 @@ hipError_t upload_zseg(DevArena &ar, ZSeg *out, int nz, int nset, hipStream_t st
     return hipSuccess;
 }
 
+// GPU z-derivative of [nb][nz][ncols] host data (used by the set-up).
 static int host_ddz(sparc_handle *h, const std::vector<double> &in, std::vector<double> &out,
                     int ncols, int nbatch, int ibc, bool use_stretch, int tri_ibc)
 {

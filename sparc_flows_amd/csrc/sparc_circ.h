@@ -53,14 +53,6 @@ __host__ __device__ inline CircShape circ_shape(int n)
     return s;
 }
 
-// The table of a line length: nk columns of plen (zeros past len).  At most
-// 1040 doubles.
-inline int circ_table_len(int n)
-{
-    const CircShape s = circ_shape(n);
-    return s.nk * s.plen;
-}
-
 // Element j of product kind k (0: u, or the line itself; 1: w) into both places of its
 // doubled line e = ext[k], whose index 0 is element -len - kCircK.
 __device__ __forceinline__ void circ_put(double2 *e, int len, int kind, int j, double2 v)

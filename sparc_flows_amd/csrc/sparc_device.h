@@ -38,7 +38,7 @@ struct Bg {
     const double *eyekx;                                   // [nx/2+1]
     const double *dmul;                                    // [nx] bin multiplier (see fft_deriv_team)
     const double2 *tw;                                     // [nx] exp(-2 pi i k/nx)
-    const double *cdx;                                     // circulant derivative columns, circ_table_len(nx) (an nx that is not a power of two)
+    const double *cdx;                                     // circulant derivative columns, nk of plen (CircShape; an nx that is not a power of two)
     double stretchx;
 };
 
