@@ -16,7 +16,7 @@
 //
 // Layout: fields [nz][ny][nx], x fastest.  The z passes run segmented
 // (sparc_zseg.hip) wherever zseg3_fits; the forms here are for the other
-// grids (nz above 512, a few nz that no cut fits, fields of 2^31 bytes and
+// grids (nz above 512, ten nz below that no cut fits, fields of 2^31 bytes and
 // more).  They give each lane one (x, y) column and stream it bottom to top and
 // back (the Thomas sweeps of dbyd2 / mtridag), so the 64 lanes of a wave touch
 // 64 consecutive doubles per row, with loads issued in chunks of rows (and four

@@ -8,8 +8,8 @@
 // FILTER_VARS_2D (physics2d.f90:509-556).
 //
 // Every column is split into P <= kSegMax segments of exactly MS rows; one
-// lane holds one segment of one field of one column, and a block covers TC
-// columns (k_colsplit below).  Each z-derivative is: dbyd2 right-hand side
+// lane holds one segment of one field of one column (k_colsplit), or of all three
+// (k_colone, batches), and a block covers TC columns.  Each z-derivative is: dbyd2 right-hand side
 // from a 7-row window, local Thomas solve of the segment, exchange of the
 // segment's end values through LDS, and the exact correction
 // y - L_{s-1} V - F_{s+1} W.  Loads use clamped row indices and 32-bit byte
@@ -38,8 +38,9 @@ enum PRow { P_AZ = 0, P_BZ, P_FZ, P_T0, P_B0, P_T1, P_B1, kPL };
 // values between 2hw and 2hw+2 zeros), and three [TC][nzp] row buffers: the
 // group-1 and group-0 parts of RHS v_z and p.
 // A set's interface rows repeat away from the column's ends, so keeping one
-// interior pair holds a block's LDS at 47 KB (TC = 4, MS = 10, nz = 300)
-// where all 2P rows took 104 KB, and its staging at 3 600 doubles for 7 300.
+// interior pair holds a block's LDS at 76 KB (TC = 4, MS = 10, nz = 300, 24 PML
+// rows) where all 2P rows took 104 KB, and the image that it stages at 3 846 doubles
+// for 7 302.
 inline size_t colsplit_staged(int tc, const SegTab &sg, int nzpml)
 {
     // rounded up to an even count, so that the end-value buffers after it
@@ -519,8 +520,8 @@ __global__ __launch_bounds__(384) void k_colsplit(Dims d, Bg bg, DbyCoef cf, Seg
 // three first derivatives one after the other, then the epilogue of a row pair
 // at a time (the next pair's nine inputs in flight meanwhile), d p/dz and the v_z
 // update.  Against the lane groups above it reads the flow once, stages the
-// tables for four times the columns per block and holds eight waves per compute
-// unit where those hold six; but a lane's chain is twice as long, so it wants
+// tables for twice the columns per block or more and holds seven or eight waves per
+// compute unit where those hold six; but a lane's chain is twice as long, so it wants
 // enough columns to fill the chip twice.  Bound: registers (244 at MS = 6, two
 // waves per SIMD; MS = 8 spills a little, longer segments more than they gain)
 // and HBM, 128 B per point.  us per launch, lane groups -> here: 16 sources at
@@ -834,7 +835,9 @@ __global__ __launch_bounds__(512) void k_colone(Dims d, Bg bg, DbyCoef cf, SegTa
     }
 }
 
-// Segment lengths of the one-lane form: longer ones do not fit its registers.
+// Segment lengths of the one-lane form: longer ones do not fit its registers.  Eight
+// rows keep 29 to 38 of them in scratch (120 to 188 bytes a lane) and 47 to 60 scalar
+// registers in spill lanes; every shape is compared with the oracle.
 #define SPARC_COLONE_SIZES(X) X(4) X(6) X(8)
 
 inline size_t colone_lds_bytes(int tc, const SegTab &sg)

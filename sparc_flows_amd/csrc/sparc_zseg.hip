@@ -367,8 +367,11 @@ __global__ __launch_bounds__(512) void k3_zp_seg(Z3 z, ZSeg sg)
 // (4.0 TB/s), 128x128x300 968 -> 360, 128x128x150 497 -> 143, 96x90x100 264 ->
 // 68, 32x32x40 91 -> 19.  Segments of at most 10 rows keep the four derivatives
 // and a row's loads in 256 registers; 19-row segments spilled (1440 us at
-// 256x256x300), and 12 to 16 rows (nz above 320) spill a little and still win
-// (256x256x448 2011 -> 1762).  One lane group per field, which reads v0 once
+// 256x256x300).  12, 14 and 16 rows (nz above 320, and 22 depths below whose last
+// segment would hold fewer than three rows otherwise: nz = 121, 122, 131, 132, 141, 142,
+// 151, 152, 241, 242, 261, 262 and so on by tens from 271 to 312) keep 160 to 536 bytes a lane in
+// scratch and still win: 128x128x121 405 -> 145, 96x90x301 920 -> 294, 256x256x301
+// 1326 -> 1296, 256x256x448 2011 -> 1762.  One lane group per field, which reads v0 once
 // per group, took 1500 us there, and blocks of 8 columns 1750: below 128 bytes
 // a row's piece is half a line.
 template <int MS, int NC>
